@@ -42,12 +42,15 @@ namespace k
     {
         // corners first (0: r = 0, s = 0; 1: r = 0, s = M-1; 2: r = M-1, s =
         // M-1; 3: r = M-1, s = 0), then the edges r = 0, s = M-1, r = M-1,
-        // s = 0 in that priority; as selects, so lanes do not diverge
+        // s = 0 in that priority; the flag's place is selected, not its
+        // value, so lanes do not diverge and the mask stays in registers (a
+        // select among its bytes makes the compiler index it in memory)
         const bool r0 = r == 0, rM = r == M - 1, s0 = s == 0, sM = s == M - 1;
         const bool corner = (r0 || rM) && (s0 || sM);
-        const bool c = r0 ? (s0 ? mk.dir[0] : mk.dir[1]) : (sM ? mk.dir[2] : mk.dir[3]);
-        const bool e = r0 ? mk.dir[4] : sM ? mk.dir[5] : rM ? mk.dir[6] : s0 ? mk.dir[7] : false;
-        return corner ? c : e;
+        const int c = r0 ? (s0 ? 0 : 1) : (sM ? 2 : 3);
+        const int e = r0 ? 4 : (sM ? 5 : (rM ? 6 : 7));
+        const uint64_t flags = __builtin_bit_cast(uint64_t, mk);
+        return (r0 || rM || s0 || sM) && ((flags >> (8 * (corner ? c : e))) & 1u) != 0;
     }
 
     // (DT)(acc + w v) evaluated in double, as the reference's transfers do

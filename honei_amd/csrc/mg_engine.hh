@@ -31,6 +31,7 @@ namespace mg
 {
     constexpr int kMaxLevels = 15;          // levels 0..14 (side 2^L + 1)
     constexpr unsigned kNormBlocks = 1024;  // reduction blocks per slot
+    constexpr int kRowCodes = 256;          // distinct matrix rows of a level with row codes
 
     enum Phase : int
     {
@@ -129,6 +130,11 @@ namespace mg
         // and the tables, ctab[16 k + t]; null otherwise
         uint64_t * codes = nullptr;
         float * ctab = nullptr;
+        // row codes instead, when those words take at most kRowCodes values:
+        // node i's row of ten floats is rtab[12 rcode[i] + k]
+        uint8_t * rcode = nullptr;
+        float * rtab = nullptr;
+        int rows = 0;
         k::Bands B() const
         {
             k::Bands r;

@@ -23,6 +23,7 @@
 #include <map>
 #include <mutex>
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
 namespace hsolve
@@ -112,6 +113,9 @@ namespace
         const float * dinv;
         int64_t n, m;
         int64_t bs;          // band stride in elements
+        const uint8_t * rcode = nullptr;    // row codes (HierLevel::rcode), or null
+        const float * rtab = nullptr;       // their rows (12 floats each)
+        int rows = 0;                       // how many
         const uint64_t * codes = nullptr;   // value codes of bands and dinv, or null
         const float * ctab = nullptr;       // their tables (16 per array)
     };
@@ -590,70 +594,29 @@ namespace
 
     // workgroups (over all slots) of the per-tick gate kernels' capped grids
     constexpr unsigned kGateBlocks = 4096;
-    constexpr int kPostLanes = 256;
-    constexpr int kPostW = kPostLanes - 6;
-    // slots per workgroup of the one-pass kernels when a tick runs several:
-    // they share each tile's band and dinv loads
-    constexpr int kPostSlots = 2;
     template <int N> using IntC = std::integral_constant<int, N>;
 
-    // Row i of A x from three rows of x in LDS (up, mid, dn: rows r - 1, r,
-    // r + 1 of the tile's column span, j the lane's column), b[0..8] the row's
-    // nine bands (LL .. UU), in q1_row's order.  GUARD: test each neighbour's
-    // index against [0, n) as q1_row does; without it every neighbour must
-    // lie in the matrix (rows 1 .. m - 2 of the grid).  Indices fit in 32 bits
-    // (levels up to 16385^2).
-    template <int MK, bool GUARD, int NB>
-    __device__ __forceinline__ float post_row(const float (&b)[NB], const float * __restrict__ up,
-                                              const float * __restrict__ mid, const float * __restrict__ dn, int j,
-                                              int i, int n, int m)
-    {
-        if (kOrd<MK> == 1)
-        {
-            float s = 0.0f;
-            if (! GUARD || i - m - 1 >= 0) s += b[0] * up[j - 1];
-            if (! GUARD || i - m >= 0)     s += b[1] * up[j];
-            if (! GUARD || i - m + 1 >= 0) s += b[2] * up[j + 1];
-            if (! GUARD || i - 1 >= 0)     s += b[3] * mid[j - 1];
-            s += b[4] * mid[j];
-            if (! GUARD || i + 1 < n)      s += b[5] * mid[j + 1];
-            if (! GUARD || i + m - 1 < n)  s += b[6] * dn[j - 1];
-            if (! GUARD || i + m < n)      s += b[7] * dn[j];
-            if (! GUARD || i + m + 1 < n)  s += b[8] * dn[j + 1];
-            return s;
-        }
-        float s = b[4] * mid[j];
-        if (! GUARD || i - m - 1 >= 0) s += b[0] * up[j - 1];
-        if (! GUARD || i - m >= 0)     s += b[1] * up[j];
-        if (! GUARD || i - m + 1 >= 0) s += b[2] * up[j + 1];
-        if (! GUARD || i - 1 >= 0)     s += b[3] * mid[j - 1];
-        if (! GUARD || i + 1 < n)      s += b[5] * mid[j + 1];
-        if (! GUARD || i + m - 1 < n)  s += b[6] * dn[j - 1];
-        if (! GUARD || i + m < n)      s += b[7] * dn[j];
-        if (! GUARD || i + m + 1 < n)  s += b[8] * dn[j + 1];
-        return s;
-    }
+#include "mg_march.hh"
 
-    // Tiles of a level of side m with th rows each (per slot).
-    inline unsigned post_tiles(int64_t m, int th)
+    // Tiles of a level of side m with th rows each, V columns per lane.
+    template <int V> unsigned march_tiles(int64_t m, int th)
     {
-        return (unsigned)(((m + kPostW - 1) / kPostW) * ((m + th - 1) / th));
+        return (unsigned)(((m + kW<V> - 1) / kW<V>) * ((m + th - 1) / th));
     }
 
     // Tile rows of the one-pass kernels: a tile's steps are sequential (th + 6
-    // of them, each waiting on memory), so the height is the even th <= 128
-    // with the fewest rounds of steps, ceil(tiles / resident) * (th + 6),
-    // where `resident` tiles fit on the device at once (the larger th on a
-    // tie: fewer halo rows).
-    inline int post_rows(int64_t m, unsigned slots, unsigned resident)
+    // of them), so the height is the even th <= 128 with the fewest rounds of
+    // steps, ceil(tiles / resident) * (th + 6), where `resident` tiles fit on
+    // the device at once (the larger th on a tie: fewer halo rows).
+    template <int V> int march_rows(int64_t m, unsigned slots, unsigned resident)
     {
         int best = 2;
         uint64_t best_cost = ~(uint64_t)0;
         for (int th = 2; th <= 128; th += 2)
         {
-            const uint64_t tiles = (uint64_t)post_tiles(m, th) * slots;
+            const uint64_t tiles = (uint64_t)march_tiles<V>(m, th) * slots;
             const uint64_t rounds = (tiles + resident - 1) / resident;
-            const uint64_t cost = rounds * (uint64_t)((th + 7) & ~1);
+            const uint64_t cost = rounds * (uint64_t)(th + 6);
             if (cost <= best_cost)
             {
                 best_cost = cost;
@@ -679,547 +642,10 @@ namespace
             return it->second;
         int cus = 0, per_cu = 0;
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kPostLanes, 0));
+        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, 0));
         const unsigned r = (unsigned)std::max(1, cus * std::max(1, per_cu));
         cache.emplace(std::make_pair(dev, fn), r);
         return r;
-    }
-
-    // ------------------------------------------- post-smoothing in one pass
-    // Two damped-Jacobi sweeps x1 = x + dinv (rhs - A x), x2 = x1 + dinv (rhs
-    // - A x1) and, with DEFECT, d = rhs - A x2, in one pass over Q1 bands
-    // (MK 0 / 2).  Every value is the one the separate sweep and defect
-    // kernels form: each row sums in q1_row's order over the same linear
-    // neighbours i +- 1, i +- m, i +- m +- 1 with the same index guards.
-    //
-    // A tile is kPostW consecutive columns of th grid rows (the last tiles of
-    // a level are narrower / shorter).  Its kPostLanes lanes each own one column
-    // offset c = c0 - 3 + lane of every row; a row's linear span [R m + c0 -
-    // 3, R m + c0 + W + 3) runs past the grid row's ends into the
-    // neighbouring rows, exactly as the linear index does.  The tile marches
-    // through its rows, down (even row blocks) or up (odd ones): march
-    // position p is grid row R0 + p or R0 + H - 1 - p.  Step s takes x at
-    // position s - 3 and the bands, dinv and rhs at s - 4 (loaded two steps
-    // ahead, in registers), then forms x1 at position s - 4, x2 at s - 5 and
-    // d at s - 6 from three-row rings of x, x1, x2 in LDS.  Each row's bands
-    // are read from HBM once per tile and kept in registers for its three
-    // stages.  A node's value does not depend on the direction: its sum
-    // reads the rows above and below from the ring either way.
-    //
-    // x2 goes to field fout, which must differ from fx: neighbouring tiles
-    // read x around their own rows while this tile writes.
-    //
-    // The steps synchronise on LDS only (lds_barrier: no wait for global
-    // loads), so the loads of the next two steps stay in flight across them;
-    // no lane reads a global value another lane of the tile wrote.
-    //
-    // PROL: x is first corrected by the prolongation of level L-1's field
-    // fcoarse, x + alpha P(coarse) (Prolongation<NONE> then ScaledSum with
-    // the fixed correction factor), formed per loaded node, so the corrected
-    // x is never stored.
-    template <int MK, int DEFECT, int PROL, int K, bool CB = false>
-    __global__ __launch_bounds__(kPostLanes) void v_post2_kernel(LevelArgs a, const Slot * T, int L, int fx, int fout,
-                                                          int fcoarse, float alpha, k::Mask mk, int th, int nslots)
-    {
-        const VB vb = vblock();
-        // the workgroup's K slots vb.z K + q: they share the tile's band and
-        // dinv loads; a slot that is not running borrows the arrays of one
-        // that is for its loads and stores nothing
-        bool on[K];
-        int pick = -1;
-#pragma unroll
-        for (int q = 0; q < K; ++q)
-        {
-            const int z = (int)vb.z * K + q;
-            on[q] = z < nslots && live(T[z]) && T[z].s->run != 0;
-            if (on[q] && pick < 0)
-                pick = q;
-        }
-        if (pick < 0)
-            return;
-        // CB: the bands and dinv come as value codes (one 64-bit word per
-        // node) and are decoded through their tables, held in LDS
-        __shared__ float ctab[CB ? 160 : 1];
-        if constexpr (CB)
-        {
-            if (threadIdx.x < 160)
-                ctab[threadIdx.x] = a.ctab[threadIdx.x];
-            __syncthreads();
-        }
-        const gptr<const uint64_t> codes = as_global<const uint64_t>(a.codes);
-        auto band_in = [&](const auto & bq, int k) -> float {
-            if constexpr (CB)
-                return ctab[k * 16 + (int)((bq >> (4 * k)) & 15u)];
-            else
-                return bq[k];
-        };
-        using BandIn = std::conditional_t<CB, uint64_t, float[10]>;
-        __shared__ float xr[K][3][kPostLanes];
-        __shared__ float x1r[K][3][kPostLanes];
-        __shared__ float x2r[K][DEFECT ? 3 : 1][kPostLanes];
-        const int n = (int)a.n, m = (int)a.m;
-        // tiles in row blocks, column strips fastest: horizontal neighbours
-        // march through the same rows at the same time on one XCD
-        // (k::xcd_block), so the cache lines they share (a row chunk's first
-        // and last, which the grid's odd side leaves unaligned) come from HBM
-        // once
-        const unsigned t = gridDim.z == 1 ? k::xcd_block(vb.x, gridDim.x) : vb.x;
-        const int nst = (m + kPostW - 1) / kPostW;
-        const int c0 = (int)(t % nst) * kPostW;
-        const int R0 = (int)(t / nst) * th;
-        const int W = min(kPostW, m - c0);
-        const int H = min(th, m - R0);
-        // even row blocks march down, odd ones up, so the halo rows two
-        // vertical neighbours share are read by both at about the same time
-        // (both at their first steps or both at their last); march position
-        // p is grid row Rs + dir p
-        const int dir = ((t / nst) & 1) ? -1 : 1;
-        const int Rs = dir > 0 ? R0 : R0 + H - 1;
-        const int j = threadIdx.x;
-        const int c = c0 - 3 + j;
-        const bool in_x = j < W + 6;
-        const bool in_1 = j >= 1 && j < W + 5;
-        const bool in_2 = j >= 2 && j < W + 4;
-        const bool own = j >= 3 && j < W + 3;
-        gptr<const float> x[K], rhs[K], xc[K];
-        gptr<float> out[K], dout[K];
-#pragma unroll
-        for (int q = 0; q < K; ++q)
-        {
-            const Slot & sl = T[(int)vb.z * K + (on[q] ? q : pick)];
-            x[q] = as_global<const float>(sl.v[L][fx]);
-            rhs[q] = as_global<const float>(sl.v[L][F_RHS]);
-            out[q] = as_global<float>(sl.v[L][fout]);
-            dout[q] = as_global<float>(sl.v[L][F_D]);
-            xc[q] = as_global<const float>(PROL ? sl.v[L - 1][fcoarse] : sl.v[L][fx]);
-        }
-        const gptr<const float> dinv = as_global<const float>(a.dinv);
-        // the nine bands from one base: band k of node i at element i + k bs
-        // (9 bs 4 < 2^32, checked on the host)
-        const gptr<const float> bands = as_global<const float>((const float *)a.B.b[0]);
-        const uint32_t bs = (uint32_t)a.bs;
-        const int Nc = (m + 1) / 2;
-
-        // grid position (R, S) of the node at march position s - 3, column
-        // offset c (c lies in [-3, 2m)), clamped to the grid
-        auto grid_pos = [&](int s, int & R, int & S) {
-            R = Rs + dir * (s - 3);
-            S = c;
-            if (S < 0)
-            {
-                S += m;
-                R -= 1;
-            }
-            else if (S >= m)
-            {
-                S -= m;
-                R += 1;
-            }
-            R = min(max(R, 0), m - 1);
-            S = min(max(S, 0), m - 1);
-        };
-        // The loads of step s: each slot's x at march position s - 3 (with
-        // PROL the four coarse values around it) and rhs at position s - 4,
-        // and the bands and dinv at s - 4 (shared).  Every lane loads, at
-        // indices clamped to the arrays, with no branch between the loads;
-        // step s decides which values count.
-        auto load = [&](int s, float (&xq)[K], float (&cq)[K][4], float (&rq)[K], BandIn & bq) {
-            const int ix = (Rs + dir * (s - 3)) * m + c;
-            const uint32_t ib = (uint32_t)min(max(ix - dir * m, 0), n - 1);
-#pragma unroll
-            for (int q = 0; q < K; ++q)
-            {
-                xq[q] = ld32(x[q], (uint32_t)min(max(ix, 0), n - 1));
-                if (PROL)
-                {
-                    int R, S;
-                    grid_pos(s, R, S);
-                    const int ra = (R >> 1) * Nc, rb = ((R + 1) >> 1) * Nc;
-                    const int jj = S >> 1, jj1 = min(jj + 1, Nc - 1);
-                    cq[q][0] = ld32(xc[q], (uint32_t)(ra + jj));
-                    cq[q][1] = ld32(xc[q], (uint32_t)(ra + jj1));
-                    cq[q][2] = ld32(xc[q], (uint32_t)(rb + jj));
-                    cq[q][3] = ld32(xc[q], (uint32_t)(rb + jj1));
-                }
-                rq[q] = ld32(rhs[q], ib);
-            }
-            if constexpr (CB)
-                bq = ld32(codes, ib);
-            else
-            {
-#pragma unroll
-                for (int k = 0; k < 9; ++k)
-                    bq[k] = ld32(bands, ib + (uint32_t)k * bs);
-                bq[9] = ld32(dinv, ib);
-            }
-        };
-        // H + 6 steps, rounded up to an even count so that the loop body is
-        // two whole steps with no branch around their loads (the extra step's
-        // rows lie outside the tile: nothing of it is stored)
-        const int steps = (H + 7) & ~1;
-        // A tile whose rows R0 - 4 .. R0 + H + 3 lie in the grid has every
-        // node the stored values depend on, and every neighbour of those, in
-        // the matrix: no index tests
-        const bool interior = R0 >= 4 && R0 + H + 4 <= m;
-        auto march = [&](auto interior_tag) {
-            constexpr bool G = ! decltype(interior_tag)::value;
-            // stage registers: march position s - 4 (stage 1), s - 5 (stage
-            // 2), s - 6 (stage 3): bands and dinv (b), each slot's rhs (r)
-            float b1[10] = {}, b2[10] = {}, b3[10] = {};
-            float r1[K] = {}, r2[K] = {}, r3[K] = {};
-            // one step; its loads, then those of step s + 2
-            auto step = [&](int s, float (&xq)[K], float (&cq)[K][4], float (&rq)[K], BandIn & bq) {
-                // ring rows: positions p, p - 1, p - 2; the row above a stage's
-                // row is the older one marching down, the newer one marching up
-                const int cur = s % 3, prv = (s + 2) % 3, old = (s + 1) % 3;
-                const int above = dir > 0 ? old : cur, below = dir > 0 ? cur : old;
-                {
-                    const int ix = (Rs + dir * (s - 3)) * m + c;
-                    const bool vx = in_x && (! G || (ix >= 0 && ix < n));
-#pragma unroll
-                    for (int q = 0; q < K; ++q)
-                    {
-                        float xv = 0.0f;
-                        if (vx)
-                        {
-                            xv = xq[q];
-                            if (PROL)
-                            {
-                                int R, S;
-                                grid_pos(s, R, S);
-                                xv = xv + alpha * k::prolongation_node_v<float>(cq[q], m, mk, R, S);
-                            }
-                        }
-                        xr[q][cur][j] = xv;
-                    }
-                    const int ib = ix - dir * m;
-                    const bool vb1 = in_1 && s >= 2 && (! G || (ib >= 0 && ib < n));
-#pragma unroll
-                    for (int k = 0; k < 10; ++k)
-                    {
-                        b3[k] = b2[k];
-                        b2[k] = b1[k];
-                        b1[k] = vb1 ? band_in(bq, k) : 0.0f;
-                    }
-#pragma unroll
-                    for (int q = 0; q < K; ++q)
-                    {
-                        r3[q] = r2[q];
-                        r2[q] = r1[q];
-                        r1[q] = vb1 ? rq[q] : 0.0f;
-                    }
-                }
-                load(s + 2, xq, cq, rq, bq);
-                lds_barrier();
-                // stage 1: x1 at position s - 4
-                if (s >= 2)
-                {
-                    const int i = (Rs + dir * (s - 4)) * m + c;
-                    const bool v1 = in_1 && (! G || (i >= 0 && i < n));
-#pragma unroll
-                    for (int q = 0; q < K; ++q)
-                    {
-                        float v = 0.0f;
-                        if (v1)
-                        {
-                            const float sum = post_row<MK, G>(b1, xr[q][above], xr[q][prv], xr[q][below], j, i, n, m);
-                            const float tt = r1[q] - sum;
-                            v = xr[q][prv][j] + tt * b1[9];
-                        }
-                        x1r[q][cur][j] = v;
-                    }
-                }
-                lds_barrier();
-                // stage 2: x2 at position s - 5
-                if (s >= 4)
-                {
-                    const int r2w = Rs + dir * (s - 5);
-                    const int i = r2w * m + c;
-                    const bool v2 = in_2 && (! G || (i >= 0 && i < n));
-                    const bool st2 = own && r2w >= R0 && r2w < R0 + H;
-#pragma unroll
-                    for (int q = 0; q < K; ++q)
-                    {
-                        float v = 0.0f;
-                        if (v2)
-                        {
-                            const float sum = post_row<MK, G>(b2, x1r[q][above], x1r[q][prv], x1r[q][below], j, i, n, m);
-                            const float tt = r2[q] - sum;
-                            v = x1r[q][prv][j] + tt * b2[9];
-                            if (st2 && on[q])
-                                st32(out[q], (uint32_t)i, v);
-                        }
-                        if (DEFECT)
-                            x2r[q][DEFECT ? cur : 0][j] = v;
-                    }
-                }
-                if (DEFECT)
-                {
-                    lds_barrier();
-                    // stage 3: d at position s - 6
-                    const int r3w = Rs + dir * (s - 6);
-                    const int i = r3w * m + c;
-                    if (s >= 6 && own && r3w >= R0 && r3w < R0 + H && (! G || (i >= 0 && i < n)))
-                    {
-#pragma unroll
-                        for (int q = 0; q < K; ++q)
-                        {
-                            const float sum = post_row<MK, G>(b3, x2r[q][DEFECT ? above : 0], x2r[q][DEFECT ? prv : 0],
-                                                              x2r[q][DEFECT ? below : 0], j, i, n, m);
-                            if (on[q])
-                                st32(dout[q], (uint32_t)i, r3[q] - sum);
-                        }
-                    }
-                }
-            };
-            float xA[K], xB[K], cA[K][4] = {}, cB[K][4] = {}, rA[K], rB[K];
-            BandIn bA, bB;
-            load(0, xA, cA, rA, bA);
-            load(1, xB, cB, rB, bB);
-            for (int s = 0; s < steps; s += 2)
-            {
-                step(s, xA, cA, rA, bA);
-                step(s + 1, xB, cB, rB, bB);
-            }
-        };
-        if (interior)
-            march(std::true_type{});
-        else
-            march(std::false_type{});
-    }
-
-    // ---------------------- pre-smoothing, defect and restriction in one pass
-    // The first two damped-Jacobi sweeps from zero (c1 = dinv d, c2 = c1 +
-    // dinv (d - A c1)), x = c2 (ACC: x = (field facc) + c2), the defect d' =
-    // rhs - A x and the coarse right-hand side Restriction<NONE>(d') with the
-    // Dirichlet mask, in one pass over Q1 bands (MK 0 / 2).  Every value is
-    // the one the separate kernels form (q1_row's order and guards,
-    // restrict_node's addition sequence); d' itself is never stored.
-    //
-    // Tiles and march directions as v_post2_kernel, with an even th, so a
-    // tile's first row is even and it owns the coarse rows r with 2r in its
-    // rows.  Step s takes march position s - 3 (d, dinv, rhs, the bands and
-    // facc, loaded two steps ahead; c1 is formed at once), forms x at s - 4
-    // and d' at s - 5, and, when that d' row is 2r + 1 (marching down) or 2r
-    // - 1 (up), coarse row r from the three d' rows in LDS (lanes on even
-    // fine columns).  The lanes cover fine columns c0 - 3
-    // .. c0 + W + 2 in linear index order, so the stencil steps are the
-    // linear index's; the restriction reads grid columns 2s - 1 .. 2s + 1 of
-    // owned columns 2s, which all lie in that span.
-    template <int MK, int ACC, int K, bool CB = false>
-    __global__ __launch_bounds__(kPostLanes) void v_pre2r_kernel(LevelArgs a, const Slot * T, int L, int fd, int facc,
-                                                          int64_t Nc64, k::Mask mk, int th, int nslots)
-    {
-        const VB vb = vblock();
-        // the workgroup's K slots, as in v_post2_kernel
-        bool on[K];
-        int pick = -1;
-#pragma unroll
-        for (int q = 0; q < K; ++q)
-        {
-            const int z = (int)vb.z * K + q;
-            on[q] = z < nslots && live(T[z]) && T[z].s->run != 0;
-            if (on[q] && pick < 0)
-                pick = q;
-        }
-        if (pick < 0)
-            return;
-        // CB: value-coded bands and dinv, as in v_post2_kernel
-        __shared__ float ctab[CB ? 160 : 1];
-        if constexpr (CB)
-        {
-            if (threadIdx.x < 160)
-                ctab[threadIdx.x] = a.ctab[threadIdx.x];
-            __syncthreads();
-        }
-        const gptr<const uint64_t> codes = as_global<const uint64_t>(a.codes);
-        auto band_in = [&](const auto & bq, int k) -> float {
-            if constexpr (CB)
-                return ctab[k * 16 + (int)((bq >> (4 * k)) & 15u)];
-            else
-                return bq[k];
-        };
-        using BandIn = std::conditional_t<CB, uint64_t, float[10]>;
-        __shared__ float c1r[K][3][kPostLanes];
-        __shared__ float xr[K][3][kPostLanes];
-        __shared__ float dr[K][3][kPostLanes];
-        const int n = (int)a.n, m = (int)a.m, Nc = (int)Nc64;
-        const unsigned t = gridDim.z == 1 ? k::xcd_block(vb.x, gridDim.x) : vb.x;
-        const int nst = (m + kPostW - 1) / kPostW;
-        const int c0 = (int)(t % nst) * kPostW;
-        const int R0 = (int)(t / nst) * th;
-        const int W = min(kPostW, m - c0);
-        const int H = min(th, m - R0);
-        // march direction as in v_post2_kernel: position p is row Rs + dir p
-        const int dir = ((t / nst) & 1) ? -1 : 1;
-        const int Rs = dir > 0 ? R0 : R0 + H - 1;
-        const int j = threadIdx.x;
-        const int c = c0 - 3 + j;
-        const bool in_x = j < W + 6;
-        const bool in_1 = j >= 1 && j < W + 5;
-        const bool in_2 = j >= 2 && j < W + 4;
-        const bool own = j >= 3 && j < W + 3;
-        const bool own_even = own && ((c & 1) == 0);
-        gptr<const float> d[K], rhs[K], acc[K];
-        gptr<float> xo[K], co[K];
-#pragma unroll
-        for (int q = 0; q < K; ++q)
-        {
-            const Slot & sl = T[(int)vb.z * K + (on[q] ? q : pick)];
-            d[q] = as_global<const float>(sl.v[L][fd]);
-            rhs[q] = as_global<const float>(sl.v[L][F_RHS]);
-            acc[q] = as_global<const float>(sl.v[L][facc]);
-            xo[q] = as_global<float>(sl.v[L][F_X]);
-            co[q] = as_global<float>(sl.v[L - 1][F_RHS]);
-        }
-        const gptr<const float> dinv = as_global<const float>(a.dinv);
-        // bands as in v_post2_kernel
-        const gptr<const float> bands = as_global<const float>((const float *)a.B.b[0]);
-        const uint32_t bs = (uint32_t)a.bs;
-
-        // march position s - 3 for step s: the 9 bands and dinv (shared) and
-        // each slot's d, rhs and facc value (pq[q][0..2]); every lane loads,
-        // at an index clamped to the arrays, with no branch between the
-        // loads; step s decides which values count
-        auto load = [&](int s, BandIn & bq, float (&pq)[K][3]) {
-            const uint32_t i = (uint32_t)min(max((Rs + dir * (s - 3)) * m + c, 0), n - 1);
-            if constexpr (CB)
-                bq = ld32(codes, i);
-            else
-            {
-#pragma unroll
-                for (int k = 0; k < 9; ++k)
-                    bq[k] = ld32(bands, i + (uint32_t)k * bs);
-                bq[9] = ld32(dinv, i);
-            }
-#pragma unroll
-            for (int q = 0; q < K; ++q)
-            {
-                pq[q][0] = ld32(d[q], i);
-                pq[q][1] = ld32(rhs[q], i);
-                pq[q][2] = ACC ? ld32(acc[q], i) : 0.0f;
-            }
-        };
-        // H + 6 steps, rounded up to an even count (as v_post2_kernel)
-        const int steps = (H + 7) & ~1;
-        // rows R0 - 4 .. R0 + H + 3 in the grid: no index tests (as v_post2_kernel)
-        const bool interior = R0 >= 4 && R0 + H + 4 <= m;
-        auto march = [&](auto interior_tag) {
-            constexpr bool G = ! decltype(interior_tag)::value;
-            // stage registers: position s - 3 (its c1 only, yet), s - 4 (x:
-            // bands, dinv, d, facc), s - 5 (d': bands, rhs); bands and dinv
-            // (bc, ba, bb) shared, d, rhs, facc per slot (pc, pa, pb)
-            float bc[10] = {}, ba[10] = {}, bb[10] = {};
-            float pc[K][3] = {}, pa[K][3] = {}, pb[K][3] = {};
-            auto step = [&](int s, BandIn & bq, float (&pq)[K][3]) {
-                // ring rows: positions p, p - 1, p - 2 (above / below as in v_post2_kernel)
-                const int cur = s % 3, prv = (s + 2) % 3, old = (s + 1) % 3;
-                const int above = dir > 0 ? old : cur, below = dir > 0 ? cur : old;
-                {
-                    const int i = (Rs + dir * (s - 3)) * m + c;
-                    const bool valid = in_x && (! G || (i >= 0 && i < n));
-#pragma unroll
-                    for (int k = 0; k < 10; ++k)
-                    {
-                        bb[k] = ba[k];
-                        ba[k] = bc[k];
-                        bc[k] = valid ? band_in(bq, k) : 0.0f;
-                    }
-#pragma unroll
-                    for (int q = 0; q < K; ++q)
-                    {
-#pragma unroll
-                        for (int k = 0; k < 3; ++k)
-                        {
-                            pb[q][k] = pa[q][k];
-                            pa[q][k] = pc[q][k];
-                            pc[q][k] = valid ? pq[q][k] : 0.0f;
-                        }
-                        c1r[q][cur][j] = bc[9] * pc[q][0];
-                    }
-                }
-                load(s + 2, bq, pq);
-                lds_barrier();
-                // x at position s - 4
-                if (s >= 2)
-                {
-                    const int rho = Rs + dir * (s - 4);
-                    const int i = rho * m + c;
-                    const bool v1 = in_1 && (! G || (i >= 0 && i < n));
-                    const bool stx = own && rho >= R0 && rho < R0 + H;
-#pragma unroll
-                    for (int q = 0; q < K; ++q)
-                    {
-                        float v = 0.0f;
-                        if (v1)
-                        {
-                            const float sum = post_row<MK, G>(ba, c1r[q][above], c1r[q][prv], c1r[q][below], j, i, n, m);
-                            const float tt = pa[q][0] - sum;
-                            const float c2 = c1r[q][prv][j] + tt * ba[9];
-                            v = ACC ? pa[q][2] + c2 : c2;
-                            if (stx && on[q])
-                                st32(xo[q], (uint32_t)i, v);
-                        }
-                        xr[q][cur][j] = v;
-                    }
-                }
-                lds_barrier();
-                // d' at position s - 5
-                if (s >= 4)
-                {
-                    const int rho = Rs + dir * (s - 5);
-                    const int i = rho * m + c;
-                    const bool v2 = in_2 && (! G || (i >= 0 && i < n));
-#pragma unroll
-                    for (int q = 0; q < K; ++q)
-                    {
-                        float v = 0.0f;
-                        if (v2)
-                        {
-                            const float sum = post_row<MK, G>(bb, xr[q][above], xr[q][prv], xr[q][below], j, i, n, m);
-                            v = pb[q][1] - sum;
-                        }
-                        dr[q][cur][j] = v;
-                    }
-                    lds_barrier();
-                    // coarse row r when this d' row is 2r + dir: rows 2r - 1,
-                    // 2r, 2r + 1 are then in the ring
-                    if (((rho - 1) & 1) == 0)
-                    {
-                        const int r = (rho - dir) >> 1;
-                        if (own_even && 2 * r >= R0 && 2 * r < R0 + H && c < m)
-                        {
-                            const int sc = c >> 1;
-#pragma unroll
-                            for (int q = 0; q < K; ++q)
-                            {
-                                const float (*ring)[kPostLanes] = dr[q];
-                                const float v = k::restrict_node<float>(
-                                    [&](int ddr, int dds) {
-                                        return ring[dir * ddr < 0 ? old : (ddr == 0 ? prv : cur)][j + dds];
-                                    },
-                                    r, sc, Nc, mk);
-                                if (on[q])
-                                    st32(co[q], (uint32_t)(r * Nc + sc), v);
-                            }
-                        }
-                    }
-                }
-            };
-            BandIn bA, bB;
-            float pA[K][3], pB[K][3];
-            load(0, bA, pA);
-            load(1, bB, pB);
-            for (int s = 0; s < steps; s += 2)
-            {
-                step(s, bA, pA);
-                step(s + 1, bB, pB);
-            }
-        };
-        if (interior)
-            march(std::true_type{});
-        else
-            march(std::false_type{});
     }
 
     // y = x + dinv * (rhs - A x)
@@ -1774,21 +1200,13 @@ namespace
 
     void warm_post_kernels()
     {
-#define HS_K(KS)                                                                                               \
-    (const void *)v_pre2r_kernel<0, 0, KS>, (const void *)v_pre2r_kernel<0, 1, KS>,                            \
-        (const void *)v_pre2r_kernel<2, 0, KS>, (const void *)v_pre2r_kernel<2, 1, KS>,                        \
-        (const void *)v_post2_kernel<0, 0, 0, KS>, (const void *)v_post2_kernel<0, 0, 1, KS>,                  \
-        (const void *)v_post2_kernel<0, 1, 0, KS>, (const void *)v_post2_kernel<0, 1, 1, KS>,                  \
-        (const void *)v_post2_kernel<2, 0, 0, KS>, (const void *)v_post2_kernel<2, 0, 1, KS>,                  \
-        (const void *)v_post2_kernel<2, 1, 0, KS>, (const void *)v_post2_kernel<2, 1, 1, KS>,                  \
-        (const void *)v_pre2r_kernel<0, 0, KS, true>, (const void *)v_pre2r_kernel<0, 1, KS, true>,            \
-        (const void *)v_post2_kernel<0, 0, 0, KS, true>, (const void *)v_post2_kernel<0, 0, 1, KS, true>,      \
-        (const void *)v_post2_kernel<0, 1, 0, KS, true>, (const void *)v_post2_kernel<0, 1, 1, KS, true>,      \
-        (const void *)v_pre2r_kernel<2, 0, KS, true>, (const void *)v_pre2r_kernel<2, 1, KS, true>,            \
-        (const void *)v_post2_kernel<2, 0, 0, KS, true>, (const void *)v_post2_kernel<2, 0, 1, KS, true>,      \
-        (const void *)v_post2_kernel<2, 1, 0, KS, true>, (const void *)v_post2_kernel<2, 1, 1, KS, true>
-        const void * fns[] = {HS_K(1), HS_K(kPostSlots)};
-#undef HS_K
+#define HS_W(MK, KS, VS, CB)                                                                                   \
+    (const void *)v_pre2r_kernel<MK, 0, KS, VS, CB>, (const void *)v_pre2r_kernel<MK, 1, KS, VS, CB>,          \
+        (const void *)v_post2_kernel<MK, 0, 0, KS, VS, CB>, (const void *)v_post2_kernel<MK, 0, 1, KS, VS, CB>, \
+        (const void *)v_post2_kernel<MK, 1, 0, KS, VS, CB>, (const void *)v_post2_kernel<MK, 1, 1, KS, VS, CB>
+        const void * fns[] = {HS_W(0, 1, 1, 0), HS_W(0, 2, 1, 0), HS_W(0, 1, 2, 1), HS_W(0, 1, 1, 2),
+                              HS_W(2, 1, 1, 0), HS_W(2, 2, 1, 0), HS_W(2, 1, 2, 1), HS_W(2, 1, 1, 2)};
+#undef HS_W
         for (const void * f : fns)
             (void)post_resident(f);
         (void)bottom_lds_limit();
@@ -1849,6 +1267,37 @@ void hierarchy_fill_poisson(Hierarchy & h, hipStream_t st)
     hierarchy_codes(h);
 }
 
+namespace
+{
+    // The distinct words of `code` (at most kRowCodes of them) and each
+    // entry's index among them; false when there are more.
+    bool row_codes(const std::vector<uint64_t> & code, std::vector<uint8_t> & rc, std::vector<uint64_t> & words)
+    {
+        std::unordered_map<uint64_t, uint8_t> at;
+        rc.resize(code.size());
+        uint64_t last = 0;
+        uint8_t last_t = 0;
+        for (size_t i = 0; i < code.size(); ++i)
+        {
+            if (i == 0 || code[i] != last)
+            {
+                auto it = at.find(code[i]);
+                if (it == at.end())
+                {
+                    if (words.size() == (size_t)kRowCodes)
+                        return false;
+                    it = at.emplace(code[i], (uint8_t)words.size()).first;
+                    words.push_back(code[i]);
+                }
+                last = code[i];
+                last_t = it->second;
+            }
+            rc[i] = last_t;
+        }
+        return true;
+    }
+}
+
 // Value-indexed storage of a level's bands (Q1, or a 9-point structured ELL
 // matrix kept as bands) and dinv (the value-index
 // compression of Kourtis, Goumas and Koziris, "Optimizing sparse
@@ -1869,6 +1318,7 @@ void hierarchy_codes(Hierarchy & h)
         HierLevel & l = h.lv[L];
         l.codes = nullptr;
         l.ctab = nullptr;
+        l.rcode = nullptr;
         if (l.n < 4225)     // the one-pass kernels run on levels of 65^2 and up
             continue;
         const uint64_t n = l.n;
@@ -1915,6 +1365,22 @@ void hierarchy_codes(Hierarchy & h)
         }
         if (! ok)
             continue;
+        std::vector<uint8_t> rc;
+        std::vector<uint64_t> words;
+        if (row_codes(code, rc, words))
+        {
+            // (16 bytes of padding on either side: the kernels load pairs)
+            std::vector<float> rows(12 * words.size(), 0.0f);
+            for (size_t t = 0; t < words.size(); ++t)
+                for (int k = 0; k < 10; ++k)
+                    std::memcpy(&rows[12 * t + k], &tab[16 * k + ((words[t] >> (4 * k)) & 15u)], sizeof(float));
+            l.rcode = (uint8_t *)h.alloc(n + 32) + 16;
+            l.rtab = (float *)h.alloc(sizeof(float) * rows.size());
+            l.rows = (int)words.size();
+            HIP_CHECK(hipMemcpy(l.rcode, rc.data(), n, hipMemcpyHostToDevice));
+            HIP_CHECK(hipMemcpy(l.rtab, rows.data(), sizeof(float) * rows.size(), hipMemcpyHostToDevice));
+            continue;
+        }
         l.codes = (uint64_t *)h.alloc(sizeof(uint64_t) * n);
         l.ctab = (float *)h.alloc(sizeof(tab));
         HIP_CHECK(hipMemcpy(l.codes, code.data(), sizeof(uint64_t) * n, hipMemcpyHostToDevice));
@@ -2251,9 +1717,25 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
         a.n = (int64_t)l.n;
         a.m = l.side;
         a.bs = (int64_t)l.bs;
+        a.rcode = h.use_codes ? l.rcode : nullptr;
+        a.rtab = l.rtab;
+        a.rows = l.rows;
         a.codes = h.use_codes ? l.codes : nullptr;
-        a.ctab = h.use_codes ? l.ctab : nullptr;
+        a.ctab = l.ctab;
         return a;
+    };
+    // The form of the one-pass kernels on a level: slots per workgroup, columns
+    // per lane, matrix storage.  Row codes leave registers for two columns a
+    // lane; with plain bands several slots share a tile's 40 bytes per node.
+    auto march_form = [&](const LevelArgs & a, auto && f) {
+        if (a.rcode)
+            f(IntC<1>{}, IntC<2>{}, IntC<1>{});
+        else if (a.codes)
+            f(IntC<1>{}, IntC<1>{}, IntC<2>{});
+        else if (S > 1)
+            f(IntC<2>{}, IntC<1>{}, IntC<0>{});
+        else
+            f(IntC<1>{}, IntC<1>{}, IntC<0>{});
     };
     auto norm_grid = [&](uint64_t nn) { return dim3(std::min<unsigned>(lanes4(nn), kNormBlocks), 1, S); };
     // row kernels: 4 rows per lane on Q1 bands, one row per lane on ELL
@@ -2396,32 +1878,20 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
                 if (pre2r)
                 {
                     const int64_t Nc = h.lv[L - 1].side;
-                    auto go = [&](auto acc_tag, auto k_tag) {
+                    auto go = [&](auto acc_tag, auto k_tag, auto v_tag, auto cb_tag) {
                         constexpr int ACC = decltype(acc_tag)::value, KS = decltype(k_tag)::value;
+                        constexpr int VS = decltype(v_tag)::value, CB = decltype(cb_tag)::value;
+                        auto kern = v_pre2r_kernel<MK, ACC, KS, VS, CB>;
                         const unsigned groups = (S + KS - 1) / KS;
-                        auto launch = [&](auto cb_tag) {
-                            constexpr bool CB = decltype(cb_tag)::value;
-                            const int th =
-                                    post_rows(a.m, groups, post_resident((const void *)v_pre2r_kernel<MK, ACC, KS, CB>));
-                            hipLaunchKernelGGL((v_pre2r_kernel<MK, ACC, KS, CB>), dim3(post_tiles(a.m, th), 1, groups),
-                                               dim3(kPostLanes), 0, st, a, T, (int)L, dsrc, ACC ? fx_top : (int)F_X, Nc,
-                                               p.mask, th, (int)S);
-                        };
-                        // value-coded bands (levels whose bands allow them)
-                        if constexpr (MK != 1)
-                        {
-                            if (a.codes)
-                                launch(std::true_type{});
-                            else
-                                launch(std::false_type{});
-                        }
-                        else
-                            launch(std::false_type{});
+                        const int th = march_rows<VS>(a.m, groups, kMarchWaves * post_resident((const void *)kern));
+                        const unsigned tiles = march_tiles<VS>(a.m, th);
+                        hipLaunchKernelGGL(kern, dim3((tiles + kMarchWaves - 1) / kMarchWaves, 1, groups), blk, 0, st,
+                                           a, T, (int)L, dsrc, ACC ? fx_top : (int)F_X, Nc, p.mask, th, tiles, (int)S);
                     };
                     if (L == maxl)
-                        S > 1 ? go(IntC<1>{}, IntC<kPostSlots>{}) : go(IntC<1>{}, IntC<1>{});
+                        march_form(a, [&](auto k_tag, auto v_tag, auto cb_tag) { go(IntC<1>{}, k_tag, v_tag, cb_tag); });
                     else
-                        S > 1 ? go(IntC<0>{}, IntC<kPostSlots>{}) : go(IntC<0>{}, IntC<1>{});
+                        march_form(a, [&](auto k_tag, auto v_tag, auto cb_tag) { go(IntC<0>{}, k_tag, v_tag, cb_tag); });
                     continue;
                 }
             }
@@ -2492,34 +1962,23 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
             return;
         }
     }
-    // v_post2_kernel on level L (DEFECT on the finest), kPostSlots slots per
-    // workgroup when the tick runs several
+    // v_post2_kernel on level L (DEFECT on the finest)
     auto post2_launch = [&](uint64_t L, const LevelArgs & a, int fcoarse, float alpha, auto prol_tag) {
         constexpr int PROL = decltype(prol_tag)::value;
-        auto go = [&](auto def_tag, auto k_tag) {
+        auto go = [&](auto def_tag, auto k_tag, auto v_tag, auto cb_tag) {
             constexpr int DEF = decltype(def_tag)::value, KS = decltype(k_tag)::value;
+            constexpr int VS = decltype(v_tag)::value, CB = decltype(cb_tag)::value;
+            auto kern = v_post2_kernel<MK, DEF, PROL, KS, VS, CB>;
             const unsigned groups = (S + KS - 1) / KS;
-            auto launch = [&](auto cb_tag) {
-                constexpr bool CB = decltype(cb_tag)::value;
-                const int th = post_rows(a.m, groups, post_resident((const void *)v_post2_kernel<MK, DEF, PROL, KS, CB>));
-                hipLaunchKernelGGL((v_post2_kernel<MK, DEF, PROL, KS, CB>), dim3(post_tiles(a.m, th), 1, groups),
-                                   dim3(kPostLanes), 0, st, a, T, (int)L, (int)F_X, (int)F_TMP, fcoarse, alpha, p.mask,
-                                   th, (int)S);
-            };
-            if constexpr (MK != 1)
-            {
-                if (a.codes)
-                    launch(std::true_type{});
-                else
-                    launch(std::false_type{});
-            }
-            else
-                launch(std::false_type{});
+            const int th = march_rows<VS>(a.m, groups, kMarchWaves * post_resident((const void *)kern));
+            const unsigned tiles = march_tiles<VS>(a.m, th);
+            hipLaunchKernelGGL(kern, dim3((tiles + kMarchWaves - 1) / kMarchWaves, 1, groups), blk, 0, st, a, T, (int)L,
+                               (int)F_X, (int)F_TMP, fcoarse, alpha, p.mask, th, tiles, (int)S);
         };
         if (L == maxl)
-            S > 1 ? go(IntC<1>{}, IntC<kPostSlots>{}) : go(IntC<1>{}, IntC<1>{});
+            march_form(a, [&](auto k_tag, auto v_tag, auto cb_tag) { go(IntC<1>{}, k_tag, v_tag, cb_tag); });
         else
-            S > 1 ? go(IntC<0>{}, IntC<kPostSlots>{}) : go(IntC<0>{}, IntC<1>{});
+            march_form(a, [&](auto k_tag, auto v_tag, auto cb_tag) { go(IntC<0>{}, k_tag, v_tag, cb_tag); });
     };
     for (uint64_t L = minl + 1; L <= maxl; ++L)
     {
