@@ -805,29 +805,16 @@ namespace
             xg[i] = x[i];
     }
 
-    // ------------------------------------------------ the bottom levels in LDS
-    // Levels minl .. top (top <= 5, below the finest) of a V-cycle on Q1
-    // bands, in one workgroup per slot with every vector and band of those
-    // levels in LDS: the same operations, per node, as the one-pass kernels
-    // and the coarse solve run there (two sweeps from zero, defect,
-    // restriction down to minl, the CG on minl, then prolongation with the
-    // correction factor and two sweeps back up to top), one level pass per
-    // barrier.  It reads the rhs of level top (written by the finest-but-
-    // one-pass kernel above it) and leaves top's smoothed iterate in its
-    // F_TMP, where the one-pass post-smoother above reads it.  It replaces
-    // two launches per level and the coarse solve's, each a chain of
-    // dependent memory round trips.  The coarse CG runs on the first wave
-    // alone, whose sequential sums read their terms from its lanes.
-    constexpr int kBottomMax = 5;
-    struct BottomArgs
+#include "mg_bottom.hh"
+
+    // The same for a coarsest level too large for one wave (minl 3 or 4):
+    // every vector and band of the levels in LDS, the coarse CG on the first
+    // wave with its vectors there.
+    struct BottomLdsArgs
     {
-        LevelArgs lv[kBottomMax + 1];
+        BottomArgs b;
         int off[kBottomMax + 1];   // float offset of each level's block in the dynamic LDS
-        int minl, top;
-        float alpha;
-        k::Mask mk;
-        double konv_rad;
-        uint64_t max_iters;
+        int minl;
     };
 
     // Row i of A x on a level held in LDS (band k at b + k n): q1_row's
@@ -877,7 +864,7 @@ namespace
     inline int bottom_floats(int n, bool coarsest) { return (coarsest ? 16 : 13) * n; }
 
     template <int MK>
-    __global__ __launch_bounds__(1024) void v_bottom_kernel(BottomArgs ba, const Slot * T)
+    __global__ __launch_bounds__(1024) void v_bottom_lds_kernel(BottomLdsArgs ba, const Slot * T)
     {
         const VB vb = vblock();
         HS_GATE_RUN
@@ -886,14 +873,14 @@ namespace
         // bands and dinv of every level: each lane issues the loads of two
         // rows of all ten arrays before it stores any, so a level costs one
         // or two memory round trips, not one per array and row
-        for (int L = ba.minl; L <= ba.top; ++L)
+        for (int L = ba.minl; L <= ba.b.top; ++L)
         {
-            const int n = (int)ba.lv[L].n;
+            const int n = (int)ba.b.lv[L].n;
             float * b = lds + ba.off[L];
             const float * src[10];
             for (int k = 0; k < 9; ++k)
-                src[k] = (const float *)ba.lv[L].B.b[k];
-            src[9] = ba.lv[L].dinv;
+                src[k] = (const float *)ba.b.lv[L].B.b[k];
+            src[9] = ba.b.lv[L].dinv;
             for (int i0 = tid; i0 < n; i0 += 2 * nt)
             {
                 float v[2][10];
@@ -919,18 +906,18 @@ namespace
             }
         }
         {
-            const int n = (int)ba.lv[ba.top].n;
-            const float * g = sl.v[ba.top][F_RHS];
-            float * rhs = lds + ba.off[ba.top] + 10 * n;
+            const int n = (int)ba.b.lv[ba.b.top].n;
+            const float * g = sl.v[ba.b.top][F_RHS];
+            float * rhs = lds + ba.off[ba.b.top] + 10 * n;
             for (int i = tid; i < n; i += nt)
                 rhs[i] = g[i];
         }
         __syncthreads();
         // down: x = c1 + dinv (rhs - A c1) with c1 = dinv rhs, d' = rhs - A x,
         // rhs of L - 1 = R d'
-        for (int L = ba.top; L > ba.minl; --L)
+        for (int L = ba.b.top; L > ba.minl; --L)
         {
-            const int n = (int)ba.lv[L].n, m = (int)ba.lv[L].m;
+            const int n = (int)ba.b.lv[L].n, m = (int)ba.b.lv[L].m;
             const float * b = lds + ba.off[L];
             const float * dinv = b + 9 * n;
             const float * rhs = b + 10 * n;
@@ -948,7 +935,7 @@ namespace
             for (int i = tid; i < n; i += nt)
                 tmp[i] = rhs[i] - lds_row<kOrd<MK>>(b, x, i, n, m);
             __syncthreads();
-            const int Nc = (int)ba.lv[L - 1].m;
+            const int Nc = (int)ba.b.lv[L - 1].m;
             float * crhs = lds + ba.off[L - 1] + 10 * Nc * Nc;
             for (int q = tid; q < Nc * Nc; q += nt)
             {
@@ -958,26 +945,26 @@ namespace
                         const int idx = (2 * r + dr) * m + 2 * sc + ds;
                         return tmp[min(max(idx, 0), n - 1)];
                     },
-                    r, sc, Nc, ba.mk);
+                    r, sc, Nc, ba.b.mk);
             }
             __syncthreads();
         }
         // the coarse solve, as v_coarse_lds_kernel, on the first wave
         {
             const int L = ba.minl;
-            const int n = (int)ba.lv[L].n;
+            const int n = (int)ba.b.lv[L].n;
             float * b = lds + ba.off[L];
-            const LdsRowOp<kOrd<MK>> A{b, n, (int)ba.lv[L].m};
+            const LdsRowOp<kOrd<MK>> A{b, n, (int)ba.b.lv[L].m};
             if (threadIdx.x < 64)
                 k::cg_konv_body_op<float, LdsRowOp<kOrd<MK>>, 64>(A, b + 10 * n, b + 11 * n, b + 12 * n, (int64_t)n,
-                                                                 ba.konv_rad, ba.max_iters, &sl.s->cg_iters);
+                                                                 ba.b.konv_rad, ba.b.max_iters, &sl.s->cg_iters);
             __syncthreads();
         }
         // up: x_in = x + alpha P (coarse iterate), then two sweeps into tmp
-        for (int L = ba.minl + 1; L <= ba.top; ++L)
+        for (int L = ba.minl + 1; L <= ba.b.top; ++L)
         {
-            const int n = (int)ba.lv[L].n, m = (int)ba.lv[L].m;
-            const int Nc = (int)ba.lv[L - 1].m;
+            const int n = (int)ba.b.lv[L].n, m = (int)ba.b.lv[L].m;
+            const int Nc = (int)ba.b.lv[L - 1].m;
             const float * cf = lds + ba.off[L - 1] + (L - 1 == ba.minl ? 11 : 12) * Nc * Nc;
             const float * b = lds + ba.off[L];
             const float * dinv = b + 9 * n;
@@ -987,7 +974,7 @@ namespace
             for (int i = tid; i < n; i += nt)
             {
                 const int R = i / m, S = i - R * m;
-                tmp[i] = x[i] + ba.alpha * k::prolongation_node<float>(cf, m, ba.mk, R, S);
+                tmp[i] = x[i] + ba.b.alpha * k::prolongation_node<float>(cf, m, ba.b.mk, R, S);
             }
             __syncthreads();
             for (int i = tid; i < n; i += nt)
@@ -1004,9 +991,9 @@ namespace
             __syncthreads();
         }
         {
-            const int n = (int)ba.lv[ba.top].n;
-            const float * tmp = lds + ba.off[ba.top] + 12 * n;
-            float * g = sl.v[ba.top][F_TMP];
+            const int n = (int)ba.b.lv[ba.b.top].n;
+            const float * tmp = lds + ba.off[ba.b.top] + 12 * n;
+            float * g = sl.v[ba.b.top][F_TMP];
             for (int i = tid; i < n; i += nt)
                 g[i] = tmp[i];
         }
@@ -1169,7 +1156,7 @@ namespace
 {
     // The occupancy of every one-pass kernel, looked up at set-up, never
     // under stream capture.
-    // Dynamic LDS v_bottom_kernel may take on the current device (cached per
+    // Dynamic LDS v_bottom_lds_kernel may take on the current device (cached per
     // device): the device's per-workgroup limit, once the kernels are allowed
     // more than 64 KiB, else 60 KiB (4 KiB of either left for its static LDS)
     inline unsigned bottom_lds_limit()
@@ -1188,9 +1175,9 @@ namespace
         const int want = v - 4096;
         unsigned r = (unsigned)std::min(std::max(want, 0), 65536 - 4096);
         if (want > 65536 &&
-            hipFuncSetAttribute((const void *)v_bottom_kernel<0>, hipFuncAttributeMaxDynamicSharedMemorySize, want) ==
+            hipFuncSetAttribute((const void *)v_bottom_lds_kernel<0>, hipFuncAttributeMaxDynamicSharedMemorySize, want) ==
                 hipSuccess &&
-            hipFuncSetAttribute((const void *)v_bottom_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, want) ==
+            hipFuncSetAttribute((const void *)v_bottom_lds_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, want) ==
                 hipSuccess)
             r = (unsigned)want;
         (void)hipGetLastError();
@@ -1755,40 +1742,45 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
     // is fixed (the adaptive one reads the level's defect again).
     const bool pre2r = post2 && p.adapt != 0.0f && ! h.prolmat;
     // With the one-pass kernels, levels minl .. btop (btop <= 5, below the
-    // finest, as many as fit the LDS of one workgroup) run in one
-    // v_bottom_kernel launch (one workgroup per slot); btop = 0: none.
+    // finest) run in one launch, one workgroup per slot: v_bottom_kernel when
+    // the coarsest level fits one wave (5^2 or less), v_bottom_lds_kernel with
+    // as many levels as fit the LDS of a workgroup otherwise; btop = 0: none.
     int btop = 0;
-    BottomArgs ba{};
+    BottomLdsArgs ba{};
     size_t bbytes = 0;
-    if (pre2r)
+    if (pre2r && maxl - 1 > minl)
     {
-        for (int top = (int)std::min<uint64_t>(kBottomMax, maxl - 1); top > (int)minl; --top)
-        {
-            size_t fl = 0;
-            for (int L = (int)minl; L <= top; ++L)
-                fl += (size_t)bottom_floats((int)h.lv[L].n, L == (int)minl);
-            if (fl * sizeof(float) <= bottom_lds_limit())
+        const int most = (int)std::min<uint64_t>(kBottomMax, maxl - 1);
+        if (minl <= 2)
+            btop = most;
+        else
+            for (int top = most; top > (int)minl; --top)
             {
-                btop = top;
-                bbytes = fl * sizeof(float);
-                break;
+                size_t fl = 0;
+                for (int L = (int)minl; L <= top; ++L)
+                    fl += (size_t)bottom_floats((int)h.lv[L].n, L == (int)minl);
+                if (fl * sizeof(float) <= bottom_lds_limit())
+                {
+                    btop = top;
+                    bbytes = fl * sizeof(float);
+                    break;
+                }
             }
-        }
         if (btop)
         {
             int off = 0;
             for (int L = (int)minl; L <= btop; ++L)
             {
-                ba.lv[L] = largs(L);
+                ba.b.lv[L] = largs(L);
                 ba.off[L] = off;
                 off += bottom_floats((int)h.lv[L].n, L == (int)minl);
             }
             ba.minl = (int)minl;
-            ba.top = btop;
-            ba.alpha = p.adapt;
-            ba.mk = p.mask;
-            ba.konv_rad = (double)1.19209290e-07F;
-            ba.max_iters = (uint64_t)(100 * h.lv[minl].n + 1000);
+            ba.b.top = btop;
+            ba.b.alpha = p.adapt;
+            ba.b.mk = p.mask;
+            ba.b.konv_rad = (double)1.19209290e-07F;
+            ba.b.max_iters = (uint64_t)(100 * h.lv[minl].n + 1000);
         }
     }
 
@@ -1946,8 +1938,12 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
         // with one level it sees the finest defect d
         const LevelArgs a = largs(minl);
         const int crhs = (minl == maxl) ? F_D : F_RHS;
-        if (btop)
-            hipLaunchKernelGGL((v_bottom_kernel<MK>), dim3(1, 1, S), dim3(1024), bbytes, st, ba, T);
+        if (btop && minl == 1)
+            hipLaunchKernelGGL((v_bottom_kernel<MK, 1>), dim3(1, 1, S), dim3(kBottomLanes), 0, st, ba.b, T);
+        else if (btop && minl == 2)
+            hipLaunchKernelGGL((v_bottom_kernel<MK, 2>), dim3(1, 1, S), dim3(kBottomLanes), 0, st, ba.b, T);
+        else if (btop)
+            hipLaunchKernelGGL((v_bottom_lds_kernel<MK>), dim3(1, 1, S), dim3(1024), bbytes, st, ba, T);
         else if (a.n <= kCoarseLdsMax)
             hipLaunchKernelGGL((v_coarse_lds_kernel<MK>), dim3(1, 1, S), dim3(64), 0, st, a, T, (int)minl, crhs,
                                (double)1.19209290e-07F, (uint64_t)(100 * a.n + 1000));
