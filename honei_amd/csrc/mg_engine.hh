@@ -32,6 +32,12 @@ namespace mg
     constexpr int kMaxLevels = 15;          // levels 0..14 (side 2^L + 1)
     constexpr unsigned kNormBlocks = 1024;  // reduction blocks per slot
     constexpr int kRowCodes = 256;          // distinct matrix rows of a level with row codes
+    // A slot's partial sums: 2 * kNormBlocks of the outer defect and of the
+    // separate norms, then kNormBlocks of an inner solve's opening, then one
+    // per tile of the finest post-smoothing.
+    constexpr unsigned kOpenPartials = 2 * kNormBlocks;
+    constexpr unsigned kCyclePartials = 3 * kNormBlocks;
+    constexpr unsigned kMaxTiles = 16384;
 
     enum Phase : int
     {
@@ -48,9 +54,8 @@ namespace mg
         int outer_active;    // 1 while the outer (FP64) loop runs
         int run;             // 1 while an inner solve runs
         int need_outer;      // the inner solve ended, outer step pending
-        int do_start;        // gates of the current tick (plan_kernel)
-        int do_outer;
         int open;            // an inner solve opens in this tick
+        int clear;           // it is the solve's first (the result array is cleared)
         int status;          // 1: outer step cap reached without convergence
         int zero_guess;      // start from x = 0 instead of the result array
         float alpha;         // correction factor when it is adapted
@@ -74,7 +79,7 @@ namespace mg
     struct Slot
     {
         Scalars * s;
-        double * partials;       // 2 * kNormBlocks
+        double * partials;       // kCyclePartials + the finest level's tiles (at most kMaxTiles)
         const double * b;        // finest right-hand side (FP64)
         double * result;         // finest solution (FP64); holds the initial guess until the start
         double * od;             // outer defect (FP64)

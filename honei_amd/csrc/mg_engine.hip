@@ -145,39 +145,43 @@ namespace
     };
 
     // ------------------------------------------------------------ tick gates
-    __global__ void plan_kernel(const Slot * T, unsigned nslots)
-    {
-        const unsigned z = blockIdx.x * blockDim.x + threadIdx.x;
-        if (z >= nslots)
-            return;
-        Scalars * s = T[z].s;
-        if (s == nullptr)
-            return;
-        const int ph = s->phase;
-        s->do_start = (ph == PH_START) ? 1 : 0;
-        s->do_outer = (ph == PH_SOLVE && s->need_outer) ? 1 : 0;
-        s->open = 0;
-        if (ph == PH_START || ph == PH_SOLVE)
-            s->ticks += 1;
-    }
+    // What a tick does for a slot before its V-cycle follows from the phase
+    // and need_outer, which hold still until outer_defect_finish_kernel: a
+    // start, the FP64 outer step that closes an inner solve, or nothing.
+    __device__ __forceinline__ bool starts(const Scalars * s) { return s->phase == PH_START; }
+    __device__ __forceinline__ bool closes(const Scalars * s) { return s->phase == PH_SOLVE && s->need_outer != 0; }
 
-    // ------------------------------------------------------ start of a solve
-    // result = initial guess (0 or the caller's) with b injected on the first
-    // row, the last row and the first column (multigrid.hh:2282-2297);
-    // x32 of the finest level = (float)result
-    __global__ __launch_bounds__(256) void start_init_kernel(const Slot * T, int L, int64_t n, int64_t sq, int fx)
+    // Start of a solve: result = initial guess (0 or the caller's) with b
+    // injected on the first row, the last row and the first column
+    // (multigrid.hh:2282-2297), x32 of the finest level = (float)result.
+    // Outer step: result += scale * (double)x32.
+    __global__ __launch_bounds__(256) void tick_begin_kernel(const Slot * T, int L, int64_t n, int64_t sq, int fx)
     {
         const VB vb = vblock();
         const Slot & sl = T[vb.z];
-        if (! live(sl) || sl.s->do_start == 0)
+        if (! live(sl))
             return;
-        for (int64_t i = (int64_t)vb.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        const Scalars * s = sl.s;
+        const int64_t i0 = (int64_t)vb.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+        if (starts(s))
         {
-            double g = sl.s->zero_guess ? 0.0 : sl.result[i];
-            if (i < sq || i >= n - sq || (i % sq) == 0)
-                g = sl.b[i];
-            sl.result[i] = g;
-            sl.v[L][fx][i] = (float)g;
+            const bool zero = s->zero_guess != 0;
+            for (int64_t i = i0; i < n; i += stride)
+            {
+                double g = zero ? 0.0 : sl.result[i];
+                if (i < sq || i >= n - sq || (i % sq) == 0)
+                    g = sl.b[i];
+                sl.result[i] = g;
+                sl.v[L][fx][i] = (float)g;
+            }
+        }
+        else if (closes(s))
+        {
+            const double scale = s->scale;
+            const gptr<double> x = as_global(sl.result);
+            const gptr<const float> c = as_global<const float>(sl.v[L][fx]);
+            for (int64_t i = i0; i < n; i += stride)
+                x[i] = x[i] + scale * (double)c[i];
         }
     }
 
@@ -186,7 +190,7 @@ namespace
     {
         const VB vb = vblock();
         const Slot & sl = T[vb.z];
-        if (! live(sl) || sl.s->do_start == 0)
+        if (! live(sl) || ! starts(sl.s))
             return;
         for (int l = minl; l < L; ++l)
             for (int64_t i = (int64_t)vb.x * blockDim.x + threadIdx.x; i < sz.n[l]; i += (int64_t)gridDim.x * blockDim.x)
@@ -194,18 +198,6 @@ namespace
     }
 
     // ------------------------------------------------------- FP64 outer step
-    // result += scale * (double)x32
-    __global__ __launch_bounds__(256) void outer_accumulate_kernel(const Slot * T, int L, int64_t n, int fx)
-    {
-        const VB vb = vblock();
-        const Slot & sl = T[vb.z];
-        if (! live(sl) || sl.s->do_outer == 0)
-            return;
-        const double scale = sl.s->scale;
-        for (int64_t i = (int64_t)vb.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-            sl.result[i] = sl.result[i] + scale * (double)sl.v[L][fx][i];
-    }
-
     // od = b - A64 result and its norm; opens the next inner solve or ends
     // the outer loop.  On a start: the initial defect.  MK 0: Q1 bands B
     // (two rows per lane, 16-byte loads inside); MK 1: the ELL matrix E.
@@ -228,9 +220,7 @@ namespace
         const Slot & sl = T[vb.z];
         if (! live(sl))
             return;
-        Scalars * s = sl.s;
-        const int start = s->do_start;
-        if (start == 0 && s->do_outer == 0)
+        if (! starts(sl.s) && ! closes(sl.s))
             return;
         const double * __restrict__ b = sl.b;
         const double * __restrict__ x = sl.result;
@@ -310,23 +300,37 @@ namespace
     }
 
     // |od| from the partials of outer_defect_kernel (nb blocks per slot), then
-    // the outer step's decisions; one block per slot (blockIdx.z)
+    // the outer step's decisions; one block per slot (blockIdx.z).  Opening an
+    // inner solve starts its V-cycles (run) and, with `fold` (no separate
+    // opening kernels), its cycle count.
     __global__ __launch_bounds__(256) void outer_defect_finish_kernel(const Slot * T, unsigned nb, double outer_eps,
-                                                                      uint64_t max_outer)
+                                                                      uint64_t max_outer, int fold)
     {
         const Slot & sl = T[blockIdx.z];
         if (! live(sl))
             return;
         Scalars * s = sl.s;
-        const int start = s->do_start;
-        if (start == 0 && s->do_outer == 0)
+        const bool start = starts(s);
+        if (! start && ! closes(s))
+        {
+            if (threadIdx.x == 0)
+            {
+                s->open = 0;
+                s->clear = 0;
+                if (s->phase == PH_SOLVE)
+                    s->ticks += 1;
+            }
             return;
+        }
         double dd, unused;
         k::sum_partials2(sl.partials, nb, dd, unused);
         if (threadIdx.x != 0)
             return;
         {
             const double nrm = sqrt(dd);
+            s->ticks += 1;
+            s->open = 0;
+            s->clear = start ? 1 : 0;
             if (start)
             {
                 s->initial_defect = nrm;
@@ -363,24 +367,69 @@ namespace
                         s->open = 1;
                 }
             }
+            if (s->open)
+            {
+                s->run = 1;
+                if (fold)
+                    s->inner_last = 0;
+            }
         }
     }
 
     // rhs32 = (float)(od * inv) (inv == 1 on the first step, so the cast of
-    // the unscaled defect); a start also clears the result array
+    // the unscaled defect); a start also clears the result array.  NORM: block
+    // partials of |rhs32|^2, the initial defect of an inner solve from zero
+    // (four entries per lane; od and rhs32 are the slot's, 16-byte aligned).
+    template <bool NORM>
     __global__ __launch_bounds__(256) void to_inner_kernel(const Slot * T, int L, int64_t n)
     {
         const VB vb = vblock();
         const Slot & sl = T[vb.z];
         if (! live(sl) || sl.s->open == 0)
             return;
+        typedef k::Vec16<double>::type D2;
+        typedef k::Vec16<float>::type F4;
         const double inv = sl.s->inv;
-        const bool clear = sl.s->do_start != 0;
-        for (int64_t i = (int64_t)vb.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        const bool clear = sl.s->clear != 0;
+        const gptr<const double> od = as_global<const double>(sl.od);
+        const gptr<float> rhs = as_global(sl.v[L][F_RHS]);
+        const gptr<double> res = as_global(sl.result);
+        double acc = 0.0;
+        for (int64_t i0 = ((int64_t)vb.x * blockDim.x + threadIdx.x) * 4; i0 < n;
+             i0 += (int64_t)gridDim.x * blockDim.x * 4)
         {
-            sl.v[L][F_RHS][i] = (float)(sl.od[i] * inv);
+            const int cnt = (int)min((int64_t)4, n - i0);
+            if (cnt == 4)
+            {
+                const D2 a = *(gptr<const D2>)(od + i0), b = *(gptr<const D2>)(od + i0 + 2);
+                F4 v;
+                v[0] = (float)(a[0] * inv);
+                v[1] = (float)(a[1] * inv);
+                v[2] = (float)(b[0] * inv);
+                v[3] = (float)(b[1] * inv);
+                *(gptr<F4>)(rhs + i0) = v;
+                if (NORM)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        acc += (double)v[q] * (double)v[q];
+            }
+            else
+                for (int q = 0; q < cnt; ++q)
+                {
+                    const float v = (float)(od[i0 + q] * inv);
+                    rhs[i0 + q] = v;
+                    acc += (double)v * (double)v;
+                }
             if (clear)
-                sl.result[i] = 0.0;
+                for (int q = 0; q < cnt; ++q)
+                    res[i0 + q] = 0.0;
+        }
+        if (NORM)
+        {
+            __shared__ double lds[16];
+            const double t = k::block_sum(acc, lds);
+            if (threadIdx.x == 0)
+                sl.partials[kOpenPartials + vb.x] = t;
         }
     }
 
@@ -420,11 +469,6 @@ namespace
             const float * x = sl.v[L][fx];
             for (int64_t i = lane0; i < n; i += lanes)
                 d[i] = rhs[i] - ell_row<float>(a.E, x, i);
-        }
-        if (vb.x == 0 && threadIdx.x == 0)
-        {
-            sl.s->run = 1;
-            sl.s->need_outer = 0;
         }
     }
 
@@ -524,6 +568,45 @@ namespace
         }
     }
 
+    // The inner stopping test after a V-cycle whose post-smoothing left the
+    // partials of |d|^2 (nd of them); FOLD: the inner solve's initial defect
+    // comes from to_inner_kernel's partials (nr) after its first cycle.
+    // One block per slot (blockIdx.z).
+    template <bool FOLD>
+    __global__ __launch_bounds__(1024) void inner_end_kernel(const Slot * T, unsigned nd, unsigned nr, float tol,
+                                                             uint64_t n_max_iter)
+    {
+        const Slot & sl = T[blockIdx.z];
+        if (! live(sl))
+            return;
+        Scalars * s = sl.s;
+        if (s->run == 0)
+            return;
+        __shared__ double lds[32];
+        const bool first = FOLD && s->inner_last == 0;
+        const gptr<const double> pd = as_global<const double>(sl.partials + kCyclePartials);
+        const gptr<const double> pr = as_global<const double>(sl.partials + kOpenPartials);
+        double d = 0.0, r = 0.0;
+        for (unsigned i = threadIdx.x; i < nd; i += blockDim.x)
+            d += pd[i];
+        if (first)
+            for (unsigned i = threadIdx.x; i < nr; i += blockDim.x)
+                r += pr[i];
+        k::block_sum2(d, r, lds);
+        if (threadIdx.x != 0)
+            return;
+        if (first)
+            s->inner_initial = sqrtf((float)r);
+        const float nrm = sqrtf((float)d);
+        s->inner_defect = nrm;
+        s->inner_last += 1;
+        if (nrm <= s->inner_initial * tol || s->inner_last >= n_max_iter)
+        {
+            s->run = 0;
+            s->need_outer = 1;
+        }
+    }
+
     // one-level hierarchy: the cycle loop is left after the coarse solve
     __global__ void one_level_end_kernel(const Slot * T, unsigned nslots)
     {
@@ -608,6 +691,7 @@ namespace
     // of them), so the height is the even th <= 128 with the fewest rounds of
     // steps, ceil(tiles / resident) * (th + 6), where `resident` tiles fit on
     // the device at once (the larger th on a tie: fewer halo rows).
+    // At most kMaxTiles tiles (a slot's room for their partial sums).
     template <int V> int march_rows(int64_t m, unsigned slots, unsigned resident)
     {
         int best = 2;
@@ -615,6 +699,8 @@ namespace
         for (int th = 2; th <= 128; th += 2)
         {
             const uint64_t tiles = (uint64_t)march_tiles<V>(m, th) * slots;
+            if (tiles > (uint64_t)slots * kMaxTiles)
+                continue;
             const uint64_t rounds = (tiles + resident - 1) / resident;
             const uint64_t cost = rounds * (uint64_t)(th + 6);
             if (cost <= best_cost)
@@ -1617,10 +1703,20 @@ void hierarchy_alloc_ell(Hierarchy & h, const Params & p, uint64_t max_level, co
     h.ell64[max_level] = upload_ell<double>(h, A64);
 }
 
+namespace
+{
+    // doubles of a slot's partial sums, finest level of side m: the regions
+    // named in mg_engine.hh
+    uint64_t slot_partials(int64_t m)
+    {
+        return kCyclePartials + std::min<uint64_t>(kMaxTiles, march_tiles<1>(m, 2));
+    }
+}
+
 uint64_t slot_bytes(const Hierarchy & h, uint64_t L, bool own_b, bool own_result)
 {
     const uint64_t n = h.lv[L].n;
-    uint64_t b = align256(sizeof(Scalars)) + align256(sizeof(double) * 2 * kNormBlocks);
+    uint64_t b = align256(sizeof(Scalars)) + align256(sizeof(double) * slot_partials(h.lv[L].side));
     b += align256(sizeof(double) * n);                                  // od
     if (own_b)
         b += align256(sizeof(double) * n);
@@ -1644,7 +1740,7 @@ Slot slot_carve(const Hierarchy & h, uint64_t L, char * base, bool own_b, bool o
         return r;
     };
     sl.s = (Scalars *)take(sizeof(Scalars));
-    sl.partials = (double *)take(sizeof(double) * 2 * kNormBlocks);
+    sl.partials = (double *)take(sizeof(double) * slot_partials(h.lv[L].side));
     sl.od = (double *)take(sizeof(double) * n);
     if (own_b)
         sl.b = (const double *)take(sizeof(double) * n);
@@ -1784,26 +1880,27 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
         }
     }
 
-    // ---- gates, start of new solves, FP64 outer step, opening of inner solves
-    hipLaunchKernelGGL(plan_kernel, dim3(grid_for(S, 64)), dim3(64), 0, st, T, S);
+    // ---- start of new solves, FP64 outer step, opening of inner solves
     // the per-tick kernels that most ticks skip (start, outer step, opening
     // of an inner solve) loop over their rows on a capped grid, so a skipped
     // launch costs a few thousand empty workgroups, not one per 256 rows
     auto ggrid = [&](uint64_t blocks) {
         return dim3((unsigned)std::min<uint64_t>(blocks, std::max<unsigned>(64u, kGateBlocks / S)), 1, S);
     };
-    hipLaunchKernelGGL(start_init_kernel, ggrid(grid_for(top.n, kBlock)), blk, 0, st, T, (int)maxl, n,
-                       top.side, fx_top);
-    if (maxl > minl)
+    // The opening of an inner solve folded into its neighbours: the cast to
+    // FP32 forms the initial norm, the first cycle reads rhs as its defect
+    // (initial_zero) and the first stopping test finishes the norm.
+    const bool fold = pre2r && p.initial_zero && ! p.convergence_check;
+    hipLaunchKernelGGL(tick_begin_kernel, ggrid(grid_for(top.n, kBlock)), blk, 0, st, T, (int)maxl, n, top.side, fx_top);
+    if (maxl > minl && ! pre2r)
     {
+        // (the one-pass kernels write every coarser iterate before it is read)
         LevelSizes sz;
         for (int l = 0; l < kMaxLevels; ++l)
             sz.n[l] = (int64_t)h.lv[l].n;
         hipLaunchKernelGGL(start_zero_kernel, ggrid(grid_for(h.lv[maxl - 1].n, kBlock)), blk, 0, st, T,
                            (int)minl, (int)maxl, sz);
     }
-    hipLaunchKernelGGL(outer_accumulate_kernel, ggrid(grid_for(top.n, kBlock)), blk, 0, st, T, (int)maxl, n,
-                       fx_top);
     const unsigned od_blocks = std::min<unsigned>(grid_for((top.n + 1) / 2, kBlock), kNormBlocks);
     bool od_coded = false;
     if constexpr (MK == 0)
@@ -1821,17 +1918,26 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
                            kBands<MK> ? h.B64(maxl) : k::Bands{}, h.ell64[maxl], T, n, top.side,
                            (const uint64_t *)nullptr, (const double *)nullptr);
     hipLaunchKernelGGL(outer_defect_finish_kernel, dim3(1, 1, S), blk, 0, st, T, od_blocks, (double)p.tolerance,
-                       p.max_outer);
-    hipLaunchKernelGGL(to_inner_kernel, ggrid(grid_for(top.n, kBlock)), blk, 0, st, T, (int)maxl, n);
-    if (p.initial_zero)
-        hipLaunchKernelGGL((open_inner_kernel<1, MK>), ggrid(lanes4(top.n)), blk, 0, st, largs(maxl), T,
-                           (int)maxl, fx_top);
+                       p.max_outer, fold ? 1 : 0);
+    unsigned open_blocks = 0;
+    if (fold)
+    {
+        open_blocks = std::min<unsigned>(ggrid(lanes4(top.n)).x, kNormBlocks);
+        hipLaunchKernelGGL((to_inner_kernel<true>), dim3(open_blocks, 1, S), blk, 0, st, T, (int)maxl, n);
+    }
     else
-        hipLaunchKernelGGL((open_inner_kernel<0, MK>), ggrid(rgrid(top.n)), blk, 0, st, largs(maxl), T,
-                           (int)maxl, fx_top);
-    hipLaunchKernelGGL((inner_norm_kernel<0>), norm_grid(top.n), blk, 0, st, T, (int)maxl, n);
-    hipLaunchKernelGGL((inner_norm_finish_kernel<0>), dim3(1, 1, S), blk, 0, st, T, norm_grid(top.n).x, p.tolerance,
-                       p.convergence_check, p.n_max_iter);
+    {
+        hipLaunchKernelGGL((to_inner_kernel<false>), ggrid(lanes4(top.n)), blk, 0, st, T, (int)maxl, n);
+        if (p.initial_zero)
+            hipLaunchKernelGGL((open_inner_kernel<1, MK>), ggrid(lanes4(top.n)), blk, 0, st, largs(maxl), T,
+                               (int)maxl, fx_top);
+        else
+            hipLaunchKernelGGL((open_inner_kernel<0, MK>), ggrid(rgrid(top.n)), blk, 0, st, largs(maxl), T,
+                               (int)maxl, fx_top);
+        hipLaunchKernelGGL((inner_norm_kernel<0>), norm_grid(top.n), blk, 0, st, T, (int)maxl, n);
+        hipLaunchKernelGGL((inner_norm_finish_kernel<0>), dim3(1, 1, S), blk, 0, st, T, norm_grid(top.n).x,
+                           p.tolerance, p.convergence_check, p.n_max_iter);
+    }
 
     // ---- one V-cycle (multigrid.hh:1660-1905)
     const uint64_t npre = p.n_pre_smooth;
@@ -1878,7 +1984,7 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
                         const int th = march_rows<VS>(a.m, groups, kMarchWaves * post_resident((const void *)kern));
                         const unsigned tiles = march_tiles<VS>(a.m, th);
                         hipLaunchKernelGGL(kern, dim3((tiles + kMarchWaves - 1) / kMarchWaves, 1, groups), blk, 0, st,
-                                           a, T, (int)L, dsrc, ACC ? fx_top : (int)F_X, Nc, p.mask, th, tiles, (int)S);
+                                           a, T, (int)L, ACC ? fx_top : (int)F_X, Nc, p.mask, th, tiles, (int)S, fold ? 1 : 0);
                     };
                     if (L == maxl)
                         march_form(a, [&](auto k_tag, auto v_tag, auto cb_tag) { go(IntC<1>{}, k_tag, v_tag, cb_tag); });
@@ -1959,6 +2065,7 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
         }
     }
     // v_post2_kernel on level L (DEFECT on the finest)
+    unsigned cycle_tiles = 0;
     auto post2_launch = [&](uint64_t L, const LevelArgs & a, int fcoarse, float alpha, auto prol_tag) {
         constexpr int PROL = decltype(prol_tag)::value;
         auto go = [&](auto def_tag, auto k_tag, auto v_tag, auto cb_tag) {
@@ -1968,6 +2075,8 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
             const unsigned groups = (S + KS - 1) / KS;
             const int th = march_rows<VS>(a.m, groups, kMarchWaves * post_resident((const void *)kern));
             const unsigned tiles = march_tiles<VS>(a.m, th);
+            if (DEF)
+                cycle_tiles = tiles;
             hipLaunchKernelGGL(kern, dim3((tiles + kMarchWaves - 1) / kMarchWaves, 1, groups), blk, 0, st, a, T, (int)L,
                                (int)F_X, (int)F_TMP, fcoarse, alpha, p.mask, th, tiles, (int)S);
         };
@@ -2034,9 +2143,18 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
         if (L == maxl)
             defect(L);
     }
-    hipLaunchKernelGGL((inner_norm_kernel<1>), norm_grid(top.n), blk, 0, st, T, (int)maxl, n);
-    hipLaunchKernelGGL((inner_norm_finish_kernel<1>), dim3(1, 1, S), blk, 0, st, T, norm_grid(top.n).x, p.tolerance,
-                       p.convergence_check, p.n_max_iter);
+    if (fold)
+        hipLaunchKernelGGL((inner_end_kernel<true>), dim3(1, 1, S), dim3(1024), 0, st, T, cycle_tiles, open_blocks,
+                           p.tolerance, p.n_max_iter);
+    else if (post2)
+        hipLaunchKernelGGL((inner_end_kernel<false>), dim3(1, 1, S), dim3(1024), 0, st, T, cycle_tiles, 0u, p.tolerance,
+                           p.n_max_iter);
+    else
+    {
+        hipLaunchKernelGGL((inner_norm_kernel<1>), norm_grid(top.n), blk, 0, st, T, (int)maxl, n);
+        hipLaunchKernelGGL((inner_norm_finish_kernel<1>), dim3(1, 1, S), blk, 0, st, T, norm_grid(top.n).x,
+                           p.tolerance, p.convergence_check, p.n_max_iter);
+    }
     HIP_CHECK(hipGetLastError());
 }
 }  // namespace

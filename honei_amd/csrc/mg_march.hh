@@ -494,7 +494,8 @@ namespace
 
     // ------------------------------------------- post-smoothing in one pass
     // Two damped-Jacobi sweeps x1 = x + dinv (rhs - A x), x2 = x1 + dinv (rhs
-    // - A x1) and, with DEFECT, d = rhs - A x2.  PROL: x is first corrected
+    // - A x1) and, with DEFECT, d = rhs - A x2 and the tile's |d|^2 (a partial
+    // sum of the slot).  PROL: x is first corrected
     // by alpha P(level L-1's field fcoarse).  x2 goes to field fout (not fx:
     // neighbouring tiles read x around their own rows).  Every value is the
     // one the separate kernels form.
@@ -539,6 +540,7 @@ namespace
             MarchProl<V, EDGE> prol[K];
             float xr[K][3][V] = {}, x1r[K][3][V] = {}, x2r[K][3][V] = {}, rr[K][3][V] = {};
             float xn[K][3][V], rn[K][3][V];
+            double dd[K] = {};                // |d|^2 over the lane's stored nodes
             auto load = [&](int I, int s) {
 #pragma unroll
                 for (int q = 0; q < K; ++q)
@@ -622,7 +624,13 @@ namespace
                                 d[o] = rr[q][O][o] - sum;
                             }
                             if (sl.on[q] && r3 >= r0 && r3 < r0 + H)
+                            {
                                 march_store<V, EDGE>(t, dout[q], r3, d);
+#pragma unroll
+                                for (int o = 0; o < V; ++o)
+                                    if (t.own(o))
+                                        dd[q] += (double)d[o] * (double)d[o];
+                            }
                         }
                     }
                 };
@@ -651,6 +659,14 @@ namespace
                 step(IntC<1>{}, s + 1);
                 step(IntC<2>{}, s + 2);
             }
+            if (DEFECT)
+#pragma unroll
+                for (int q = 0; q < K; ++q)
+                {
+                    const double sum = k::wave_sum(dd[q]);
+                    if (sl.on[q] && t.lane == 0)
+                        T[sl.at[q]].partials[kCyclePartials + tile] = sum;
+                }
         };
         if (t.edge)
             march(std::true_type{});
@@ -664,14 +680,14 @@ namespace
     // rhs - A x and the coarse right-hand side Restriction<NONE>(d') with the
     // Dirichlet mask.  Every value is the one the separate kernels form; d'
     // is never stored.  th is even, so a tile's first row is even and it owns
-    // the coarse rows r with 2r in its rows.  ACC 0: d is field F_RHS itself.
+    // the coarse rows r with 2r in its rows.
     //
     // Step s takes d and the matrix at row r0 + s - 3 (loaded three steps
     // ahead), forms c1 there, x at row s - 4 and d' at s - 5, and, when that
     // row is 2r + 1, coarse row r.
     template <int MK, int ACC, int K, int V, int CB>
-    __global__ __launch_bounds__(64 * kMarchWaves) void v_pre2r_kernel(LevelArgs a, const Slot * T, int L, int fd,
-            int facc, int64_t Nc64, k::Mask mk, int th, unsigned tiles, int nslots)
+    __global__ __launch_bounds__(64 * kMarchWaves) void v_pre2r_kernel(LevelArgs a, const Slot * T, int L, int facc,
+            int64_t Nc64, k::Mask mk, int th, unsigned tiles, int nslots, int fold)
     {
         const VB vb = vblock();
         MarchSlots<K> sl;
@@ -692,7 +708,10 @@ namespace
         for (int q = 0; q < K; ++q)
         {
             const Slot & z = T[sl.at[q]];
-            d[q] = as_global<const float>(z.v[L][ACC ? fd : (int)F_RHS]);
+            // d is field F_D on the finest level (ACC), but rhs itself in an
+            // inner solve's first cycle where no F_D was written (fold)
+            const bool from_rhs = ! ACC || (fold && z.s->inner_last == 0);
+            d[q] = as_global<const float>(z.v[L][from_rhs ? F_RHS : F_D]);
             rhs[q] = as_global<const float>(z.v[L][F_RHS]);
             acc[q] = as_global<const float>(z.v[L][facc]);
             xo[q] = as_global<float>(z.v[L][F_X]);
