@@ -424,13 +424,31 @@ namespace
 
     // the level's table (CB 1: its distinct rows; CB 2: its values) in LDS
     template <int CB> constexpr int kTabFloats = CB == 1 ? 12 * kRowCodes : (CB == 2 ? 160 : 4);
-    template <int CB> __device__ __forceinline__ void march_table(const LevelArgs & a, float * tab)
+    // (fetch: the lane's first entry, loaded while the slot's pointers are
+    // still on their way; store: to LDS)
+    template <int CB> __device__ __forceinline__ int tab_count(const LevelArgs & a)
     {
-        const float * src = CB == 1 ? a.rtab : a.ctab;
-        const int cnt = CB == 1 ? 12 * a.rows : 160;
-        for (int q = threadIdx.x; q < cnt; q += 64 * kMarchWaves)
-            tab[q] = src[q];
-        __syncthreads();
+        return CB == 1 ? 12 * a.rows : (CB == 2 ? 160 : 0);
+    }
+    template <int CB> __device__ __forceinline__ float march_table_fetch(const LevelArgs & a)
+    {
+        if constexpr (CB == 0)
+            return 0.0f;
+        else
+            return as_global<const float>(CB == 1 ? a.rtab : a.ctab)[min((int)threadIdx.x, tab_count<CB>(a) - 1)];
+    }
+    template <int CB> __device__ __forceinline__ void march_table_store(const LevelArgs & a, float first, float * tab)
+    {
+        if constexpr (CB != 0)
+        {
+            const gptr<const float> src = as_global<const float>(CB == 1 ? a.rtab : a.ctab);
+            const int cnt = tab_count<CB>(a);
+            if ((int)threadIdx.x < cnt)
+                tab[threadIdx.x] = first;
+            for (int q = threadIdx.x + 64 * kMarchWaves; q < cnt; q += 64 * kMarchWaves)
+                tab[q] = src[q];
+            lds_barrier();
+        }
     }
     template <int V, int CB>
     __device__ __forceinline__ void march_matrix(MarchRows<V, CB> & rows, const LevelArgs & a, const float * tab)
@@ -508,12 +526,12 @@ namespace
             int fout, int fcoarse, float alpha, k::Mask mk, int th, unsigned tiles, int nslots)
     {
         const VB vb = vblock();
+        const float tab0 = march_table_fetch<CB>(a);
         MarchSlots<K> sl;
         if (! sl.find(T, vb.z, nslots))
             return;
         __shared__ __align__(16) float tab[kTabFloats<CB>];
-        if constexpr (CB != 0)
-            march_table<CB>(a, tab);
+        march_table_store<CB>(a, tab0, tab);
         const unsigned blk = gridDim.z == 1 ? k::xcd_block(vb.x, gridDim.x) : vb.x;
         const unsigned tile = blk * kMarchWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         if (tile >= tiles)
@@ -574,7 +592,8 @@ namespace
                 load(I, s + 3);
                 const int r1 = r0 + s - 4, r2 = r1 - 1, r3 = r1 - 2;
                 // stage rows 2 .. m - 3: every neighbour of every lane's node
-                // lies in the matrix
+                // lies in the matrix (a first step's stages whose rows have
+                // not entered yet form values that no stored one depends on)
                 const bool inside = r3 >= 2 && r1 <= m - 3;
                 // coef(J, o, b): the matrix row of ring entry J in column o
                 auto stage = [&](auto g_tag, auto && coef) {
@@ -635,7 +654,7 @@ namespace
                     }
                 };
                 auto look_up = [&](int J, int o, float (&b)[10]) { rows.row(J, o, b); };
-                if (same && inside && s >= 6)
+                if (same && inside)
                 {
                     if constexpr (CB == 1)
                         stage(std::false_type{}, [&](int, int o, float (&b)[10]) {
@@ -690,12 +709,12 @@ namespace
             int64_t Nc64, k::Mask mk, int th, unsigned tiles, int nslots, int fold)
     {
         const VB vb = vblock();
+        const float tab0 = march_table_fetch<CB>(a);
         MarchSlots<K> sl;
         if (! sl.find(T, vb.z, nslots))
             return;
         __shared__ __align__(16) float tab[kTabFloats<CB>];
-        if constexpr (CB != 0)
-            march_table<CB>(a, tab);
+        march_table_store<CB>(a, tab0, tab);
         const unsigned blk = gridDim.z == 1 ? k::xcd_block(vb.x, gridDim.x) : vb.x;
         const unsigned tile = blk * kMarchWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         if (tile >= tiles)
@@ -806,7 +825,7 @@ namespace
                     }
                 };
                 auto look_up = [&](int J, int o, float (&b)[10]) { rows.row(J, o, b); };
-                if (same && inside && s >= 4)
+                if (same && inside)
                 {
                     if constexpr (CB == 1)
                         stage(std::false_type{}, [&](int, int o, float (&b)[10]) {
