@@ -27,6 +27,13 @@ namespace hsolve
 namespace
 {
     constexpr int kSolverBlocks = 2048;   // fixed grid of the fused reduction kernels
+    constexpr int kMaxDevices = 64;
+    // Systems that may be solved in one cooperative launch (solvers_persist.hh):
+    // at most one row per thread of the fixed grid; their device scratch is
+    // three sets, used in turn, of two partials per block, and a flag.
+    constexpr uint64_t kPersistRows = 256 * (uint64_t)kSolverBlocks;
+    constexpr size_t kPersistSums = 3 * 2 * kSolverBlocks;
+    constexpr size_t kPersistBytes = sizeof(uint64_t) * (kPersistSums + 8);
 
     // --------------------------------------------------------------- operators
     // A row of y = A x for the fused kernels.
@@ -427,6 +434,22 @@ namespace
     }
 
     // beta = (z.r) / (r.z)_old; the stopping test ||r|| < eps ||r0|| or the cap
+    template <typename DT> __device__ __forceinline__ void jac_test(CgScalars<DT> & s, double zr, double rr)
+    {
+        s.talpha = div_guard<DT>((DT)zr, s.temp);
+        s.temp = (DT)zr;
+        ++s.iters;
+        const DT cur = (DT)sqrt((DT)rr);
+        s.current_defect = cur;
+        if (cur < s.initial_defect * s.eps_relative)
+        {
+            s.converged = 1;
+            s.run = 0;
+        }
+        else if (s.iters == s.max_iters)
+            s.run = 0;
+    }
+
     template <typename DT>
     __global__ __launch_bounds__(256) void jac_update_finish(const double * partials, unsigned nb,
                                                              CgScalars<DT> * s)
@@ -437,18 +460,9 @@ namespace
         k::sum_partials2(partials, nb, zr, rr);
         if (threadIdx.x != 0)
             return;
-        s->talpha = div_guard<DT>((DT)zr, s->temp);
-        s->temp = (DT)zr;
-        ++s->iters;
-        const DT cur = (DT)sqrt((DT)rr);
-        s->current_defect = cur;
-        if (cur < s->initial_defect * s->eps_relative)
-        {
-            s->converged = 1;
-            s->run = 0;
-        }
-        else if (s->iters == s->max_iters)
-            s->run = 0;
+        CgScalars<DT> t = *s;
+        jac_test<DT>(t, zr, rr);
+        *s = t;
     }
 
     // d = z + beta d (ScaledSum(d, z, temp_0, beta) with temp_0 a copy of d)
@@ -526,6 +540,7 @@ namespace
         DT * p2 = nullptr;                // the other direction buffer of cg_spmv_dir_kernel
         double * partials = nullptr;
         double * partials2 = nullptr;     // a second set, for kernels that read one set and write the other
+        uint64_t * sums = nullptr;        // scratch of the one-launch solve (systems of at most kPersistRows)
         CgScalars<DT> * s = nullptr;
         void * block = nullptr;
         bool owned = false;
@@ -533,7 +548,8 @@ namespace
         static size_t vector_bytes(uint64_t n) { return ((sizeof(DT) * n + 255) / 256) * 256; }
         static size_t bytes_for(uint64_t n)
         {
-            return 4 * vector_bytes(n) + sizeof(double) * 4 * kSolverBlocks + sizeof(CgScalars<DT>) + 256;
+            return 4 * vector_bytes(n) + sizeof(double) * 4 * kSolverBlocks + sizeof(CgScalars<DT>) + 256 +
+                   (n <= kPersistRows ? kPersistBytes : 0);
         }
 
         explicit CgWork(uint64_t n, void * external = nullptr)
@@ -555,6 +571,11 @@ namespace
             p2 = (DT *)c; c += vb;
             partials = (double *)c; c += sizeof(double) * 2 * kSolverBlocks;
             partials2 = (double *)c; c += sizeof(double) * 2 * kSolverBlocks;
+            if (n <= kPersistRows)
+            {
+                sums = (uint64_t *)c;
+                c += kPersistBytes;
+            }
             s = (CgScalars<DT> *)c;
         }
         ~CgWork()
@@ -564,12 +585,37 @@ namespace
         }
     };
 
+#include "solvers_persist.hh"
+
+    template <typename DT> PersistMatrix persist_matrix(const Q1Op<DT> & A)
+    {
+        PersistMatrix m{};
+        m.B = A.B;
+        m.m = A.m;
+        return m;
+    }
+    template <typename DT, typename IT, typename LT> PersistMatrix persist_matrix(const EllOp<DT, IT, LT> & A)
+    {
+        PersistMatrix m{};
+        m.Aj = A.Aj;
+        m.Ax = A.Ax;
+        m.Arl = A.Arl;
+        m.idx_kind = std::is_signed<IT>::value ? 1 : 0;
+        m.len_bytes = (int)sizeof(LT);
+        m.stride = A.stride;
+        return m;
+    }
+    template <typename DT> constexpr bool is_q1(const Q1Op<DT> &) { return true; }
+    template <typename DT, typename IT, typename LT> constexpr bool is_q1(const EllOp<DT, IT, LT> &) { return false; }
+
+    // width: the longest row of an ELL matrix with one lane per row (0: the
+    // one-launch solve is not tried); Q1 matrices give 9
     // work: NULL (the workspace is allocated for this solve) or a device
     // block of at least CgWork<DT>::bytes_for(n) bytes
     template <typename DT, typename Op, bool VAR>
     void run_cg(const Op & A, uint64_t n, const DT * b, DT * x, const DT * P, uint64_t max_iters, double eps,
-                uint64_t * used_iters, double * defect_out, hipStream_t st, int * converged_out, int plain = 0,
-                void * work = nullptr)
+                uint64_t * used_iters, double * defect_out, hipStream_t st, int * converged_out, uint64_t width,
+                int plain = 0, void * work = nullptr)
     {
         CgWork<DT> w(n, work);
         CgScalars<DT> h;
@@ -577,14 +623,36 @@ namespace
         h.eps_relative = (DT)eps;
         h.max_iters = max_iters;
         h.plain = plain;
-        HIP_CHECK(hipMemcpyAsync(w.s, &h, sizeof(h), hipMemcpyHostToDevice, st));
+        const CgScalars<DT> h0 = h;
         const unsigned grid = std::min<unsigned>(grid_for(n, kBlock), kSolverBlocks);
         const bool fused = grid <= 512;
-        hipLaunchKernelGGL((cg_init_kernel<DT, Op, VAR>), dim3(grid), dim3(kBlock), 0, st, A, b, x, w.r, w.p, P,
-                           (int64_t)n, w.partials);
-        hipLaunchKernelGGL((cg_init_finish<DT, VAR>), dim3(1), dim3(kBlock), 0, st, (const double *)w.partials, grid,
-                           w.s);
-        HIP_CHECK(hipGetLastError());
+        auto start = [&] {
+            HIP_CHECK(hipMemcpyAsync(w.s, &h0, sizeof(h0), hipMemcpyHostToDevice, st));
+            hipLaunchKernelGGL((cg_init_kernel<DT, Op, VAR>), dim3(grid), dim3(kBlock), 0, st, A, b, x, w.r, w.p, P,
+                               (int64_t)n, w.partials);
+            hipLaunchKernelGGL((cg_init_finish<DT, VAR>), dim3(1), dim3(kBlock), 0, st, (const double *)w.partials,
+                               grid, w.s);
+            HIP_CHECK(hipGetLastError());
+        };
+        auto finish = [&] {
+            if (used_iters)
+                *used_iters = h.iters;
+            if (defect_out)
+                *defect_out = (h.initial_defect > 0) ? (double)h.current_defect / (double)h.initial_defect
+                                                     : (double)h.current_defect;
+            if (converged_out)
+                *converged_out = h.converged;
+        };
+        start();
+        if (width != 0)
+        {
+            const PersistEnd e = run_persist<DT, VAR ? PK_VAR : PK_NONE>(persist_matrix(A), is_q1(A), width, w, x, P,
+                                                                         n, &h, st);
+            if (e == PE_DONE)
+                return finish();
+            if (e == PE_GAVE_UP)
+                start();
+        }
         // chunks of iterations between host checks; every kernel of an
         // iteration that starts after the stop is a no-op
         uint64_t enqueued = 0;
@@ -656,13 +724,7 @@ namespace
                     chunk *= 2;
             }
         }
-        if (used_iters)
-            *used_iters = h.iters;
-        if (defect_out)
-            *defect_out = (h.initial_defect > 0) ? (double)h.current_defect / (double)h.initial_defect
-                                                 : (double)h.current_defect;
-        if (converged_out)
-            *converged_out = h.converged;
+        finish();
     }
 
     k::Bands bands9(const void * const * b)
@@ -681,7 +743,7 @@ namespace
     // z has its own vector.
     template <typename DT, typename Op>
     void run_pcg_jac(const Op & A, uint64_t n, const DT * b, DT * x, const DT * dd, uint64_t max_iters, double eps,
-                     uint64_t * used_iters, double * defect_out, hipStream_t st, int * converged_out)
+                     uint64_t * used_iters, double * defect_out, hipStream_t st, int * converged_out, uint64_t width)
     {
         CgWork<DT> w(n);
         DeviceArray<DT> zbuf(n);
@@ -690,13 +752,34 @@ namespace
         std::memset(&h, 0, sizeof(h));
         h.eps_relative = (DT)eps;
         h.max_iters = max_iters;
-        HIP_CHECK(hipMemcpyAsync(w.s, &h, sizeof(h), hipMemcpyHostToDevice, st));
+        const CgScalars<DT> h0 = h;
         const unsigned grid = std::min<unsigned>(grid_for(n, kBlock), kSolverBlocks);
-        hipLaunchKernelGGL((jac_init_kernel<DT, Op>), dim3(grid), dim3(kBlock), 0, st, A, b, (const DT *)x, dd, w.r,
-                           z, w.p, (int64_t)n, w.partials);
-        hipLaunchKernelGGL((jac_init_finish<DT>), dim3(1), dim3(kBlock), 0, st, (const double *)w.partials, grid,
-                           w.s);
-        HIP_CHECK(hipGetLastError());
+        auto start = [&] {
+            HIP_CHECK(hipMemcpyAsync(w.s, &h0, sizeof(h0), hipMemcpyHostToDevice, st));
+            hipLaunchKernelGGL((jac_init_kernel<DT, Op>), dim3(grid), dim3(kBlock), 0, st, A, b, (const DT *)x, dd,
+                               w.r, z, w.p, (int64_t)n, w.partials);
+            hipLaunchKernelGGL((jac_init_finish<DT>), dim3(1), dim3(kBlock), 0, st, (const double *)w.partials, grid,
+                               w.s);
+            HIP_CHECK(hipGetLastError());
+        };
+        auto finish = [&] {
+            if (used_iters)
+                *used_iters = h.iters;
+            if (defect_out)
+                *defect_out = (h.initial_defect > 0) ? (double)h.current_defect / (double)h.initial_defect
+                                                     : (double)h.current_defect;
+            if (converged_out)
+                *converged_out = h.converged;
+        };
+        start();
+        if (width != 0)
+        {
+            const PersistEnd e = run_persist<DT, PK_JAC>(persist_matrix(A), is_q1(A), width, w, x, dd, n, &h, st);
+            if (e == PE_DONE)
+                return finish();
+            if (e == PE_GAVE_UP)
+                start();
+        }
         uint64_t enqueued = 0, chunk = 8;
         // small grids (launch-bound solves): three launches per iteration, as
         // run_cg; pv[cp] holds the current direction
@@ -758,14 +841,11 @@ namespace
             if (chunk < 64)
                 chunk *= 2;
         }
-        if (used_iters)
-            *used_iters = h.iters;
-        if (defect_out)
-            *defect_out = (h.initial_defect > 0) ? (double)h.current_defect / (double)h.initial_defect
-                                                 : (double)h.current_defect;
-        if (converged_out)
-            *converged_out = h.converged;
+        finish();
     }
+
+    // `width` of run_cg and run_pcg_jac for a handle
+    uint64_t persist_width(const hsolve_ell_s * m) { return m->threads == 1 && m->rows > 0 ? m->ncpr : 0; }
 
     template <typename DT, bool VAR>
     void run_cg_ell(const hsolve_ell_s * m, const DT * b, DT * x, const DT * P, uint64_t max_iters, double eps,
@@ -777,7 +857,8 @@ namespace
             using IT = std::remove_const_t<std::remove_pointer_t<decltype(Aj)>>;
             using LT = std::remove_const_t<std::remove_pointer_t<decltype(Arl)>>;
             EllOp<DT, IT, LT> A{Aj, (const DT *)m->Ax, Arl, m->stride, (uint32_t)m->threads};
-            run_cg<DT, EllOp<DT, IT, LT>, VAR>(A, n, b, x, P, max_iters, eps, used, defect, st, conv, plain, work);
+            run_cg<DT, EllOp<DT, IT, LT>, VAR>(A, n, b, x, P, max_iters, eps, used, defect, st, conv,
+                                               persist_width(m), plain, work);
         });
     }
 
@@ -918,7 +999,6 @@ namespace
     constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
     static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
-    constexpr int kMaxDevices = 64;
     std::mutex g_scratch_mutex;
     void * g_scratch_ptr[kMaxDevices] = {};
 
@@ -962,13 +1042,13 @@ int hsolve_cg_q1(int dtype, const void * const * bands, uint64_t size, const voi
     {
         Q1Op<double> A{bands9(bands), (int64_t)size, m};
         run_cg<double, Q1Op<double>, false>(A, size, (const double *)b, (double *)x, nullptr, max_iters, eps,
-                                            used_iters, defect_out, st, &conv);
+                                            used_iters, defect_out, st, &conv, 9);
     }
     else
     {
         Q1Op<float> A{bands9(bands), (int64_t)size, m};
         run_cg<float, Q1Op<float>, false>(A, size, (const float *)b, (float *)x, nullptr, max_iters, eps, used_iters,
-                                          defect_out, st, &conv);
+                                          defect_out, st, &conv, 9);
     }
     if (! conv && max_iters > 0)
     {
@@ -1014,13 +1094,13 @@ int hsolve_pcg_jac_ell(hsolve_ell m, const void * dd_inverted, const void * b, v
         {
             EllOp<double, IT, LT> A{Aj, (const double *)m->Ax, Arl, m->stride, (uint32_t)m->threads};
             run_pcg_jac<double>(A, m->rows, (const double *)b, (double *)x, (const double *)dd_inverted, max_iters,
-                                eps, used_iters, defect_out, st, &conv);
+                                eps, used_iters, defect_out, st, &conv, persist_width(m));
         }
         else
         {
             EllOp<float, IT, LT> A{Aj, (const float *)m->Ax, Arl, m->stride, (uint32_t)m->threads};
             run_pcg_jac<float>(A, m->rows, (const float *)b, (float *)x, (const float *)dd_inverted, max_iters,
-                               eps, used_iters, defect_out, st, &conv);
+                               eps, used_iters, defect_out, st, &conv, persist_width(m));
         }
     });
     if (! conv && max_iters > 0)
