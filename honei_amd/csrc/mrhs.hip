@@ -39,7 +39,7 @@ namespace
     constexpr int kMaxCols = 64;           // columns of a multivector (one per lane)
     constexpr int kTileK = 16;             // most ELL slots per row a tile keeps in registers
     constexpr unsigned kMvBlocks = 2048;   // grid cap of the multivector kernels
-    constexpr int kFinThreads = 1024;      // threads of the one-block finish launches
+    constexpr int kFinThreads = 256;       // threads of the finish launches (one block per column)
 
     template <typename DT, typename IT, typename LT> struct MvEll
     {
@@ -149,6 +149,49 @@ namespace
         }
     }
 
+    // The slots of a tile's rows (lane l: row base + l) of a Q1-structured
+    // matrix in their 9 neighbour positions: values and presence bits.
+    template <typename DT, typename IT, typename LT>
+    __device__ __forceinline__ void q1_slots(const MvEll<DT, IT, LT> & A, int64_t base, DT (&ap)[9], uint32_t & mask)
+    {
+        const int lane = threadIdx.x & 63;
+        const int64_t n = A.n, M = A.q1_side;
+        const int64_t myrow = base + lane;
+        const uint32_t self = myrow < n ? (uint32_t)myrow : 0u;
+        const uint32_t len = myrow < n ? (uint32_t)A.Arl[myrow] : 0u;
+        IT rc[9];
+        DT ra[9];
+#pragma unroll
+        for (int kk = 0; kk < 9; ++kk)
+        {
+            rc[kk] = IT(0);
+            ra[kk] = DT(0);
+            if ((uint32_t)kk < A.ncpr)
+            {
+                const uint64_t at = (uint64_t)kk * A.stride + (uint64_t)self;
+                rc[kk] = k::ld_stream(A.Aj + at);
+                ra[kk] = k::ld_stream(A.Ax + at);
+            }
+        }
+        mask = 0;
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+            ap[q] = DT(0);
+#pragma unroll
+        for (int kk = 0; kk < 9; ++kk)
+        {
+            if ((uint32_t)kk < len)
+            {
+                const int64_t d = (int64_t)k::col_of<IT>(rc[kk], (uint64_t)myrow) - myrow;
+                const int p = d < -1 ? (int)(d + M) + 1 : (d > 1 ? (int)(d - M) + 7 : (int)d + 4);
+#pragma unroll
+                for (int q = 0; q < 9; ++q)
+                    ap[q] = (p == q) ? ra[kk] : ap[q];
+                mask |= 1u << p;
+            }
+        }
+    }
+
     // The same for Q1-structured matrices (every stored column of row
     // (y, x) is a neighbour (y + dy, x + dx), |dy|, |dx| <= 1, ascending, on
     // a side-M grid).  The tile's slots are first sorted into their 9
@@ -168,42 +211,10 @@ namespace
     {
         const int lane = threadIdx.x & 63;
         const int64_t n = A.n, M = A.q1_side;
-        const int64_t myrow = base + lane;
         const int rows = (int)(n - base < 64 ? n - base : 64);
-        const uint32_t self = myrow < n ? (uint32_t)myrow : 0u;
-        const uint32_t len = myrow < n ? (uint32_t)A.Arl[myrow] : 0u;
-        IT rc[9];
-        DT ra[9];
-#pragma unroll
-        for (int kk = 0; kk < 9; ++kk)
-        {
-            rc[kk] = IT(0);
-            ra[kk] = DT(0);
-            if ((uint32_t)kk < A.ncpr)
-            {
-                const uint64_t at = (uint64_t)kk * A.stride + (uint64_t)self;
-                rc[kk] = k::ld_stream(A.Aj + at);
-                ra[kk] = k::ld_stream(A.Ax + at);
-            }
-        }
         DT ap[9];
-        uint32_t mask = 0;
-#pragma unroll
-        for (int q = 0; q < 9; ++q)
-            ap[q] = DT(0);
-#pragma unroll
-        for (int kk = 0; kk < 9; ++kk)
-        {
-            if ((uint32_t)kk < len)
-            {
-                const int64_t d = (int64_t)k::col_of<IT>(rc[kk], (uint64_t)myrow) - myrow;
-                const int p = d < -1 ? (int)(d + M) + 1 : (d > 1 ? (int)(d - M) + 7 : (int)d + 4);
-#pragma unroll
-                for (int q = 0; q < 9; ++q)
-                    ap[q] = (p == q) ? ra[kk] : ap[q];
-                mask |= 1u << p;
-            }
-        }
+        uint32_t mask;
+        q1_slots(A, base, ap, mask);
         auto at = [&](int64_t c) { return X[(uint64_t)(c < 0 ? 0 : (c >= n ? n - 1 : c)) * R + lane]; };
         auto row_sum = [&](int r, const DT (&w)[9]) {
             const uint32_t mr = rlane(mask, r);
@@ -340,19 +351,19 @@ namespace
         }
     }
 
-    // f(row0, cnt) for the wave's rows in groups of 4 (cnt < 4 only at the
+    // f(row0, cnt) for the wave's rows in groups of G (cnt < G only at the
     // end of the matrix), in ascending row order: the callers issue the loads
     // of a group before its first store.
-    template <typename F>
-    __device__ __forceinline__ void for_rows4(int64_t n, F && f)
+    template <int G, typename F>
+    __device__ __forceinline__ void for_rows(int64_t n, F && f)
     {
         const TileRange t = wave_tiles((n + 63) / 64);
         for (int64_t tile = t.first; tile < t.end; tile += t.step)
         {
             const int64_t base = tile * 64;
             const int rows = (int)(n - base < 64 ? n - base : 64);
-            for (int r = 0; r < rows; r += 4)
-                f(base + r, rows - r < 4 ? rows - r : 4);
+            for (int r = 0; r < rows; r += G)
+                f(base + r, rows - r < G ? rows - r : G);
         }
     }
 
@@ -378,6 +389,7 @@ namespace
         DT initial_defect[kMaxCols], current_defect[kMaxCols];
         uint64_t iters[kMaxCols];
         int run[kMaxCols], converged[kMaxCols];
+        int pbuf[kMaxCols];  // the direction buffer of the column's last step (run_mcg's fused steps)
         DT eps_relative;
         uint64_t max_iters;
         int active;          // columns still iterating
@@ -398,10 +410,11 @@ namespace
 
     // Per-column reductions in two launches.  Each block stores, per column,
     // the sum of its 4 waves' lane sums in wave order (mput, no fence and no
-    // atomic); a following one-block launch sums those stores per column
-    // (msum: wave w over blocks w, w + W, ..., then the waves in order) and
-    // applies the scalar step on lane j < R of its first wave.  The kernel
-    // boundary orders the stores.
+    // atomic; column after column, so that a column's partials lie together);
+    // a following launch of one block per column sums them (msum: 16 sums
+    // over blocks w, w + 16, ..., then those in order) and applies the scalar
+    // step on thread 0.  The kernel boundary orders the stores.  (One block for
+    // all columns read its 0.5 to 1 MB of partials in 10 to 18 us.)
     template <int V>
     __device__ __forceinline__ void mput(const double (&acc)[V], double * partials)
     {
@@ -420,46 +433,46 @@ namespace
                 s += lds[1][v][lane];
                 s += lds[2][v][lane];
                 s += lds[3][v][lane];
-                partials[((uint64_t)blockIdx.x * V + v) * 64 + lane] = s;
+                partials[(uint64_t)(v * kMaxCols + lane) * gridDim.x + blockIdx.x] = s;
             }
         }
     }
 
-    // in a one-block launch of kFinThreads threads (kFinThreads / 64 waves)
+    // block blockIdx.x sums column blockIdx.x's nb partials (kFinThreads threads)
     template <int V, typename F>
-    __device__ __forceinline__ void msum(const double * partials, unsigned nb, unsigned R, F && fin)
+    __device__ __forceinline__ void msum(const double * partials, unsigned nb, F && fin)
     {
-        constexpr int W = kFinThreads / 64;
-        __shared__ double lds[W][V][64];
-        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-        double t[V];
+        constexpr int W = 16;
+        __shared__ double lds[V][kMvBlocks];
+        __shared__ double sums[V][W];
+        const unsigned j = blockIdx.x;
 #pragma unroll
         for (int v = 0; v < V; ++v)
-            t[v] = 0.0;
-#pragma unroll 8
-        for (unsigned b = (unsigned)wid; b < nb; b += W)
-        {
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                t[v] += partials[((uint64_t)b * V + v) * 64 + lane];
-        }
-#pragma unroll
-        for (int v = 0; v < V; ++v)
-            lds[wid][v][lane] = t[v];
+            for (unsigned b = threadIdx.x; b < nb; b += kFinThreads)
+                lds[v][b] = partials[(uint64_t)(v * kMaxCols + j) * nb + b];
         __syncthreads();
-        if (wid == 0)
+        if (threadIdx.x < (unsigned)(V * W))
+        {
+            const unsigned v = threadIdx.x / W, w = threadIdx.x % W;
+            double t = 0.0;
+#pragma unroll 8
+            for (unsigned b = w; b < nb; b += W)
+                t += lds[v][b];
+            sums[v][w] = t;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
         {
             double tot[V];
 #pragma unroll
             for (int v = 0; v < V; ++v)
             {
-                double s = lds[0][v][lane];
+                double s = sums[v][0];
                 for (int w = 1; w < W; ++w)
-                    s += lds[w][v][lane];
+                    s += sums[v][w];
                 tot[v] = s;
             }
-            if ((unsigned)lane < R)
-                fin(lane, tot);
+            fin((int)j, tot);
         }
     }
 
@@ -490,7 +503,7 @@ namespace
     __global__ __launch_bounds__(kFinThreads) void mcg_init_finish(const double * partials, unsigned nb, unsigned R,
             MState<DT> * s)
     {
-        msum<2>(partials, nb, R, [&](int j, const double (&t)[2]) {
+        msum<2>(partials, nb, [&](int j, const double (&t)[2]) {
             s->iters[j] = 0;
             s->converged[j] = 0;
             s->run[j] = (s->max_iters > 0) ? 1 : 0;
@@ -533,11 +546,9 @@ namespace
     __global__ __launch_bounds__(kFinThreads) void mcg_spmv_finish(const double * partials, unsigned nb, unsigned R,
             MState<DT> * s)
     {
-        if (s->active == 0)
+        if (s->run[blockIdx.x] == 0)
             return;
-        msum<1>(partials, nb, R, [&](int j, const double (&t)[1]) {
-            if (s->run[j] == 0)
-                return;
+        msum<1>(partials, nb, [&](int j, const double (&t)[1]) {
             const DT temp = (DT)t[0];
             if (VAR)
                 s->lambda[j] = s->alpha_new[j] / guard_signed<DT>(temp);
@@ -561,7 +572,7 @@ namespace
         double acc[2] = {0.0, 0.0};
         if (on)
         {
-            for_rows4(n, [&](int64_t row0, int cnt) {
+            for_rows<4>(n, [&](int64_t row0, int cnt) {
                 DT xv[4], pv[4], rv[4], vv[4], pc[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
@@ -595,14 +606,13 @@ namespace
 
     template <typename DT, bool VAR>
     __global__ __launch_bounds__(kFinThreads) void mcg_update_finish(const double * partials, unsigned nb, unsigned R,
-            MState<DT> * s)
+            MState<DT> * s, int pbuf)
     {
-        if (s->active == 0)
+        if (s->run[blockIdx.x] == 0)
             return;
-        msum<2>(partials, nb, R, [&](int j, const double (&t)[2]) {
-            if (s->run[j] == 0)
-                return;
+        msum<2>(partials, nb, [&](int j, const double (&t)[2]) {
             const DT eps = s->eps_relative;
+            s->pbuf[j] = pbuf;
             bool stop = false;
             if (VAR)
             {
@@ -642,8 +652,261 @@ namespace
             if (stop)
             {
                 s->run[j] = 0;
-                atomicSub(&s->active, 1);   // lanes of one wave, block-local
+                atomicSub(&s->active, 1);
             }
+        });
+    }
+
+    // One step of every running column on a Q1-structured matrix, in one
+    // pass: the update of X that the last step left (X += lambda P), the next
+    // direction P' = P * talpha + Pc * R (VAR) or P * talpha + R, V = A P' and
+    // the partials of v.p'.  The window of tile_rows_q1 holds P', formed
+    // wherever it is read with the operations of mcg_direction_kernel; each
+    // row stores its own into the other direction buffer.  With the update of
+    // R alone in mcg_residual_kernel, a step moves nine vectors instead of
+    // eleven and launches four kernels instead of five (513^2, 64 columns:
+    // 221 + 72 us instead of 97 + 183 + 83).  X, V and P' pass the caches by
+    // (non-temporal: the window's lines of P and R stay in L2, 496 instead of
+    // 561 MB read; V and X are not read again before they would be evicted).
+    // It moves 0.90 GB at 4.1 TB/s.
+    template <typename DT, typename IT, typename LT, bool VAR>
+    __global__ __launch_bounds__(256) void mcg_step_kernel(MvEll<DT, IT, LT> A, const DT * __restrict__ Pold,
+            const DT * __restrict__ Rv, const DT * __restrict__ Pc, DT * __restrict__ Pnew, DT * __restrict__ Vv,
+            DT * __restrict__ X, unsigned R, double * partials, const MState<DT> * s)
+    {
+        if (s->active == 0)
+            return;
+        const unsigned lane = threadIdx.x & 63;
+        const bool on = lane < R && s->run[lane] != 0;
+        const DT talpha = on ? s->talpha[lane] : DT(0), lambda = on ? s->lambda[lane] : DT(0);
+        const int64_t n = A.n, M = A.q1_side;
+        double acc[1] = {0.0};
+        // P and Pc * R (or R) at row c, clamped to the matrix; dir: P'
+        auto old_at = [&](int64_t c) { return on ? Pold[(uint64_t)c * R + lane] : DT(0); };
+        auto res_at = [&](int64_t c) { return on ? Rv[(uint64_t)c * R + lane] : DT(0); };
+        auto dir = [&](DT p, DT r, DT pc) {
+            const DT t = p * talpha;
+            return t + (VAR ? pc * r : r);
+        };
+        auto clamp = [&](int64_t c) { return c < 0 ? (int64_t)0 : (c >= n ? n - 1 : c); };
+        // the tile's matrix values per wave, read back row by row (kept in
+        // registers they leave room for four waves per SIMD instead of five,
+        // and 1029 blocks of four waves then run in two rounds)
+        __shared__ DT slots[4][64][9];
+        DT (*const sl)[9] = slots[threadIdx.x >> 6];
+        const TileRange t = wave_tiles((n + 63) / 64);
+        for (int64_t tile = t.first; tile < t.end; tile += t.step)
+        {
+            const int64_t base = tile * 64;
+            const int rows = (int)(n - base < 64 ? n - base : 64);
+            uint32_t mask;
+            {
+                DT ap[9];
+                q1_slots(A, base, ap, mask);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int q = 0; q < 9; ++q)
+                    sl[lane][q] = ap[q];
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
+            auto row_out = [&](int r, const DT (&w)[9], DT po, DT xv) {
+                const uint32_t mr = rlane(mask, r);
+                DT sum = DT(0);
+#pragma unroll
+                for (int q = 0; q < 9; ++q)
+                {
+                    if ((mr >> q) & 1u)
+                        sum += sl[r][q] * w[q];
+                }
+                if (on)
+                {
+                    const uint64_t e = (uint64_t)(base + r) * R + lane;
+                    __builtin_nontemporal_store(xv + lambda * po, X + e);
+                    __builtin_nontemporal_store(w[4], Pnew + e);
+                    __builtin_nontemporal_store(sum, Vv + e);
+                    acc[0] += (double)sum * (double)w[4];
+                }
+            };
+            // window columns x - 1 and x of the next row (P'), and P at (y, x)
+            DT c0[3], c1[3], c1o = DT(0);
+            bool have = false;
+            int64_t x = base % M;
+            int r = 0;
+            while (r < rows)
+            {
+                const int64_t i = base + r;
+                if (x == 0 || ! have)
+                {
+                    DT p[3][2], rr[3][2], pc[3][2];
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+#pragma unroll
+                        for (int d = 0; d < 2; ++d)
+                        {
+                            const int64_t c = clamp(i + (b - 1) * M - 1 + d);
+                            p[b][d] = old_at(c);
+                            rr[b][d] = res_at(c);
+                            pc[b][d] = VAR ? Pc[c] : DT(0);
+                        }
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+                    {
+                        c0[b] = dir(p[b][0], rr[b][0], pc[b][0]);
+                        c1[b] = dir(p[b][1], rr[b][1], pc[b][1]);
+                    }
+                    c1o = p[1][1];
+                }
+                const bool four = r + 4 <= rows && x + 3 < M;
+                const int cnt = four ? 4 : 1;
+                DT p[3][4], rr[3][4], pc[3][4], xv[4];
+                if (four)
+                {
+                    // 4 rows of one grid line: their 28 loads in flight at once
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                        {
+                            const int64_t c = clamp(i + (b - 1) * M + 1 + u);
+                            p[b][u] = old_at(c);
+                            rr[b][u] = res_at(c);
+                            pc[b][u] = VAR ? Pc[c] : DT(0);
+                        }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        xv[u] = on ? k::ld_stream(X + (uint64_t)(i + u) * R + lane) : DT(0);
+                    DT v[3][4];
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            v[b][u] = dir(p[b][u], rr[b][u], pc[b][u]);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                    {
+                        DT w[9];
+#pragma unroll
+                        for (int b = 0; b < 3; ++b)
+#pragma unroll
+                            for (int d = 0; d < 3; ++d)
+                            {
+                                const int k = u + d;       // column x - 1 + k of band b
+                                w[b * 3 + d] = k == 0 ? c0[b] : (k == 1 ? c1[b] : v[b][k - 2]);
+                            }
+                        row_out(r + u, w, u == 0 ? c1o : p[1][u > 0 ? u - 1 : 0], xv[u]);
+                    }
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+                    {
+                        c0[b] = v[b][2];
+                        c1[b] = v[b][3];
+                    }
+                    c1o = p[1][3];
+                }
+                else
+                {
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+                    {
+                        const int64_t c = clamp(i + (b - 1) * M + 1);
+                        p[b][0] = old_at(c);
+                        rr[b][0] = res_at(c);
+                        pc[b][0] = VAR ? Pc[c] : DT(0);
+                    }
+                    xv[0] = on ? k::ld_stream(X + (uint64_t)i * R + lane) : DT(0);
+                    DT w[9];
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+                    {
+                        w[b * 3] = c0[b];
+                        w[b * 3 + 1] = c1[b];
+                        w[b * 3 + 2] = dir(p[b][0], rr[b][0], pc[b][0]);
+                    }
+                    row_out(r, w, c1o, xv[0]);
+#pragma unroll
+                    for (int b = 0; b < 3; ++b)
+                    {
+                        c0[b] = w[b * 3 + 1];
+                        c1[b] = w[b * 3 + 2];
+                    }
+                    c1o = p[1][0];
+                }
+                r += cnt;
+                x += cnt;
+                if (x >= M)
+                    x -= M;
+                have = true;
+            }
+        }
+        mput<1>(acc, partials);
+    }
+
+    // R += (-lambda) V; per column r.r (and r.(Pc r)): mcg_update_kernel
+    // without its update of X, which mcg_step_kernel or mcg_flush_kernel makes
+    template <typename DT, bool VAR>
+    __global__ __launch_bounds__(256) void mcg_residual_kernel(DT * __restrict__ Rv, const DT * __restrict__ Vv,
+            const DT * __restrict__ Pc, int64_t n, unsigned R, double * partials, const MState<DT> * s)
+    {
+        if (s->active == 0)
+            return;
+        const unsigned lane = threadIdx.x & 63;
+        const bool on = lane < R && s->run[lane] != 0;
+        const DT mlambda = on ? -s->lambda[lane] : DT(0);
+        double acc[2] = {0.0, 0.0};
+        if (on)
+        {
+            for_rows<16>(n, [&](int64_t row0, int cnt) {
+                DT rv[16], vv[16], pc[16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u)
+                {
+                    const int64_t row = row0 + (u < cnt ? u : 0);
+                    const uint64_t e = (uint64_t)row * R + lane;
+                    rv[u] = Rv[e];
+                    vv[u] = k::ld_stream(Vv + e);
+                    pc[u] = VAR ? Pc[row] : DT(0);
+                }
+#pragma unroll
+                for (int u = 0; u < 16; ++u)
+                {
+                    if (u < cnt)
+                    {
+                        const DT ri = rv[u] + mlambda * vv[u];
+                        Rv[(uint64_t)(row0 + u) * R + lane] = ri;
+                        acc[0] += (double)ri * (double)ri;
+                        if (VAR)
+                            acc[1] += (double)ri * (double)(pc[u] * ri);
+                    }
+                }
+            });
+        }
+        mput<2>(acc, partials);
+    }
+
+    // The update of X that each column's last step left: X += lambda P, P in
+    // the direction buffer of that step.
+    template <typename DT>
+    __global__ __launch_bounds__(256) void mcg_flush_kernel(DT * __restrict__ X, const DT * __restrict__ P0,
+            const DT * __restrict__ P1, int64_t n, unsigned R, const MState<DT> * s)
+    {
+        const unsigned lane = threadIdx.x & 63;
+        if (! (lane < R && s->iters[lane] != 0))
+            return;
+        const DT lambda = s->lambda[lane];
+        const DT * P = s->pbuf[lane] ? P1 : P0;
+        for_rows<4>(n, [&](int64_t row0, int cnt) {
+            DT xv[4], pv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+            {
+                const uint64_t e = (uint64_t)(row0 + (u < cnt ? u : 0)) * R + lane;
+                xv[u] = X[e];
+                pv[u] = P[e];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (u < cnt)
+                    X[(uint64_t)(row0 + u) * R + lane] = xv[u] + lambda * pv[u];
         });
     }
 
@@ -658,7 +921,7 @@ namespace
         if (! (lane < R && s->run[lane] != 0))
             return;
         const DT talpha = s->talpha[lane];
-        for_rows4(n, [&](int64_t row0, int cnt) {
+        for_rows<4>(n, [&](int64_t row0, int cnt) {
             DT pv[4], rv[4], pc[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
@@ -723,8 +986,19 @@ namespace
         const size_t vb = ((sizeof(DT) * n * R + 255) / 256) * 256;
         const unsigned grid = mv_grid(n);
         const size_t pb = sizeof(double) * 2 * 64 * grid;
+        // Q1-structured matrices: fused steps with a second direction buffer
+        // (a step's gathers read P and R, three of each per row through the
+        // window; other matrices would gather both for every entry)
+        const size_t rest = pb + sizeof(MState<DT>) + 256;
         void * block = nullptr;
-        if (hipMalloc(&block, 3 * vb + pb + sizeof(MState<DT>) + 256) != hipSuccess)
+        bool fused = K < 0;
+        if (fused && hipMalloc(&block, 4 * vb + rest) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            block = nullptr;
+            fused = false;
+        }
+        if (! block && hipMalloc(&block, 3 * vb + rest) != hipSuccess)
             throw Error(HSOLVE_ERR_ALLOC, "cg_ell_multi: workspace allocation failed");
         struct Free
         {
@@ -735,6 +1009,12 @@ namespace
         DT * Rv = (DT *)c; c += vb;
         DT * Pv = (DT *)c; c += vb;
         DT * Vv = (DT *)c; c += vb;
+        DT * pv[2] = {Pv, Pv};
+        if (fused)
+        {
+            pv[1] = (DT *)c;
+            c += vb;
+        }
         double * partials = (double *)c; c += pb;
         MState<DT> * s = (MState<DT> *)c;
 
@@ -745,25 +1025,44 @@ namespace
         HIP_CHECK(hipMemcpyAsync(s, &h, sizeof(h), hipMemcpyHostToDevice, st));
         hipLaunchKernelGGL((mcg_init_kernel<DT, IT, LT, K, VAR>), dim3(grid), dim3(kBlock), 0, st, A, Bv,
                            (const DT *)X, Rv, Pv, Pc, R, partials);
-        hipLaunchKernelGGL((mcg_init_finish<DT, VAR>), dim3(1), dim3(kFinThreads), 0, st, (const double *)partials, grid,
+        hipLaunchKernelGGL((mcg_init_finish<DT, VAR>), dim3(R), dim3(kFinThreads), 0, st, (const double *)partials, grid,
                            R, s);
         HIP_CHECK(hipGetLastError());
         uint64_t enqueued = 0, chunk = 8;
+        int cp = 0;             // pv[cp] holds the current direction
         while (true)
         {
             for (uint64_t i = 0; i < chunk && enqueued < max_iters; ++i, ++enqueued)
             {
-                hipLaunchKernelGGL((mcg_spmv_kernel<DT, IT, LT, K>), dim3(grid), dim3(kBlock), 0, st, A,
-                                   (const DT *)Pv, Vv, R, partials, (const MState<DT> *)s);
-                hipLaunchKernelGGL((mcg_spmv_finish<DT, VAR>), dim3(1), dim3(kFinThreads), 0, st,
+                bool step = false;
+                if constexpr (K < 0)
+                {
+                    if (fused && enqueued > 0)
+                    {
+                        hipLaunchKernelGGL((mcg_step_kernel<DT, IT, LT, VAR>), dim3(grid), dim3(kBlock), 0, st, A,
+                                           (const DT *)pv[cp], (const DT *)Rv, Pc, pv[cp ^ 1], Vv, X, R, partials,
+                                           (const MState<DT> *)s);
+                        cp ^= 1;
+                        step = true;
+                    }
+                }
+                if (! step)
+                    hipLaunchKernelGGL((mcg_spmv_kernel<DT, IT, LT, K>), dim3(grid), dim3(kBlock), 0, st, A,
+                                       (const DT *)pv[cp], Vv, R, partials, (const MState<DT> *)s);
+                hipLaunchKernelGGL((mcg_spmv_finish<DT, VAR>), dim3(R), dim3(kFinThreads), 0, st,
                                    (const double *)partials, grid, R, s);
-                hipLaunchKernelGGL((mcg_update_kernel<DT, VAR>), dim3(grid), dim3(kBlock), 0, st, X, Rv,
-                                   (const DT *)Pv, (const DT *)Vv, Pc, (int64_t)n, R, partials,
-                                   (const MState<DT> *)s);
-                hipLaunchKernelGGL((mcg_update_finish<DT, VAR>), dim3(1), dim3(kFinThreads), 0, st,
-                                   (const double *)partials, grid, R, s);
-                hipLaunchKernelGGL((mcg_direction_kernel<DT, VAR>), dim3(grid), dim3(kBlock), 0, st, Pv,
-                                   (const DT *)Rv, Pc, (int64_t)n, R, (const MState<DT> *)s);
+                if (fused)
+                    hipLaunchKernelGGL((mcg_residual_kernel<DT, VAR>), dim3(grid), dim3(kBlock), 0, st, Rv,
+                                       (const DT *)Vv, Pc, (int64_t)n, R, partials, (const MState<DT> *)s);
+                else
+                    hipLaunchKernelGGL((mcg_update_kernel<DT, VAR>), dim3(grid), dim3(kBlock), 0, st, X, Rv,
+                                       (const DT *)Pv, (const DT *)Vv, Pc, (int64_t)n, R, partials,
+                                       (const MState<DT> *)s);
+                hipLaunchKernelGGL((mcg_update_finish<DT, VAR>), dim3(R), dim3(kFinThreads), 0, st,
+                                   (const double *)partials, grid, R, s, cp);
+                if (! fused)
+                    hipLaunchKernelGGL((mcg_direction_kernel<DT, VAR>), dim3(grid), dim3(kBlock), 0, st, Pv,
+                                       (const DT *)Rv, Pc, (int64_t)n, R, (const MState<DT> *)s);
             }
             HIP_CHECK(hipGetLastError());
             HIP_CHECK(hipMemcpyAsync(&h, s, sizeof(h), hipMemcpyDeviceToHost, st));
@@ -772,6 +1071,13 @@ namespace
                 break;
             if (chunk < 64)
                 chunk *= 2;
+        }
+        if (fused)
+        {
+            hipLaunchKernelGGL((mcg_flush_kernel<DT>), dim3(grid), dim3(kBlock), 0, st, X, (const DT *)pv[0],
+                               (const DT *)pv[1], (int64_t)n, R, (const MState<DT> *)s);
+            HIP_CHECK(hipGetLastError());
+            HIP_CHECK(hipStreamSynchronize(st));
         }
         for (unsigned j = 0; j < R; ++j)
         {
