@@ -65,6 +65,16 @@ namespace
         return (size_t)(w * vs + 16);
     }
 
+    // 9-point structured matrices up to this many rows go one row per lane
+    // (ell_stencil_row), larger ones two (ell_spmv_r2).  One row per lane has
+    // twice the wavefronts and a shorter chain, which is what a product of a
+    // few microseconds needs; two need half the instructions per byte, which
+    // is what the memory rate needs.  Measured on MI355X, product, one row
+    // against two, us: FP32 257^2 4.3 / 5.9, 513^2 4.4 / 6.4, 1025^2 8.2 /
+    // 11.8, 2049^2 31.8 / 41.5, 2897^2 72.5 / 75.4; FP64 513^2 5.7 / 8.2,
+    // 1025^2 17.8 / 23.0, 2049^2 67.1 / 69.6, 2897^2 131.8 / 129.2.
+    constexpr uint64_t kStencilRowRows = 1 << 23;
+
     // rows [r0, r1) (r0 even: the rows pair up as in the whole product)
     template <typename DT, typename IT, typename LT, int MODE, int K>
     bool ell_launch_r2(const hsolve_ell_s * m, int v, const DT * x, DT * y, const IT * Aj, const DT * Ax,
@@ -206,6 +216,19 @@ namespace
                 HIP_CHECK(hipGetLastError());
                 return;
             }
+            // 9-point structured matrices (the automatic choice only; their
+            // columns and lengths always fit the short types below this many
+            // rows)
+            if constexpr (sizeof(IT) == 2 && sizeof(LT) == 1)
+                if (m->q1_side != 0 && (v & HSOLVE_ELL_FULL) && (m->variant & HSOLVE_ELL_SET) == 0 && m->ncpr != 0 &&
+                    r1 - r0 <= kStencilRowRows)
+                {
+                    hipLaunchKernelGGL((k::ell_stencil_row<DT, IT, LT, MODE>), dim3(grid_for(r1 - r0, 64)), dim3(64), 0,
+                                       st, x, y, Aj, Ax, Arl, rhs, dinv, r0, r1, m->stride, (uint32_t)m->ncpr,
+                                       (int64_t)m->q1_side);
+                    HIP_CHECK(hipGetLastError());
+                    return;
+                }
             if (r2_ok && (ell_launch_r2<DT, IT, LT, MODE, 4>(m, v, x, y, Aj, Ax, Arl, rhs, dinv, st, r0, r1) ||
                           ell_launch_r2<DT, IT, LT, MODE, 9>(m, v, x, y, Aj, Ax, Arl, rhs, dinv, st, r0, r1) ||
                           ell_launch_r2<DT, IT, LT, MODE, 13>(m, v, x, y, Aj, Ax, Arl, rhs, dinv, st, r0, r1) ||

@@ -113,6 +113,47 @@ namespace k
     template <> struct Vec2<int16_t> { typedef short type __attribute__((ext_vector_type(2))); };
     template <> struct Vec2<uint32_t> { typedef unsigned type __attribute__((ext_vector_type(2))); };
 
+    // 16-byte vectors: 4 floats or 2 doubles per lane
+    template <typename DT> struct Vec16;
+    template <> struct Vec16<float>
+    {
+        static constexpr int V = 4;
+        typedef float type __attribute__((ext_vector_type(4)));
+    };
+    template <> struct Vec16<double>
+    {
+        static constexpr int V = 2;
+        typedef double type __attribute__((ext_vector_type(2)));
+    };
+
+    // N consecutive elements from any element address, in loads of 16 and 8
+    // bytes (a vector load needs its address aligned to 4 bytes only)
+    template <int N, typename DT>
+    __device__ __forceinline__ void ld_window(const DT * __restrict__ p, DT (&w)[N])
+    {
+        constexpr int V = Vec16<DT>::V;
+        typedef DT VW __attribute__((ext_vector_type(V), aligned(sizeof(DT))));
+        typedef DT V2 __attribute__((ext_vector_type(2), aligned(sizeof(DT))));
+        static_assert(N % 2 == 0, "an even number of elements");
+#pragma unroll
+        for (int j = 0; j < N; j += V)
+        {
+            if (j + V <= N)
+            {
+                const VW v = *(const VW *)(p + j);
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+                    w[j + e] = v[e];
+            }
+            else
+            {
+                const V2 v = *(const V2 *)(p + j);
+                w[j] = v.x;
+                w[j + 1] = v.y;
+            }
+        }
+    }
+
     // Two consecutive rows per lane (threads == 1 layout): the value and
     // index streams are read as 2-element vectors, halving the load
     // instructions per byte.  FULL loads every slot below num_cols_per_row
@@ -134,9 +175,11 @@ namespace k
         typedef typename Vec2<DT>::type V;
         typedef typename Vec2<IT>::type VI;
         const uint32_t b = XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-        const uint64_t r0 = row_start + ((uint64_t)b * blockDim.x + threadIdx.x) * 2;
-        if (r0 >= row_end)
-            return;
+        const uint64_t rr = row_start + ((uint64_t)b * 256 + threadIdx.x) * 2;
+        // a lane past the end repeats the first pair and stores nothing: no
+        // branch stands between the launch and the loads
+        const bool live = rr < row_end;
+        const uint64_t r0 = live ? rr : row_start;
         const bool two = r0 + 1 < row_end;
         // the defect / sweep operands of both rows load up front (the second
         // row's index clamped to the first when there is none), not after
@@ -158,8 +201,21 @@ namespace k
         const uint32_t len0 = (uint32_t)Arl[r0];
         const uint32_t len1 = two ? (uint32_t)Arl[r0 + 1] : 0u;
         const uint32_t lmax = len0 > len1 ? len0 : len1;
-        // STENCIL: both rows full, columns from the offsets
-        const bool implied = STENCIL && len0 == 9 && (len1 == 9 || ! two);
+        // STENCIL: both rows full, columns from the offsets.  The two rows'
+        // 3 x 3 neighbourhoods share three windows of four x values, loaded
+        // with the slots and not after the lengths (a window that would leave
+        // x, possible only where a row is short, is moved inside and not used).
+        const bool implied = STENCIL && len0 == 9 && len1 == 9;
+        DT w[STENCIL ? 3 : 1][4];
+        if (STENCIL)
+        {
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+            {
+                const int64_t c = (int64_t)r0 + (int64_t)(d - 1) * m - 1, last = m * m - 4;
+                ld_window<4>(x + (c < 0 ? 0 : c > last ? last : c), w[d]);
+            }
+        }
         DT a0[MAXK], a1[MAXK];
         IT c0[MAXK], c1[MAXK];
         // A slot past the rows' lengths (past num_cols_per_row with FULL)
@@ -183,37 +239,36 @@ namespace k
         DT s0 = DT(0), s1 = DT(0);
         if (implied)
         {
-            // the two rows' 3 x 3 neighbourhoods share three windows of four
-            // x values (12 loads instead of 18); slot k = 3 (dy + 1) + dx + 1
-            DT w[3][4];
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-            {
-                const int64_t c = (int64_t)r0 + (int64_t)(d - 1) * m - 1;
-                w[d][0] = x[c];
-                w[d][1] = x[c + 1];
-                w[d][2] = x[c + 2];
-                w[d][3] = x[two ? c + 3 : c + 2];
-            }
+            // slot k = 3 (dy + 1) + dx + 1
 #pragma unroll
             for (int k = 0; k < MAXK; ++k)
             {
-                s0 += a0[k] * w[k / 3][k % 3];
-                if (two)
-                    s1 += a1[k] * w[k / 3][k % 3 + 1];
+                s0 += a0[k] * w[STENCIL ? k / 3 : 0][k % 3];
+                s1 += a1[k] * w[STENCIL ? k / 3 : 0][k % 3 + 1];
             }
         }
         else
         {
+            // a slot past the row's length gathers x[0] and is not added: under
+            // guards each of the gathers is a round trip of its own (measured:
+            // FP64 product of 4097 x 4097 277.6 -> 265.5 us, 5.6 TB/s)
+            DT x0v[MAXK], x1v[MAXK];
 #pragma unroll
             for (int k = 0; k < MAXK; ++k)
             {
-                if ((uint32_t)k < len0)
-                    s0 += a0[k] * x[col_of<IT>(c0[k], r0)];
-                if ((uint32_t)k < len1)
-                    s1 += a1[k] * x[col_of<IT>(c1[k], r0 + 1)];
+                x0v[k] = x[(uint32_t)k < len0 ? col_of<IT>(c0[k], r0) : 0];
+                x1v[k] = x[(uint32_t)k < len1 ? col_of<IT>(c1[k], r0 + 1) : 0];
+            }
+#pragma unroll
+            for (int k = 0; k < MAXK; ++k)
+            {
+                const DT t0 = a0[k] * x0v[k], t1 = a1[k] * x1v[k];
+                s0 = (uint32_t)k < len0 ? s0 + t0 : s0;
+                s1 = (uint32_t)k < len1 ? s1 + t1 : s1;
             }
         }
+        if (! live)
+            return;
         if (MODE == 0)
         {
             y[r0] = s0;
@@ -235,6 +290,76 @@ namespace k
                 const DT t1 = b1 - s1;
                 y[r0 + 1] = x1 + t1 * d1;
             }
+        }
+    }
+
+    // One row per lane of a 9-point structured matrix (ell_spmv_r2's STENCIL
+    // rules).  Bound by latency on the sizes it is used for: the length, the
+    // nine slots and the nine x values of a full row load at once, and only a
+    // wave that holds a shorter row goes on to the columns and then to its
+    // gathers.  Blocks of one wave reach every CU from 16,384 rows on.
+    // Measured on MI355X, FP32 defect of 513 x 513, call to call: two rows per
+    // lane with guarded gathers 9.1 us, without guards 7.2, this kernel 4.5.
+    template <typename DT, typename IT, typename LT, int MODE>
+    __global__ __launch_bounds__(64) void ell_stencil_row(
+            const DT * __restrict__ x, DT * __restrict__ y, const IT * __restrict__ Aj,
+            const DT * __restrict__ Ax, const LT * __restrict__ Arl, const DT * __restrict__ rhs,
+            const DT * __restrict__ dinv, uint64_t row_start, uint64_t row_end, uint64_t stride,
+            uint32_t ncpr, int64_t m)
+    {
+        const uint64_t r = row_start + (uint64_t)blockIdx.x * 64 + threadIdx.x;
+        const uint64_t row = r < row_end ? r : row_end - 1;
+        const uint32_t len = (uint32_t)Arl[row];
+        DT b = DT(0), x0 = DT(0), d = DT(0);
+        if (MODE != 0)
+            b = rhs[row];
+        if (MODE == 2)
+        {
+            x0 = x[row];
+            d = dinv[row];
+        }
+        DT a[9], w[9];
+        const int64_t n = m * m;
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+        {
+            const int64_t c = (int64_t)row + (int64_t)(k / 3 - 1) * m + (k % 3 - 1);
+            a[k] = ld_stream(Ax + row + ((uint32_t)k < ncpr ? (uint64_t)k : 0) * stride);
+            w[k] = x[c < 0 || c >= n ? (int64_t)row : c];
+        }
+        DT s = DT(0);
+        if (len == 9)
+        {
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+                s += a[k] * w[k];
+        }
+        else
+        {
+            IT c[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+                c[k] = ld_stream(Aj + row + ((uint32_t)k < ncpr ? (uint64_t)k : 0) * stride);
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+                w[k] = x[(uint32_t)k < len ? col_of<IT>(c[k], row) : row];
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+            {
+                const DT t = a[k] * w[k];
+                s = (uint32_t)k < len ? s + t : s;
+            }
+        }
+        if (r >= row_end)
+            return;
+        if (MODE == 0)
+            y[r] = s;
+        else if (MODE == 1)
+            y[r] = b - s;
+        else
+        {
+            const DT t = b - s;
+            y[r] = x0 + t * d;
         }
     }
 
@@ -600,68 +725,53 @@ namespace k
     __device__ __forceinline__ DT q1_row(const Bands & B, const XV & x, int64_t i, int64_t n, int64_t m)
     {
         const DT * const * b = reinterpret_cast<const DT * const *>(B.b);
-        if (ORD == 1)
+        // A neighbour outside [0, n) is replaced by the node itself and its
+        // product is not added, so that no branch separates the 18 loads:
+        // under guards each one is a round trip of its own, and the first
+        // and last m rows are the last to finish on a small grid.
+        DT s = ORD == 1 ? DT(0) : ld_stream(b[4] + i) * x[i];
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
         {
-            DT s = DT(0);
-            if (i - m - 1 >= 0) s += ld_stream(b[0] + i) * x[i - m - 1];
-            if (i - m >= 0)     s += ld_stream(b[1] + i) * x[i - m];
-            if (i - m + 1 >= 0) s += ld_stream(b[2] + i) * x[i - m + 1];
-            if (i - 1 >= 0)     s += ld_stream(b[3] + i) * x[i - 1];
-            s += ld_stream(b[4] + i) * x[i];
-            if (i + 1 < n)      s += ld_stream(b[5] + i) * x[i + 1];
-            if (i + m - 1 < n)  s += ld_stream(b[6] + i) * x[i + m - 1];
-            if (i + m < n)      s += ld_stream(b[7] + i) * x[i + m];
-            if (i + m + 1 < n)  s += ld_stream(b[8] + i) * x[i + m + 1];
-            return s;
+            const int64_t j = i + (k / 3 - 1) * m + (k % 3 - 1);
+            if (k == 4)
+            {
+                if (ORD == 1)
+                    s += ld_stream(b[4] + i) * x[i];
+                continue;
+            }
+            const bool in = k < 4 ? j >= 0 : j < n;
+            const DT t = ld_stream(b[k] + i) * x[in ? j : i];
+            s = in ? s + t : s;
         }
-        DT s = ld_stream(b[4] + i) * x[i];
-        if (i - m - 1 >= 0) s += ld_stream(b[0] + i) * x[i - m - 1];
-        if (i - m >= 0)     s += ld_stream(b[1] + i) * x[i - m];
-        if (i - m + 1 >= 0) s += ld_stream(b[2] + i) * x[i - m + 1];
-        if (i - 1 >= 0)     s += ld_stream(b[3] + i) * x[i - 1];
-        if (i + 1 < n)      s += ld_stream(b[5] + i) * x[i + 1];
-        if (i + m - 1 < n)  s += ld_stream(b[6] + i) * x[i + m - 1];
-        if (i + m < n)      s += ld_stream(b[7] + i) * x[i + m];
-        if (i + m + 1 < n)  s += ld_stream(b[8] + i) * x[i + m + 1];
         return s;
     }
+
+    // One-wave blocks: 129 x 129 rows reach all 256 CUs.
+    constexpr int kQ1Block = 64;
 
     // mode 0: y = A x; mode 1: y = rhs - A x;
     // mode 2: y = x + (rhs - A x) * dinv (one Jacobi sweep into y)
     template <typename DT, int MODE>
-    __global__ __launch_bounds__(256) void q1_kernel(Bands B, const DT * __restrict__ x,
+    __global__ __launch_bounds__(kQ1Block) void q1_kernel(Bands B, const DT * __restrict__ x,
             DT * __restrict__ y, const DT * __restrict__ rhs, const DT * __restrict__ dinv,
-            int64_t n, int64_t m, const int * __restrict__ active)
+            int64_t n, int64_t m)
     {
-        if (active && *active == 0)
-            return;
-        const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-        if (i >= n)
-            return;
-        const DT s = q1_row<DT>(B, x, i, n, m);
-        if (MODE == 0)
-            y[i] = s;
-        else if (MODE == 1)
-            y[i] = rhs[i] - s;
-        else
+        // a lane past the end repeats the last row: no branch stands between
+        // the launch and the loads
+        const int64_t r = (int64_t)blockIdx.x * kQ1Block + threadIdx.x;
+        const int64_t i = r < n ? r : n - 1;
+        DT o = q1_row<DT>(B, x, i, n, m);
+        if (MODE == 1)
+            o = rhs[i] - o;
+        else if (MODE == 2)
         {
-            const DT t = rhs[i] - s;
-            y[i] = x[i] + t * dinv[i];
+            const DT t = rhs[i] - o;
+            o = x[i] + t * dinv[i];
         }
+        if (r < n)
+            y[r] = o;
     }
-
-    // 16-byte vectors: 4 floats or 2 doubles per lane
-    template <typename DT> struct Vec16;
-    template <> struct Vec16<float>
-    {
-        static constexpr int V = 4;
-        typedef float type __attribute__((ext_vector_type(4)));
-    };
-    template <> struct Vec16<double>
-    {
-        static constexpr int V = 2;
-        typedef double type __attribute__((ext_vector_type(2)));
-    };
 
     // Q1 row sums of V consecutive rows i0..i0+V-1 that lie away from both
     // ends of the vector (every index guard of q1_row holds): bands come in
@@ -679,13 +789,9 @@ namespace k
         for (int k = 0; k < 9; ++k)
             bv[k] = __builtin_nontemporal_load((const VT *)(b[k] + i0));
         DT xm[V + 2], xc[V + 2], xp[V + 2];
-#pragma unroll
-        for (int j = 0; j < V + 2; ++j)
-        {
-            xm[j] = x[i0 - m - 1 + j];
-            xc[j] = x[i0 - 1 + j];
-            xp[j] = x[i0 + m - 1 + j];
-        }
+        ld_window<V + 2>(x + i0 - m - 1, xm);
+        ld_window<V + 2>(x + i0 - 1, xc);
+        ld_window<V + 2>(x + i0 + m - 1, xp);
         if (ORD == 1)
         {
 #pragma unroll
@@ -736,6 +842,9 @@ namespace k
             return;
         if (i0 - m - 1 < 0 || i0 + V + m >= n)
         {
+            // (one row at a time: unrolled, the 72 loads in flight cost a
+            // wave of occupancy)
+#pragma unroll 1
             for (int v = 0; v < V && i0 + v < n; ++v)
             {
                 const int64_t i = i0 + v;
@@ -787,34 +896,42 @@ namespace k
     template <typename DT, int MODE>
     __global__ __launch_bounds__(256) void q1_kernel_v(Bands B, const DT * __restrict__ x,
             DT * __restrict__ y, const DT * __restrict__ rhs, const DT * __restrict__ dinv,
-            int64_t n, int64_t m, const int * __restrict__ active)
+            int64_t n, int64_t m)
     {
-        if (active && *active == 0)
-            return;
         q1_body_v<DT, MODE>(B, x, y, rhs, dinv, n, m, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
     }
 
     inline bool aligned16(const void * p) { return ((uintptr_t)p & 15u) == 0; }
 
-    // Launches the vectorised Q1 kernel when every streamed array is 16-byte
-    // aligned, else the one-row-per-lane form.  MODE as q1_kernel.
+    // Grids up to this many rows go one row per lane: more wavefronts and a
+    // shorter chain for a product that lasts a few microseconds.  Above, the
+    // 16-byte loads win.  Measured on MI355X, jacobi, one row per lane against
+    // the vector form, us: FP32 129^2 4.3 (6.5 with guarded loads in the vector
+    // form), 513^2 4.3 / 7.3, 1025^2 11.3 / 14.3, 2049^2 39.8 / 41.0, 2897^2
+    // 84.6 / 77.6, 4097^2 150 / 142; FP64 1025^2 19.6 / 21.9, 2049^2 69.5 /
+    // 73.3, 2897^2 145 / 151, 4097^2 322 / 270.
+    constexpr int64_t kQ1RowRows = 1 << 23;
+
+    // Launches the vectorised Q1 kernel on a large grid whose streamed arrays
+    // are all 16-byte aligned, else the one-row-per-lane form.  MODE as
+    // q1_kernel.
     template <typename DT, int MODE>
     inline void q1_launch(const Bands & B, const DT * x, DT * y, const DT * rhs, const DT * dinv, int64_t n,
-                          int64_t m, const int * active, hipStream_t st)
+                          int64_t m, hipStream_t st)
     {
         bool vec = aligned16(y) && (MODE == 0 || aligned16(rhs)) && (MODE != 2 || aligned16(dinv));
         for (int k = 0; k < 9; ++k)
             vec = vec && aligned16(B.b[k]);
-        if (vec)
+        if (vec && n > kQ1RowRows)
         {
             constexpr int V = Vec16<DT>::V;
             const uint64_t lanes = ((uint64_t)n + V - 1) / V;
             hipLaunchKernelGGL((q1_kernel_v<DT, MODE>), dim3(grid_for(lanes, 256)), dim3(256), 0, st, B, x, y, rhs,
-                               dinv, n, m, active);
+                               dinv, n, m);
         }
         else
-            hipLaunchKernelGGL((q1_kernel<DT, MODE>), dim3(grid_for((uint64_t)n, 256)), dim3(256), 0, st, B, x, y, rhs,
-                               dinv, n, m, active);
+            hipLaunchKernelGGL((q1_kernel<DT, MODE>), dim3(grid_for((uint64_t)n, kQ1Block)), dim3(kQ1Block), 0, st, B, x,
+                               y, rhs, dinv, n, m);
     }
 
     // ------------------------------------------------------------ reductions

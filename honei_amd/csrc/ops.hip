@@ -72,11 +72,11 @@ namespace hsolve
         const int64_t m = (int64_t)std::sqrt((double)n);
         require((uint64_t)(m * m) == n, HSOLVE_ERR_SIZE, "Q1 size is not a square");
         if (mode == 0)
-            k::q1_launch<DT, 0>(B, x, y, rhs, dinv, (int64_t)n, m, nullptr, st);
+            k::q1_launch<DT, 0>(B, x, y, rhs, dinv, (int64_t)n, m, st);
         else if (mode == 1)
-            k::q1_launch<DT, 1>(B, x, y, rhs, dinv, (int64_t)n, m, nullptr, st);
+            k::q1_launch<DT, 1>(B, x, y, rhs, dinv, (int64_t)n, m, st);
         else
-            k::q1_launch<DT, 2>(B, x, y, rhs, dinv, (int64_t)n, m, nullptr, st);
+            k::q1_launch<DT, 2>(B, x, y, rhs, dinv, (int64_t)n, m, st);
         HIP_CHECK(hipGetLastError());
     }
 
