@@ -221,6 +221,13 @@ def lib():
     return L
 
 
+def calls():
+    """The entry points of the shortest calls without ctypes (csrc/pycalls.c)."""
+    lib()
+    from . import _calls
+    return _calls
+
+
 def check(code, what=""):
     if code != 0:
         msg = lib().hsolve_last_error().decode(errors="replace")

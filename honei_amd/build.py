@@ -1,4 +1,5 @@
-"""Build libhsolve.so (gfx950) in-tree with hipcc.
+"""Build libhsolve.so (gfx950) in-tree with hipcc, and the CPython module
+_calls.so over it with gcc.
 
 Every HIP translation unit is compiled with
   --offload-arch=gfx950 -O3 -ffp-contract=off
@@ -13,12 +14,14 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libhsolve.so")
+CALLS = os.path.join(HERE, "_calls.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -52,6 +55,14 @@ def build(verbose: bool = True) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
+    tmp = CALLS + ".tmp"
+    cmd = ["gcc", "-O2", "-std=c11", "-Wall", "-shared", "-fPIC", "-I", sysconfig.get_paths()["include"],
+           "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, "pycalls.c"), "-L", HERE, "-l:libhsolve.so",
+           "-Wl,-rpath,$ORIGIN", "-Wl,-rpath-link,/opt/rocm/lib", "-o", tmp]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"_calls failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, CALLS)
     if verbose:
         print(f"built {LIB}")
     return LIB

@@ -7,7 +7,7 @@ import ctypes as C
 
 import numpy as np
 
-from ._lib import EllHost, MGParams, ServeParams, ServeResult, ServeStats, check, lib, u64, vp
+from ._lib import EllHost, MGParams, ServeParams, ServeResult, ServeStats, calls, check, lib, u64, vp
 
 _DT = {np.dtype(np.float32): 0, np.dtype(np.float64): 1}
 
@@ -112,9 +112,9 @@ class Q1Matrix:
         self.root = int(round(np.sqrt(self.size)))
         self.bands = [DeviceVector.from_numpy(b) for b in bands]
         self.ptrs = (vp * 9)(*[b.ptr for b in self.bands])
-
-    def band_ptrs(self):
-        return [vp(b.ptr) for b in self.bands]
+        self._bands = C.addressof(self.ptrs)
+        self._product, self._defect, self._jacobi = (
+            getattr(calls(), f"{stem}_{_sfx(self.dtype)}") for stem in ("product_bmdv_q1", "defect_q1", "jacobi_q1"))
 
 
 def fill_poisson_q1(A: Q1Matrix, stream=None):
@@ -140,6 +140,7 @@ class EllMatrix:
                                       u64(num_cols_per_row), u64(threads), Aj.ctypes.data_as(vp),
                                       Ax.ctypes.data_as(vp), arl_p, C.byref(h)), "ell_create")
         self.handle = h.value
+        self._spmv, self._jacobi = calls().ell_spmv, calls().ell_jacobi
         vals = [u64() for _ in range(7)]
         check(lib().hsolve_ell_info(vp(self.handle), *[C.byref(v) for v in vals]), "ell_info")
         (self.rows, self.columns, self.stride, self.ncpr, self.threads, self.nnz,
@@ -161,8 +162,9 @@ class EllMatrix:
         return v.value
 
     def spmv(self, x, y, rhs=None, stream=None):
-        check(lib().hsolve_ell_spmv(vp(self.handle), vp(x.ptr), vp(y.ptr), vp(rhs.ptr) if rhs else None,
-                                    vp(stream)), "ell_spmv")
+        rc = self._spmv(self.handle, x.ptr, y.ptr, rhs.ptr if rhs else None, stream)
+        if rc:
+            check(rc, "ell_spmv")
 
     def spmv_rows(self, x, y, row_start, row_end, rhs=None, stream=None):
         """Rows [row_start, row_end) of y = A x (or rhs - A x); the rest of y untouched."""
@@ -175,8 +177,9 @@ class EllMatrix:
                                     vp(stream)), "ell_spmm")
 
     def jacobi(self, rhs, dinv, x_old, x_new, stream=None):
-        check(lib().hsolve_ell_jacobi(vp(self.handle), vp(rhs.ptr), vp(dinv.ptr), vp(x_old.ptr), vp(x_new.ptr),
-                                      vp(stream)), "ell_jacobi")
+        rc = self._jacobi(self.handle, rhs.ptr, dinv.ptr, x_old.ptr, x_new.ptr, stream)
+        if rc:
+            check(rc, "ell_jacobi")
 
     def __del__(self):
         try:
@@ -271,18 +274,21 @@ def copy_kernel(src: DeviceBuffer, dst: DeviceBuffer, nbytes: int, stream=None):
 
 # ----------------------------------------------------------------- ops
 def q1_product(A: Q1Matrix, x: DeviceVector, y: DeviceVector, stream=None):
-    f = getattr(lib(), f"hsolve_product_bmdv_q1_{_sfx(A.dtype)}")
-    check(f(*A.band_ptrs(), vp(x.ptr), vp(y.ptr), u64(A.size), u64(A.root), vp(stream)), "product_q1")
+    rc = A._product(A._bands, x.ptr, y.ptr, A.size, A.root, stream)
+    if rc:
+        check(rc, "product_q1")
 
 
 def q1_defect(A: Q1Matrix, rhs: DeviceVector, x: DeviceVector, y: DeviceVector, stream=None):
-    f = getattr(lib(), f"hsolve_defect_q1_{_sfx(A.dtype)}")
-    check(f(vp(rhs.ptr), *A.band_ptrs(), vp(x.ptr), vp(y.ptr), u64(A.size), u64(A.root), vp(stream)), "defect_q1")
+    rc = A._defect(rhs.ptr, A._bands, x.ptr, y.ptr, A.size, A.root, stream)
+    if rc:
+        check(rc, "defect_q1")
 
 
 def q1_jacobi(A: Q1Matrix, rhs, dinv, x_old, x_new, stream=None):
-    f = getattr(lib(), f"hsolve_jacobi_q1_{_sfx(A.dtype)}")
-    check(f(vp(rhs.ptr), A.ptrs, vp(dinv.ptr), vp(x_old.ptr), vp(x_new.ptr), u64(A.size), vp(stream)), "jacobi_q1")
+    rc = A._jacobi(rhs.ptr, A._bands, dinv.ptr, x_old.ptr, x_new.ptr, A.size, stream)
+    if rc:
+        check(rc, "jacobi_q1")
 
 
 def dot(a: DeviceVector, b: DeviceVector, stream=None):
