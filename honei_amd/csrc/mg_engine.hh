@@ -222,8 +222,15 @@ namespace mg
     // Host image of a slot's scalars at admission.
     Scalars start_scalars(bool zero_guess);
 
-    // Enqueues one tick for table entries [0, nslots) of finest level L.
-    void enqueue_tick(const Hierarchy & h, uint64_t L, const Slot * table, unsigned nslots, hipStream_t st);
+    // The halves of a tick: start of new solves, FP64 outer step and opening
+    // of inner solves (which also finds a solve done); the V-cycle with its
+    // stopping test.
+    constexpr unsigned kTickOpen = 1, kTickCycle = 2;
+
+    // Enqueues one tick, or a half of one, for table entries [0, nslots) of
+    // finest level L.
+    void enqueue_tick(const Hierarchy & h, uint64_t L, const Slot * table, unsigned nslots, hipStream_t st,
+                      unsigned part = kTickOpen | kTickCycle);
     // Copies every slot's report into `reports` (device, nslots entries).
     void enqueue_report(const Slot * table, unsigned nslots, Report * reports, hipStream_t st);
     // b = U[-1, 1] from SplitMix64(seed, stream) with zero Dirichlet nodes

@@ -1781,7 +1781,7 @@ void enqueue_report(const Slot * table, unsigned nslots, Report * reports, hipSt
 namespace
 {
 template <int MK>
-void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, hipStream_t st)
+void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, unsigned part, hipStream_t st)
 {
     const Params & p = h.p;
     const uint64_t minl = p.min_level;
@@ -1891,52 +1891,59 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
     // FP32 forms the initial norm, the first cycle reads rhs as its defect
     // (initial_zero) and the first stopping test finishes the norm.
     const bool fold = pre2r && p.initial_zero && ! p.convergence_check;
-    hipLaunchKernelGGL(tick_begin_kernel, ggrid(grid_for(top.n, kBlock)), blk, 0, st, T, (int)maxl, n, top.side, fx_top);
-    if (maxl > minl && ! pre2r)
+    const unsigned open_blocks = fold ? std::min<unsigned>(ggrid(lanes4(top.n)).x, kNormBlocks) : 0;
+    if (part & kTickOpen)
     {
-        // (the one-pass kernels write every coarser iterate before it is read)
-        LevelSizes sz;
-        for (int l = 0; l < kMaxLevels; ++l)
-            sz.n[l] = (int64_t)h.lv[l].n;
-        hipLaunchKernelGGL(start_zero_kernel, ggrid(grid_for(h.lv[maxl - 1].n, kBlock)), blk, 0, st, T,
-                           (int)minl, (int)maxl, sz);
-    }
-    const unsigned od_blocks = std::min<unsigned>(grid_for((top.n + 1) / 2, kBlock), kNormBlocks);
-    bool od_coded = false;
-    if constexpr (MK == 0)
-    {
-        if (h.use_codes && h.codes64[maxl])
+        hipLaunchKernelGGL(tick_begin_kernel, ggrid(grid_for(top.n, kBlock)), blk, 0, st, T, (int)maxl, n, top.side, fx_top);
+        if (maxl > minl && ! pre2r)
         {
-            hipLaunchKernelGGL((outer_defect_kernel<MK, true>), dim3(od_blocks, 1, S), blk, 0, st, h.B64(maxl),
-                               h.ell64[maxl], T, n, top.side, (const uint64_t *)h.codes64[maxl],
-                               (const double *)h.ctab64[maxl]);
-            od_coded = true;
+            // (the one-pass kernels write every coarser iterate before it is read)
+            LevelSizes sz;
+            for (int l = 0; l < kMaxLevels; ++l)
+                sz.n[l] = (int64_t)h.lv[l].n;
+            hipLaunchKernelGGL(start_zero_kernel, ggrid(grid_for(h.lv[maxl - 1].n, kBlock)), blk, 0, st, T,
+                               (int)minl, (int)maxl, sz);
+        }
+        const unsigned od_blocks = std::min<unsigned>(grid_for((top.n + 1) / 2, kBlock), kNormBlocks);
+        bool od_coded = false;
+        if constexpr (MK == 0)
+        {
+            if (h.use_codes && h.codes64[maxl])
+            {
+                hipLaunchKernelGGL((outer_defect_kernel<MK, true>), dim3(od_blocks, 1, S), blk, 0, st, h.B64(maxl),
+                                   h.ell64[maxl], T, n, top.side, (const uint64_t *)h.codes64[maxl],
+                                   (const double *)h.ctab64[maxl]);
+                od_coded = true;
+            }
+        }
+        if (! od_coded)
+            hipLaunchKernelGGL((outer_defect_kernel<MK>), dim3(od_blocks, 1, S), blk, 0, st,
+                               kBands<MK> ? h.B64(maxl) : k::Bands{}, h.ell64[maxl], T, n, top.side,
+                               (const uint64_t *)nullptr, (const double *)nullptr);
+        hipLaunchKernelGGL(outer_defect_finish_kernel, dim3(1, 1, S), blk, 0, st, T, od_blocks, (double)p.tolerance,
+                           p.max_outer, fold ? 1 : 0);
+        if (fold)
+        {
+            hipLaunchKernelGGL((to_inner_kernel<true>), dim3(open_blocks, 1, S), blk, 0, st, T, (int)maxl, n);
+        }
+        else
+        {
+            hipLaunchKernelGGL((to_inner_kernel<false>), ggrid(lanes4(top.n)), blk, 0, st, T, (int)maxl, n);
+            if (p.initial_zero)
+                hipLaunchKernelGGL((open_inner_kernel<1, MK>), ggrid(lanes4(top.n)), blk, 0, st, largs(maxl), T,
+                                   (int)maxl, fx_top);
+            else
+                hipLaunchKernelGGL((open_inner_kernel<0, MK>), ggrid(rgrid(top.n)), blk, 0, st, largs(maxl), T,
+                                   (int)maxl, fx_top);
+            hipLaunchKernelGGL((inner_norm_kernel<0>), norm_grid(top.n), blk, 0, st, T, (int)maxl, n);
+            hipLaunchKernelGGL((inner_norm_finish_kernel<0>), dim3(1, 1, S), blk, 0, st, T, norm_grid(top.n).x,
+                               p.tolerance, p.convergence_check, p.n_max_iter);
         }
     }
-    if (! od_coded)
-        hipLaunchKernelGGL((outer_defect_kernel<MK>), dim3(od_blocks, 1, S), blk, 0, st,
-                           kBands<MK> ? h.B64(maxl) : k::Bands{}, h.ell64[maxl], T, n, top.side,
-                           (const uint64_t *)nullptr, (const double *)nullptr);
-    hipLaunchKernelGGL(outer_defect_finish_kernel, dim3(1, 1, S), blk, 0, st, T, od_blocks, (double)p.tolerance,
-                       p.max_outer, fold ? 1 : 0);
-    unsigned open_blocks = 0;
-    if (fold)
+    if (! (part & kTickCycle))
     {
-        open_blocks = std::min<unsigned>(ggrid(lanes4(top.n)).x, kNormBlocks);
-        hipLaunchKernelGGL((to_inner_kernel<true>), dim3(open_blocks, 1, S), blk, 0, st, T, (int)maxl, n);
-    }
-    else
-    {
-        hipLaunchKernelGGL((to_inner_kernel<false>), ggrid(lanes4(top.n)), blk, 0, st, T, (int)maxl, n);
-        if (p.initial_zero)
-            hipLaunchKernelGGL((open_inner_kernel<1, MK>), ggrid(lanes4(top.n)), blk, 0, st, largs(maxl), T,
-                               (int)maxl, fx_top);
-        else
-            hipLaunchKernelGGL((open_inner_kernel<0, MK>), ggrid(rgrid(top.n)), blk, 0, st, largs(maxl), T,
-                               (int)maxl, fx_top);
-        hipLaunchKernelGGL((inner_norm_kernel<0>), norm_grid(top.n), blk, 0, st, T, (int)maxl, n);
-        hipLaunchKernelGGL((inner_norm_finish_kernel<0>), dim3(1, 1, S), blk, 0, st, T, norm_grid(top.n).x,
-                           p.tolerance, p.convergence_check, p.n_max_iter);
+        HIP_CHECK(hipGetLastError());
+        return;
     }
 
     // ---- one V-cycle (multigrid.hh:1660-1905)
@@ -2159,14 +2166,14 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, h
 }
 }  // namespace
 
-void enqueue_tick(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, hipStream_t st)
+void enqueue_tick(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, hipStream_t st, unsigned part)
 {
     if (h.kind == 1)
-        tick_impl<1>(h, maxl, T, S, st);
+        tick_impl<1>(h, maxl, T, S, part, st);
     else if (h.kind == 2)
-        tick_impl<2>(h, maxl, T, S, st);
+        tick_impl<2>(h, maxl, T, S, part, st);
     else
-        tick_impl<0>(h, maxl, T, S, st);
+        tick_impl<0>(h, maxl, T, S, part, st);
 }
 
 }  // namespace mg

@@ -78,11 +78,21 @@ namespace
         }
         HIP_CHECK(hipMemcpyAsync(mg->table, tab.data(), sizeof(mg::Slot) * count, hipMemcpyHostToDevice, st));
         const unsigned S = (unsigned)count;
+        // A solve is found done in the first half of a tick, so a chunk ends
+        // there: the V-cycle of its last tick, 6 to 14 launches that would find
+        // nothing to do, follows only when a slot goes on (measured on
+        // MI355X, a solve to 1e-8: 129^2 677 -> 661 us, 1025^2 1675 -> 1655 us).
         uint64_t chunk = mg->last_ticks > 2 ? mg->last_ticks : 2;
+        bool first = true;
         while (true)
         {
             for (uint64_t c = 0; c < chunk; ++c)
-                mg::enqueue_tick(mg->h, mg->max_level, mg->table, S, st);
+            {
+                if (! first)
+                    mg::enqueue_tick(mg->h, mg->max_level, mg->table, S, st, mg::kTickCycle);
+                mg::enqueue_tick(mg->h, mg->max_level, mg->table, S, st, mg::kTickOpen);
+                first = false;
+            }
             mg::enqueue_report(mg->table, S, mg->report, st);
             HIP_CHECK(hipMemcpyAsync(mg->report_host, mg->report, sizeof(mg::Report) * S, hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
