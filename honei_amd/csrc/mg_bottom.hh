@@ -1,7 +1,7 @@
 // mg_bottom.hh -- the V-cycle's bottom levels in one workgroup per slot.
 // Included by mg_engine.hip.
 //
-// Levels minl .. top (top <= 5, below the finest) of a V-cycle on Q1 bands:
+// Levels minl .. top (top <= 6, below the finest) of a V-cycle on Q1 bands:
 // two sweeps from zero, defect and restriction down to minl, the coarse CG,
 // then prolongation with the correction factor and two sweeps back up, the
 // same operations per node as the one-pass kernels and the coarse solve run
@@ -11,7 +11,7 @@
 
 namespace
 {
-    constexpr int kBottomMax = 5;
+    constexpr int kBottomMax = 6;
     constexpr int kBottomLanes = 1024;
     template <int L> constexpr int kSide = (1 << L) + 1;
     template <int L> constexpr int kSize = kSide<L> * kSide<L>;
@@ -21,7 +21,7 @@ namespace
     // selects the value away
     template <int L> constexpr int kBottomOff = kBottomOff<L - 1> + 3 * kSize<L - 1>;
     template <> constexpr int kBottomOff<1> = kSide<kBottomMax> + 1;
-    constexpr int kBottomFloats = kBottomOff<kBottomMax> + 3 * kSize<kBottomMax> + kSide<kBottomMax> + 1;
+    template <int L> constexpr int kBottomFloats = kBottomOff<L> + 3 * kSize<L> + kSide<L> + 1;
 
     struct BottomArgs
     {
@@ -125,9 +125,16 @@ namespace
     }
 
     // MINL: the coarsest level (1 or 2: a lane per node in the CG).  Each lane
-    // owns rows tid, tid + 1024 of every level and keeps their bands and dinv
-    // in registers, all loaded in one round trip; LDS holds the vectors.
-    template <int MK, int MINL>
+    // owns rows tid, tid + 1024, ... of every level and keeps their bands and
+    // dinv in registers; LDS holds the vectors.  Up to level 5 every band is
+    // loaded in one round trip.  TOP6 (top is 6): level 6 takes 50 registers
+    // for its five rows, so its bands are loaded twice, for the way down with
+    // level 5's and for the way up before or after the coarse solve, which with
+    // the levels between hides them.
+    // With level 6 here a cycle saves two launches of 7 to 10 us (measured on
+    // MI355X, a solve: 129^2 661 -> 598 us, 1025^2 1655 -> 1583 us, 4097^2
+    // 4957 -> 4887 us, 64 of 513^2 1.03x).  Level 7 would need 17 rows a lane.
+    template <int MK, int MINL, bool TOP6>
     __global__ __launch_bounds__(kBottomLanes) void v_bottom_kernel(BottomArgs ba, const Slot * T)
     {
         const VB vb = vblock();
@@ -135,30 +142,44 @@ namespace
         if (! live(sl) || sl.s->run == 0)
             return;
         constexpr int ORD = kOrd<MK>;
-        __shared__ float lds[kBottomFloats];
+        __shared__ float lds[kBottomFloats<TOP6 ? 6 : 5>];
         const int tid = threadIdx.x;
-        float b5[2][10], b4[10], b3[10], b2[10], b1[10];
-        auto load = [&](auto l_tag, int r, float (&b)[10]) {
+        float b6[TOP6 ? kRowsPerLane<6> : 1][10], b5[2][10], b4[10], b3[10], b2[10], b1[10];
+        auto load_from = [&](auto l_tag, int r, int k0, float (&b)[10]) {
             constexpr int L = decltype(l_tag)::value;
             const LevelArgs & a = ba.lv[L];
-            const int i = min(tid + r * kBottomLanes, kSize<L> - 1);
+            const int i = min(tid + r * kBottomLanes, kSize<L> - 1) + k0;
 #pragma unroll
             for (int k = 0; k < 10; ++k)
                 b[k] = as_global<const float>(k < 9 ? (const float *)a.B.b[k] : a.dinv)[i];
         };
-        const int top = ba.top;
+        auto load = [&](auto l_tag, int r, float (&b)[10]) { load_from(l_tag, r, 0, b); };
+        auto load6 = [&]() {
+            int zero = 0;
+            asm volatile("" : "+v"(zero));   // a second load, not the first one's registers kept
+#pragma unroll
+            for (int r = 0; r < kRowsPerLane<6>; ++r)
+                load_from(IntC<6>{}, r, zero, b6[TOP6 ? r : 0]);
+        };
+        auto load_low = [&](int top) {
+            if (top >= 4)
+                load(IntC<4>{}, 0, b4);
+            if (top >= 3)
+                load(IntC<3>{}, 0, b3);
+            load(IntC<2>{}, 0, b2);
+            if (MINL == 1)
+                load(IntC<1>{}, 0, b1);
+        };
+        const int top = TOP6 ? 6 : ba.top;
+        if constexpr (TOP6)
+            load6();
         if (top >= 5)
         {
             load(IntC<5>{}, 0, b5[0]);
             load(IntC<5>{}, 1, b5[1]);
         }
-        if (top >= 4)
-            load(IntC<4>{}, 0, b4);
-        if (top >= 3)
-            load(IntC<3>{}, 0, b3);
-        load(IntC<2>{}, 0, b2);
-        if (MINL == 1)
-            load(IntC<1>{}, 0, b1);
+        if (! TOP6)
+            load_low(top);
         {
             auto take = [&](auto l_tag) {
                 constexpr int L = decltype(l_tag)::value;
@@ -166,7 +187,9 @@ namespace
                 for (int i = tid; i < kSize<L>; i += kBottomLanes)
                     lds[kBottomOff<L> + i] = g[i];
             };
-            if (top == 5)
+            if constexpr (TOP6)
+                take(IntC<6>{});
+            else if (top == 5)
                 take(IntC<5>{});
             else if (top == 4)
                 take(IntC<4>{});
@@ -179,7 +202,9 @@ namespace
         // the rows' bands of level L
         auto bands = [&](auto l_tag, int r) -> const float (&)[10] {
             constexpr int L = decltype(l_tag)::value;
-            if constexpr (L == 5)
+            if constexpr (L == 6)
+                return b6[TOP6 ? r : 0];
+            else if constexpr (L == 5)
                 return b5[r];
             else if constexpr (L == 4)
                 return b4;
@@ -212,10 +237,10 @@ namespace
             });
             each(l_tag, [&](int i, const float (&b)[10]) { tmp[i] = rhs[i] - bottom_row<L, ORD>(b, x, i); });
             float * crhs = lds + kBottomOff<L - 1>;
-            if (tid < Nc * Nc)
+            for (int c = tid; c < Nc * Nc; c += kBottomLanes)
             {
-                const int r = tid / Nc, s = tid - r * Nc;
-                crhs[tid] = k::restrict_node<float>(
+                const int r = c / Nc, s = c - r * Nc;
+                crhs[c] = k::restrict_node<float>(
                     [&](int dr, int ds) { return tmp[min(max((2 * r + dr) * m + 2 * s + ds, 0), n - 1)]; }, r, s, Nc,
                     ba.mk);
             }
@@ -244,10 +269,17 @@ namespace
                 tmp[i] = x[i] + t * b[9];
             });
         };
+        if constexpr (TOP6)
+        {
+            down(IntC<6>{});
+            load_low(6);
+        }
         if (top >= 5) down(IntC<5>{});
         if (top >= 4) down(IntC<4>{});
         if (top >= 3) down(IntC<3>{});
         if (MINL == 1 && top >= 2) down(IntC<2>{});
+        if constexpr (TOP6 && MINL == 2)
+            load6();
         if (tid < 64)
         {
             constexpr int n = kSize<MINL>;
@@ -258,9 +290,13 @@ namespace
         }
         lds_barrier();
         if (MINL == 1 && top >= 2) up(IntC<2>{});
+        if constexpr (TOP6 && MINL == 1)
+            load6();
         if (top >= 3) up(IntC<3>{});
         if (top >= 4) up(IntC<4>{});
         if (top >= 5) up(IntC<5>{});
+        if constexpr (TOP6)
+            up(IntC<6>{});
         {
             auto leave = [&](auto l_tag) {
                 constexpr int L = decltype(l_tag)::value;
@@ -268,7 +304,9 @@ namespace
                 for (int i = tid; i < kSize<L>; i += kBottomLanes)
                     g[i] = lds[kBottomOff<L> + 2 * kSize<L> + i];
             };
-            if (top == 5)
+            if constexpr (TOP6)
+                leave(IntC<6>{});
+            else if (top == 5)
                 leave(IntC<5>{});
             else if (top == 4)
                 leave(IntC<4>{});

@@ -1837,7 +1837,7 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, u
     // when the transfers are the structured ones and the correction factor
     // is fixed (the adaptive one reads the level's defect again).
     const bool pre2r = post2 && p.adapt != 0.0f && ! h.prolmat;
-    // With the one-pass kernels, levels minl .. btop (btop <= 5, below the
+    // With the one-pass kernels, levels minl .. btop (btop <= 6, below the
     // finest) run in one launch, one workgroup per slot: v_bottom_kernel when
     // the coarsest level fits one wave (5^2 or less), v_bottom_lds_kernel with
     // as many levels as fit the LDS of a workgroup otherwise; btop = 0: none.
@@ -2051,10 +2051,18 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, u
         // with one level it sees the finest defect d
         const LevelArgs a = largs(minl);
         const int crhs = (minl == maxl) ? F_D : F_RHS;
-        if (btop && minl == 1)
-            hipLaunchKernelGGL((v_bottom_kernel<MK, 1>), dim3(1, 1, S), dim3(kBottomLanes), 0, st, ba.b, T);
+        auto bottom = [&](auto minl_tag, auto top6_tag) {
+            hipLaunchKernelGGL((v_bottom_kernel<MK, decltype(minl_tag)::value, decltype(top6_tag)::value != 0>),
+                               dim3(1, 1, S), dim3(kBottomLanes), 0, st, ba.b, T);
+        };
+        if (btop == 6 && minl == 1)
+            bottom(IntC<1>{}, IntC<1>{});
+        else if (btop == 6 && minl == 2)
+            bottom(IntC<2>{}, IntC<1>{});
+        else if (btop && minl == 1)
+            bottom(IntC<1>{}, IntC<0>{});
         else if (btop && minl == 2)
-            hipLaunchKernelGGL((v_bottom_kernel<MK, 2>), dim3(1, 1, S), dim3(kBottomLanes), 0, st, ba.b, T);
+            bottom(IntC<2>{}, IntC<0>{});
         else if (btop)
             hipLaunchKernelGGL((v_bottom_lds_kernel<MK>), dim3(1, 1, S), dim3(1024), bbytes, st, ba, T);
         else if (a.n <= kCoarseLdsMax)

@@ -96,6 +96,25 @@ def test_bottom_levels_equal_oracle(hip, oracle, level, minl):
         assert np.array_equal(xd.get(), ref["x"]), (mask, np.count_nonzero(xd.get() != ref["x"]))
 
 
+@pytest.mark.parametrize("level,minl", [(7, 1), (8, 1), (8, 2)])
+def test_bottom_up_to_65_equals_oracle(hip, oracle, level, minl):
+    """The bottom kernel with 65^2 as its top level, on both coarsest levels of one wave."""
+    g = np.random.default_rng(10 * level + minl)
+    n = P.side_of_level(level) ** 2
+    a32 = {L: _bands("plain", L, g) for L in range(minl, level + 1)}
+    d32 = {L: dinv_reference(a32[L][4]) for L in a32}
+    A64 = [b.astype(np.float64) for b in a32[level]]
+    for mask in MASKS.values():
+        b = g.uniform(-1, 1, n)
+        ref = oracle.mg_mixed_q1(A64, b, np.zeros(n), a32, d32, min_level=minl, max_level=level, mask=mask, max_outer=1)
+        assert np.isfinite(ref["x"]).all()
+        mg = hip.MGSolver(hip.mg_params(minl, level, mask=mask, max_outer=1), A64, a32, d32)
+        xd = hip.DeviceVector.zeros(n)
+        info = mg.solve(hip.DeviceVector.from_numpy(b), xd, raise_on_cap=False)
+        assert (info["outer"], info["inner"]) == (ref["outer"], ref["inner"])
+        assert np.array_equal(xd.get(), ref["x"]), (mask, np.count_nonzero(xd.get() != ref["x"]))
+
+
 @pytest.mark.parametrize("level", [6, 9])
 def test_batch_of_three_equals_single(hip, level):
     """Two slots share a workgroup's matrix loads, the third has one alone."""
