@@ -773,21 +773,26 @@ namespace k
             y[r] = o;
     }
 
-    // Q1 row sums of V consecutive rows i0..i0+V-1 that lie away from both
-    // ends of the vector (every index guard of q1_row holds): bands come in
-    // as one 16-byte load each, x from the three row windows.  Each row's
-    // sum runs in q1_row's order.
-    template <typename DT, int ORD = 0>
-    __device__ __forceinline__ void q1_rows_v(const Bands & B, const DT * __restrict__ x, int64_t i0, int64_t m,
-                                              DT (&out)[Vec16<DT>::V])
+    // The nine bands of V consecutive rows i0..i0+V-1, one 16-byte load each
+    template <typename DT>
+    __device__ __forceinline__ void q1_bands_v(const Bands & B, int64_t i0, typename Vec16<DT>::type (&bv)[9])
     {
-        constexpr int V = Vec16<DT>::V;
         typedef typename Vec16<DT>::type VT;
         const DT * const * b = reinterpret_cast<const DT * const *>(B.b);
-        VT bv[9];
 #pragma unroll
         for (int k = 0; k < 9; ++k)
             bv[k] = __builtin_nontemporal_load((const VT *)(b[k] + i0));
+    }
+
+    // Q1 row sums of V consecutive rows i0..i0+V-1 that lie away from both
+    // ends of the vector (every index guard of q1_row holds) from their bands;
+    // x comes from the three row windows.  Each row's sum runs in q1_row's
+    // order.
+    template <typename DT, int ORD = 0>
+    __device__ __forceinline__ void q1_sums_v(const typename Vec16<DT>::type (&bv)[9], const DT * __restrict__ x,
+                                              int64_t i0, int64_t m, DT (&out)[Vec16<DT>::V])
+    {
+        constexpr int V = Vec16<DT>::V;
         DT xm[V + 2], xc[V + 2], xp[V + 2];
         ld_window<V + 2>(x + i0 - m - 1, xm);
         ld_window<V + 2>(x + i0 - 1, xc);
@@ -825,6 +830,16 @@ namespace k
             s += bv[8][v] * xp[v + 2];
             out[v] = s;
         }
+    }
+
+    // both of them
+    template <typename DT, int ORD = 0>
+    __device__ __forceinline__ void q1_rows_v(const Bands & B, const DT * __restrict__ x, int64_t i0, int64_t m,
+                                              DT (&out)[Vec16<DT>::V])
+    {
+        typename Vec16<DT>::type bv[9];
+        q1_bands_v<DT>(B, i0, bv);
+        q1_sums_v<DT, ORD>(bv, x, i0, m, out);
     }
 
     // Vectorised form of q1_kernel: V = 16 / sizeof(DT) rows per lane; lane

@@ -177,11 +177,30 @@ namespace
         }
         else if (closes(s))
         {
+            // four rows a lane (result is the caller's, 8-byte aligned; x32 is
+            // the slot's): a workgroup's accesses cover 8 KB of every array
+            // (measured on MI355X, 64 slots of 513^2: 92 -> 70 us, one row a
+            // lane before; one slot of 4097^2: 48 us both ways)
+            typedef double D4 __attribute__((ext_vector_type(4), aligned(8)));
+            typedef float F4 __attribute__((ext_vector_type(4)));
             const double scale = s->scale;
             const gptr<double> x = as_global(sl.result);
             const gptr<const float> c = as_global<const float>(sl.v[L][fx]);
-            for (int64_t i = i0; i < n; i += stride)
-                x[i] = x[i] + scale * (double)c[i];
+            for (int64_t i = 4 * i0; i < n; i += 4 * stride)
+            {
+                if (i + 4 <= n)
+                {
+                    D4 v = *(gptr<const D4>)(x + i);
+                    const F4 w = *(gptr<const F4>)(c + i);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        v[q] = v[q] + scale * (double)w[q];
+                    *(gptr<D4>)(x + i) = v;
+                }
+                else
+                    for (int64_t j = i; j < n; ++j)
+                        x[j] = x[j] + scale * (double)c[j];
+            }
         }
     }
 
@@ -205,10 +224,16 @@ namespace
     // CB: the interior rows read the bands as value codes (one 64-bit word
     // per row, band k in bits 4k .. 4k + 3) and look them up in ctab
     // (16 per band, copied to LDS); the same values, the same sums.
-    template <int MK, bool CB = false>
+    //
+    // KS: slots per workgroup.  The bands are 72 bytes a node where a slot's
+    // vectors are 24, so with several slots one load of them serves KS (bands
+    // without codes).  Bound by the L2: measured on MI355X, 64 slots of 513^2,
+    // one slot a workgroup 172 us (9.4 TB/s of L2 and HBM together), four 133.
+    template <int MK, bool CB = false, int KS = 1>
     __global__ __launch_bounds__(256) void outer_defect_kernel(k::Bands B, EllMat64 E, const Slot * T, int64_t n,
-            int64_t m, const uint64_t * __restrict__ codes, const double * __restrict__ ctab)
+            int64_t m, const uint64_t * __restrict__ codes, const double * __restrict__ ctab, int S)
     {
+        static_assert(KS == 1 || (kBands<MK> && ! CB), "several slots: plain bands");
         __shared__ double tab[CB ? 144 : 1];
         if constexpr (CB)
         {
@@ -217,24 +242,34 @@ namespace
             __syncthreads();
         }
         const VB vb = vblock();
-        const Slot & sl = T[vb.z];
-        if (! live(sl))
+        bool on[KS], any = false;
+        const double * b[KS];
+        const double * x[KS];
+        double * od[KS];
+        double acc[KS];
+#pragma unroll
+        for (int q = 0; q < KS; ++q)
+        {
+            const int z = (int)vb.z * KS + q;
+            const Slot & sl = T[z < S ? z : 0];
+            on[q] = z < S && live(sl) && (starts(sl.s) || closes(sl.s));
+            any = any || on[q];
+            b[q] = (const double *)as_global<const double>(sl.b);
+            x[q] = (const double *)as_global<const double>(sl.result);
+            od[q] = (double *)as_global(sl.od);
+            acc[q] = 0.0;
+        }
+        if (! any)
             return;
-        if (! starts(sl.s) && ! closes(sl.s))
-            return;
-        const double * __restrict__ b = sl.b;
-        const double * __restrict__ x = sl.result;
-        double * __restrict__ od = sl.od;
-        double acc = 0.0;
         if (MK == 1)
         {
             // one row per lane and pass, lanes on consecutive rows
             const int64_t stride1 = (int64_t)gridDim.x * blockDim.x;
             for (int64_t i = (int64_t)vb.x * blockDim.x + threadIdx.x; i < n; i += stride1)
             {
-                const double di = b[i] - ell_row<double>(E, x, i);
-                od[i] = di;
-                acc += di * di;
+                const double di = b[0][i] - ell_row<double>(E, x[0], i);
+                od[0][i] = di;
+                acc[0] += di * di;
             }
         }
         const int64_t stride = (int64_t)gridDim.x * blockDim.x * 2;
@@ -243,60 +278,74 @@ namespace
             if (i0 - m - 1 >= 0 && i0 + 2 + m < n)
             {
                 // b and x are the caller's arrays (8-byte aligned), od is the slot's
-                double prod[2];
-                if constexpr (CB)
-                {
-                    // q1_rows_v's sums (Product<Q1>'s order: dd first) with
-                    // the band values from the codes of rows i0, i0 + 1
-                    typedef uint64_t U2 __attribute__((ext_vector_type(2)));
-                    const U2 cw = __builtin_nontemporal_load((const U2 *)(codes + i0));
-                    double xm[4], xc[4], xp[4];
-#pragma unroll
-                    for (int jj = 0; jj < 4; ++jj)
-                    {
-                        xm[jj] = x[i0 - m - 1 + jj];
-                        xc[jj] = x[i0 - 1 + jj];
-                        xp[jj] = x[i0 + m - 1 + jj];
-                    }
-#pragma unroll
-                    for (int v = 0; v < 2; ++v)
-                    {
-                        const uint64_t w = cw[v];
-                        auto bk = [&](int k) { return tab[16 * k + (int)((w >> (4 * k)) & 15u)]; };
-                        double sum = bk(4) * xc[v + 1];
-                        sum += bk(0) * xm[v];
-                        sum += bk(1) * xm[v + 1];
-                        sum += bk(2) * xm[v + 2];
-                        sum += bk(3) * xc[v];
-                        sum += bk(5) * xc[v + 2];
-                        sum += bk(6) * xp[v];
-                        sum += bk(7) * xp[v + 1];
-                        sum += bk(8) * xp[v + 2];
-                        prod[v] = sum;
-                    }
-                }
-                else
-                    k::q1_rows_v<double, kOrd<MK>>(B, x, i0, m, prod);
                 typedef k::Vec16<double>::type V2;
-                V2 o;
-                o[0] = __builtin_nontemporal_load(b + i0) - prod[0];
-                o[1] = __builtin_nontemporal_load(b + i0 + 1) - prod[1];
-                *(V2 *)(od + i0) = o;
-                acc += o[0] * o[0];
-                acc += o[1] * o[1];
+                typedef double U2 __attribute__((ext_vector_type(2), aligned(8)));
+                V2 bv[9];
+                if constexpr (! CB)
+                    k::q1_bands_v<double>(B, i0, bv);
+#pragma unroll
+                for (int q = 0; q < KS; ++q)
+                {
+                    if (! on[q])
+                        continue;
+                    const U2 bb = __builtin_nontemporal_load((const U2 *)(b[q] + i0));
+                    double prod[2];
+                    if constexpr (CB)
+                    {
+                        // q1_sums_v's sums (Product<Q1>'s order: dd first) with
+                        // the band values from the codes of rows i0, i0 + 1
+                        typedef uint64_t C2 __attribute__((ext_vector_type(2)));
+                        const C2 cw = __builtin_nontemporal_load((const C2 *)(codes + i0));
+                        double xm[4], xc[4], xp[4];
+                        k::ld_window<4>(x[q] + i0 - m - 1, xm);
+                        k::ld_window<4>(x[q] + i0 - 1, xc);
+                        k::ld_window<4>(x[q] + i0 + m - 1, xp);
+#pragma unroll
+                        for (int v = 0; v < 2; ++v)
+                        {
+                            const uint64_t w = cw[v];
+                            auto bk = [&](int k) { return tab[16 * k + (int)((w >> (4 * k)) & 15u)]; };
+                            double sum = bk(4) * xc[v + 1];
+                            sum += bk(0) * xm[v];
+                            sum += bk(1) * xm[v + 1];
+                            sum += bk(2) * xm[v + 2];
+                            sum += bk(3) * xc[v];
+                            sum += bk(5) * xc[v + 2];
+                            sum += bk(6) * xp[v];
+                            sum += bk(7) * xp[v + 1];
+                            sum += bk(8) * xp[v + 2];
+                            prod[v] = sum;
+                        }
+                    }
+                    else
+                        k::q1_sums_v<double, kOrd<MK>>(bv, x[q], i0, m, prod);
+                    V2 o;
+                    o[0] = bb[0] - prod[0];
+                    o[1] = bb[1] - prod[1];
+                    *(V2 *)(od[q] + i0) = o;
+                    acc[q] += o[0] * o[0];
+                    acc[q] += o[1] * o[1];
+                }
             }
             else
             {
                 for (int64_t i = i0; i < i0 + 2 && i < n; ++i)
-                {
-                    const double prod = k::q1_row<double, kOrd<MK>>(B, x, i, n, m);
-                    const double di = b[i] - prod;
-                    od[i] = di;
-                    acc += di * di;
-                }
+#pragma unroll
+                    for (int q = 0; q < KS; ++q)
+                    {
+                        if (! on[q])
+                            continue;
+                        const double prod = k::q1_row<double, kOrd<MK>>(B, x[q], i, n, m);
+                        const double di = b[q][i] - prod;
+                        od[q][i] = di;
+                        acc[q] += di * di;
+                    }
             }
         }
-        k::put_partials2(acc, 0.0, sl.partials, vb.x);
+#pragma unroll
+        for (int q = 0; q < KS; ++q)
+            if (on[q])
+                k::put_partials2(acc[q], 0.0, T[vb.z * KS + q].partials, vb.x);
     }
 
     // |od| from the partials of outer_defect_kernel (nb blocks per slot), then
@@ -1912,14 +1961,30 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, u
             {
                 hipLaunchKernelGGL((outer_defect_kernel<MK, true>), dim3(od_blocks, 1, S), blk, 0, st, h.B64(maxl),
                                    h.ell64[maxl], T, n, top.side, (const uint64_t *)h.codes64[maxl],
-                                   (const double *)h.ctab64[maxl]);
+                                   (const double *)h.ctab64[maxl], (int)S);
                 od_coded = true;
             }
         }
         if (! od_coded)
-            hipLaunchKernelGGL((outer_defect_kernel<MK>), dim3(od_blocks, 1, S), blk, 0, st,
-                               kBands<MK> ? h.B64(maxl) : k::Bands{}, h.ell64[maxl], T, n, top.side,
-                               (const uint64_t *)nullptr, (const double *)nullptr);
+        {
+            auto go = [&](auto k_tag) {
+                constexpr int KS = decltype(k_tag)::value;
+                hipLaunchKernelGGL((outer_defect_kernel<MK, false, KS>), dim3(od_blocks, 1, (S + KS - 1) / KS), blk, 0, st,
+                                   kBands<MK> ? h.B64(maxl) : k::Bands{}, h.ell64[maxl], T, n, top.side,
+                                   (const uint64_t *)nullptr, (const double *)nullptr, (int)S);
+            };
+            if constexpr (kBands<MK>)
+            {
+                if (S > 2)
+                    go(IntC<4>{});
+                else if (S == 2)
+                    go(IntC<2>{});
+                else
+                    go(IntC<1>{});
+            }
+            else
+                go(IntC<1>{});
+        }
         hipLaunchKernelGGL(outer_defect_finish_kernel, dim3(1, 1, S), blk, 0, st, T, od_blocks, (double)p.tolerance,
                            p.max_outer, fold ? 1 : 0);
         if (fold)

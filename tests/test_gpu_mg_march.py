@@ -132,3 +132,26 @@ def test_batch_of_three_equals_single(hip, level):
         one.fill(0.0)
         mg.solve(b, one, raise_on_cap=False)
         assert np.array_equal(x.get(), one.get())
+
+
+@pytest.mark.parametrize("S", [2, 5, 8])
+def test_outer_defect_of_several_slots_equals_single(hip, S):
+    """Groups of two and four slots share a workgroup's FP64 bands; the last group of five holds one.  Columns of
+    different smoothness end their inner solves, and the whole solve, in different ticks."""
+    level = 7
+    n = P.side_of_level(level) ** 2
+    g = np.random.default_rng(S)
+    prm = hip.mg_params(MINL, level, mask=P.DIFFUSION_MASK)
+    a32 = {L: P.diffusion_ell(L, dtype=np.float32) for L in range(MINL, level + 1)}
+    A64 = P.diffusion_ell(level)
+    B = [np.ones(n) if j % 3 == 1 else g.uniform(-1, 1, n) * (np.arange(n) < n // (1 + j)) for j in range(S)]
+    mg = hip.MGSolver.from_ell(prm, A64, a32, slots=S)
+    bd = [hip.DeviceVector.from_numpy(b) for b in B]
+    xd = [hip.DeviceVector.zeros(n) for _ in B]
+    infos = mg.solve_batch(bd, xd)
+    one = hip.MGSolver.from_ell(prm, A64, a32)
+    for j in range(S):
+        x = hip.DeviceVector.zeros(n)
+        info = one.solve(bd[j], x)
+        assert np.array_equal(x.get(), xd[j].get()), j
+        assert (info["outer"], info["inner"]) == (infos[j]["outer"], infos[j]["inner"])
