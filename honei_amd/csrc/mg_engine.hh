@@ -162,6 +162,9 @@ namespace mg
         uint64_t bs64[kMaxLevels] = {};
         uint64_t * codes64[kMaxLevels] = {};  // value codes of the FP64 bands (as HierLevel::codes,
         double * ctab64[kMaxLevels] = {};     // nine arrays), or null
+        uint8_t * rcode64[kMaxLevels] = {};   // row codes instead (as HierLevel::rcode), the nine values
+        double * rtab64[kMaxLevels] = {};     // of each distinct row, and their number; or null
+        int rows64[kMaxLevels] = {};
         EllMat64 ell64[kMaxLevels];          // FP64 finest ELL matrix (ELL hierarchies)
         std::vector<void *> allocations;
         uint64_t bytes = 0;

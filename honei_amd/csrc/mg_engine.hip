@@ -177,8 +177,8 @@ namespace
         }
         else if (closes(s))
         {
-            // four rows a lane (result is the caller's, 8-byte aligned; x32 is
-            // the slot's): a workgroup's accesses cover 8 KB of every array
+            // four rows a lane where there is more than one (result is the
+            // caller's, 8-byte aligned; x32 is the slot's): a workgroup's accesses cover 8 KB of every array
             // (measured on MI355X, 64 slots of 513^2: 92 -> 70 us, one row a
             // lane before; one slot of 4097^2: 48 us both ways)
             typedef double D4 __attribute__((ext_vector_type(4), aligned(8)));
@@ -186,6 +186,12 @@ namespace
             const double scale = s->scale;
             const gptr<double> x = as_global(sl.result);
             const gptr<const float> c = as_global<const float>(sl.v[L][fx]);
+            if (n <= stride)
+            {
+                if (i0 < n)
+                    x[i0] = x[i0] + scale * (double)c[i0];
+                return;
+            }
             for (int64_t i = 4 * i0; i < n; i += 4 * stride)
             {
                 if (i + 4 <= n)
@@ -221,26 +227,29 @@ namespace
     // the outer loop.  On a start: the initial defect.  MK 0: Q1 bands B
     // (two rows per lane, 16-byte loads inside); MK 1: the ELL matrix E.
     //
-    // CB: the interior rows read the bands as value codes (one 64-bit word
-    // per row, band k in bits 4k .. 4k + 3) and look them up in ctab
-    // (16 per band, copied to LDS); the same values, the same sums.
+    // CB: the interior rows read the bands as codes and look the values up in a
+    // table copied to LDS; the same values, the same sums.  CB 1: row codes
+    // (one byte per row; ctab: the nine values of each of `rows` rows), 2:
+    // value codes (one 64-bit word per row, band k in bits 4k .. 4k + 3; ctab:
+    // 16 values per band).  Bound by HBM: measured on MI355X, one slot of
+    // 4097^2, value codes 91 us (32 bytes a node, 5.9 TB/s), row codes
+    // 84 us (25 bytes, 5.0 TB/s).
     //
     // KS: slots per workgroup.  The bands are 72 bytes a node where a slot's
     // vectors are 24, so with several slots one load of them serves KS (bands
     // without codes).  Bound by the L2: measured on MI355X, 64 slots of 513^2,
     // one slot a workgroup 172 us (9.4 TB/s of L2 and HBM together), four 133.
-    template <int MK, bool CB = false, int KS = 1>
+    template <int MK, int CB = 0, int KS = 1>
     __global__ __launch_bounds__(256) void outer_defect_kernel(k::Bands B, EllMat64 E, const Slot * T, int64_t n,
-            int64_t m, const uint64_t * __restrict__ codes, const double * __restrict__ ctab, int S)
+            int64_t m, const void * __restrict__ codes, const double * __restrict__ ctab, int rows, int S)
     {
-        static_assert(KS == 1 || (kBands<MK> && ! CB), "several slots: plain bands");
-        __shared__ double tab[CB ? 144 : 1];
-        if constexpr (CB)
-        {
-            if (threadIdx.x < 144)
-                tab[threadIdx.x] = ctab[threadIdx.x];
-            __syncthreads();
-        }
+        static_assert(KS == 1 || (kBands<MK> && CB == 0), "several slots: plain bands");
+        __shared__ double tab[CB == 1 ? 9 * kRowCodes : (CB == 2 ? 144 : 1)];
+        // (the table's first entries are on their way while the gate is read)
+        const int entries = CB == 1 ? 9 * rows : 144;
+        double entry = 0.0;
+        if (CB != 0)
+            entry = ctab[min((int)threadIdx.x, entries - 1)];
         const VB vb = vblock();
         bool on[KS], any = false;
         const double * b[KS];
@@ -261,6 +270,12 @@ namespace
         }
         if (! any)
             return;
+        if constexpr (CB != 0)
+        {
+            for (int i = threadIdx.x; i < entries; i += 256)
+                tab[i] = i < 256 ? entry : ctab[i];
+            __syncthreads();
+        }
         if (MK == 1)
         {
             // one row per lane and pass, lanes on consecutive rows
@@ -281,7 +296,7 @@ namespace
                 typedef k::Vec16<double>::type V2;
                 typedef double U2 __attribute__((ext_vector_type(2), aligned(8)));
                 V2 bv[9];
-                if constexpr (! CB)
+                if constexpr (CB == 0)
                     k::q1_bands_v<double>(B, i0, bv);
 #pragma unroll
                 for (int q = 0; q < KS; ++q)
@@ -290,12 +305,17 @@ namespace
                         continue;
                     const U2 bb = __builtin_nontemporal_load((const U2 *)(b[q] + i0));
                     double prod[2];
-                    if constexpr (CB)
+                    if constexpr (CB != 0)
                     {
                         // q1_sums_v's sums (Product<Q1>'s order: dd first) with
                         // the band values from the codes of rows i0, i0 + 1
                         typedef uint64_t C2 __attribute__((ext_vector_type(2)));
-                        const C2 cw = __builtin_nontemporal_load((const C2 *)(codes + i0));
+                        C2 cw = {0, 0};
+                        uint32_t rw = 0;
+                        if constexpr (CB == 1)
+                            rw = __builtin_nontemporal_load((const uint16_t *)((const uint8_t *)codes + i0));
+                        else
+                            cw = __builtin_nontemporal_load((const C2 *)((const uint64_t *)codes + i0));
                         double xm[4], xc[4], xp[4];
                         k::ld_window<4>(x[q] + i0 - m - 1, xm);
                         k::ld_window<4>(x[q] + i0 - 1, xc);
@@ -304,7 +324,10 @@ namespace
                         for (int v = 0; v < 2; ++v)
                         {
                             const uint64_t w = cw[v];
-                            auto bk = [&](int k) { return tab[16 * k + (int)((w >> (4 * k)) & 15u)]; };
+                            const double * row = tab + 9 * ((rw >> (8 * v)) & 255u);
+                            auto bk = [&](int k) {
+                                return CB == 1 ? row[k] : tab[16 * k + (int)((w >> (4 * k)) & 15u)];
+                            };
                             double sum = bk(4) * xc[v + 1];
                             sum += bk(0) * xm[v];
                             sum += bk(1) * xm[v + 1];
@@ -1428,8 +1451,10 @@ namespace
 // patterns) over the level's n nodes, node i's ten 4-bit indices go into one
 // 64-bit word and the values into a 16-entry table per array.  The one-pass
 // kernels then read 8 bytes per node instead of 40 and look the values up
-// in LDS: the same floats, so the same bits.  Levels whose arrays hold more
-// values keep the plain bands only.
+// in LDS: the same floats, so the same bits.  Where at most kRowCodes of the
+// words are distinct (Poisson rows: a handful) a node keeps one byte, the
+// index of its row among them.  Levels whose arrays hold more values keep the
+// plain bands only.  The FP64 bands of a finest level likewise.
 void hierarchy_codes(Hierarchy & h)
 {
     if (h.kind == 1)    // ELL matrices: no bands
@@ -1514,6 +1539,7 @@ void hierarchy_codes(Hierarchy & h)
     {
         h.codes64[L] = nullptr;
         h.ctab64[L] = nullptr;
+        h.rcode64[L] = nullptr;
         if (! h.bands64[L] || size_of(L) < 4225)
             continue;
         const uint64_t n = size_of(L);
@@ -1558,6 +1584,21 @@ void hierarchy_codes(Hierarchy & h)
         }
         if (! ok)
             continue;
+        std::vector<uint8_t> rc;
+        std::vector<uint64_t> words;
+        if (row_codes(code, rc, words))
+        {
+            std::vector<uint64_t> rows(9 * words.size());
+            for (size_t t = 0; t < words.size(); ++t)
+                for (int k = 0; k < 9; ++k)
+                    rows[9 * t + k] = tab[16 * k + ((words[t] >> (4 * k)) & 15u)];
+            h.rcode64[L] = (uint8_t *)h.alloc(n);
+            h.rtab64[L] = (double *)h.alloc(sizeof(double) * rows.size());
+            h.rows64[L] = (int)words.size();
+            HIP_CHECK(hipMemcpy(h.rcode64[L], rc.data(), n, hipMemcpyHostToDevice));
+            HIP_CHECK(hipMemcpy(h.rtab64[L], rows.data(), sizeof(double) * rows.size(), hipMemcpyHostToDevice));
+            continue;
+        }
         h.codes64[L] = (uint64_t *)h.alloc(sizeof(uint64_t) * n);
         h.ctab64[L] = (double *)h.alloc(sizeof(tab));
         HIP_CHECK(hipMemcpy(h.codes64[L], code.data(), sizeof(uint64_t) * n, hipMemcpyHostToDevice));
@@ -1957,21 +1998,23 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, u
         bool od_coded = false;
         if constexpr (MK == 0)
         {
-            if (h.use_codes && h.codes64[maxl])
-            {
-                hipLaunchKernelGGL((outer_defect_kernel<MK, true>), dim3(od_blocks, 1, S), blk, 0, st, h.B64(maxl),
-                                   h.ell64[maxl], T, n, top.side, (const uint64_t *)h.codes64[maxl],
-                                   (const double *)h.ctab64[maxl], (int)S);
+            auto go = [&](auto cb_tag, const void * codes, const double * tab) {
+                hipLaunchKernelGGL((outer_defect_kernel<MK, decltype(cb_tag)::value>), dim3(od_blocks, 1, S), blk, 0, st,
+                                   h.B64(maxl), h.ell64[maxl], T, n, top.side, codes, tab, h.rows64[maxl], (int)S);
                 od_coded = true;
-            }
+            };
+            if (h.use_codes && h.rcode64[maxl])
+                go(IntC<1>{}, h.rcode64[maxl], h.rtab64[maxl]);
+            else if (h.use_codes && h.codes64[maxl])
+                go(IntC<2>{}, h.codes64[maxl], h.ctab64[maxl]);
         }
         if (! od_coded)
         {
             auto go = [&](auto k_tag) {
                 constexpr int KS = decltype(k_tag)::value;
-                hipLaunchKernelGGL((outer_defect_kernel<MK, false, KS>), dim3(od_blocks, 1, (S + KS - 1) / KS), blk, 0, st,
+                hipLaunchKernelGGL((outer_defect_kernel<MK, 0, KS>), dim3(od_blocks, 1, (S + KS - 1) / KS), blk, 0, st,
                                    kBands<MK> ? h.B64(maxl) : k::Bands{}, h.ell64[maxl], T, n, top.side,
-                                   (const uint64_t *)nullptr, (const double *)nullptr, (int)S);
+                                   (const void *)nullptr, (const double *)nullptr, 0, (int)S);
             };
             if constexpr (kBands<MK>)
             {

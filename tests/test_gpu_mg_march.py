@@ -155,3 +155,26 @@ def test_outer_defect_of_several_slots_equals_single(hip, S):
         info = one.solve(bd[j], x)
         assert np.array_equal(x.get(), xd[j].get()), j
         assert (info["outer"], info["inner"]) == (infos[j]["outer"], infos[j]["inner"])
+
+
+@pytest.mark.parametrize("kind", ["rows", "layers", "values"])
+@pytest.mark.parametrize("level", [6, 7, 8])
+def test_coded_outer_defect_equals_bands(hip, level, kind):
+    """The FP64 outer defect from row codes, value codes and the bands themselves: four outer steps, so that the
+    defect of an iterate enters the next inner solve."""
+    g = np.random.default_rng(level)
+    n = P.side_of_level(level) ** 2
+    a32 = {L: _bands(kind, L, g) for L in range(MINL, level + 1)}
+    d32 = {L: dinv_reference(a32[L][4]) for L in a32}
+    A64 = [b.astype(np.float64) for b in a32[level]]
+    mg = hip.MGSolver(hip.mg_params(MINL, level, mask=MASKS[level], max_outer=4), A64, a32, d32)
+    b = hip.DeviceVector.from_numpy(g.uniform(-1, 1, n))
+    got = []
+    for codes in (True, False):
+        mg.set_value_codes(codes)
+        x = hip.DeviceVector.zeros(n)
+        info = mg.solve(b, x, raise_on_cap=False)
+        got.append((x.get(), info))
+    # (one of the matrices makes the iteration diverge, to the same NaN)
+    assert np.array_equal(list(got[0][1].values()), list(got[1][1].values()), equal_nan=True)
+    assert np.array_equal(got[0][0], got[1][0], equal_nan=True)
