@@ -230,10 +230,11 @@ namespace mg
     // stopping test.
     constexpr unsigned kTickOpen = 1, kTickCycle = 2;
 
-    // Enqueues one tick, or a half of one, for table entries [0, nslots) of
-    // finest level L.
-    void enqueue_tick(const Hierarchy & h, uint64_t L, const Slot * table, unsigned nslots, hipStream_t st,
-                      unsigned part = kTickOpen | kTickCycle);
+    // Enqueues one tick for table entries [0, nslots) of finest level L.
+    void enqueue_tick(const Hierarchy & h, uint64_t L, const Slot * table, unsigned nslots, hipStream_t st);
+    // The same, but only the halves in `part`.
+    void enqueue_tick_part(const Hierarchy & h, uint64_t L, const Slot * table, unsigned nslots, unsigned part,
+                           hipStream_t st);
     // Copies every slot's report into `reports` (device, nslots entries).
     void enqueue_report(const Slot * table, unsigned nslots, Report * reports, hipStream_t st);
     // b = U[-1, 1] from SplitMix64(seed, stream) with zero Dirichlet nodes

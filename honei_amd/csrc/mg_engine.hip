@@ -2282,7 +2282,12 @@ void tick_impl(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, u
 }
 }  // namespace
 
-void enqueue_tick(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, hipStream_t st, unsigned part)
+void enqueue_tick(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, hipStream_t st)
+{
+    enqueue_tick_part(h, maxl, T, S, kTickOpen | kTickCycle, st);
+}
+
+void enqueue_tick_part(const Hierarchy & h, uint64_t maxl, const Slot * T, unsigned S, unsigned part, hipStream_t st)
 {
     if (h.kind == 1)
         tick_impl<1>(h, maxl, T, S, part, st);

@@ -89,8 +89,8 @@ namespace
             for (uint64_t c = 0; c < chunk; ++c)
             {
                 if (! first)
-                    mg::enqueue_tick(mg->h, mg->max_level, mg->table, S, st, mg::kTickCycle);
-                mg::enqueue_tick(mg->h, mg->max_level, mg->table, S, st, mg::kTickOpen);
+                    mg::enqueue_tick_part(mg->h, mg->max_level, mg->table, S, mg::kTickCycle, st);
+                mg::enqueue_tick_part(mg->h, mg->max_level, mg->table, S, mg::kTickOpen, st);
                 first = false;
             }
             mg::enqueue_report(mg->table, S, mg->report, st);
