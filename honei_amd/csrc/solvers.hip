@@ -28,7 +28,7 @@ namespace
 {
     constexpr int kSolverBlocks = 2048;   // fixed grid of the fused reduction kernels
     constexpr int kMaxDevices = 64;
-    // Systems that may be solved in one cooperative launch (solvers_persist.hh):
+    // Systems that may be solved in one launch (solvers_persist.hh):
     // at most one row per thread of the fixed grid; their device scratch is
     // three sets, used in turn, of two partials per block, and a flag.
     constexpr uint64_t kPersistRows = 256 * (uint64_t)kSolverBlocks;

@@ -1,5 +1,5 @@
 // solvers_persist.hh -- CG, CGSolver<VAR> and ConjugateGradients<JAC> on small
-// systems in one cooperative launch.  Included by solvers.hip.
+// systems in one launch.  Included by solvers.hip.
 //
 // Systems whose vectors stay in cache are bound by latency: three to five
 // launches per iteration, each a few dependent memory round trips.  Measured
@@ -26,6 +26,13 @@
 // Waits are bounded: a workgroup that has polled kSpins times gives up, and
 // the host then solves by launches; results go to buffers of the solve's own
 // until every workgroup has finished.
+//
+// The launch is an ordinary one, of at most one workgroup per CU (checked to
+// fit), so that all of them are resident as soon as other streams' kernels
+// leave room; a lock keeps two such solves of a process from sharing a device.
+// A cooperative launch promises the same, but the queue that the runtime
+// opens for it stays: streams of the process that run side by side afterwards
+// (the request server's) took 10.7 ms instead of 8.5 ms for 48 mixed requests.
 #pragma once
 
     constexpr int kPersistThreads = 512;                      // two blocks of 256 rows side by side
@@ -455,8 +462,16 @@
         return PersistKernel();
     }
 
-    // Compute units of the current device when it can launch cooperatively,
-    // else 0 (cached per device).
+    // Compute units of the current device (cached per device; 0: none known),
+    // and the lock under which its one-launch solves run.
+    inline std::mutex & persist_lock()
+    {
+        static std::mutex mu[kMaxDevices];
+        int dev = 0;
+        HIP_CHECK(hipGetDevice(&dev));
+        return mu[dev >= 0 && dev < kMaxDevices ? dev : 0];
+    }
+
     inline unsigned persist_cus()
     {
         static std::mutex mu;
@@ -469,10 +484,9 @@
         std::lock_guard<std::mutex> lock(mu);
         if (! known[dev])
         {
-            int coop = 0, cu = 0;
-            HIP_CHECK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+            int cu = 0;
             HIP_CHECK(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev));
-            cus[dev] = coop ? cu : 0;
+            cus[dev] = cu;
             known[dev] = true;
         }
         return (unsigned)cus[dev];
@@ -497,13 +511,18 @@
         const PersistKernel kern = rpt ? persist_kernel<DT, KIND>(q1, width, rpt) : PersistKernel();
         if (! kern.fn)
             return PE_NOT;
+        const dim3 grid(grid_for(nb, 2 * rpt));
+        int fit = 0;
+        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kern.fn, kPersistThreads, kern.lds));
+        if (fit < 1 || grid.x > cus)
+            return PE_NOT;
+        std::lock_guard<std::mutex> lock(persist_lock());
         hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);
         PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0};
-        const dim3 grid(grid_for(nb, 2 * rpt));
         while (true)
         {
             void * args[] = {&ar};
-            if (hipLaunchCooperativeKernel(kern.fn, grid, dim3(kPersistThreads), args, (unsigned)kern.lds, st) != hipSuccess)
+            if (hipLaunchKernel(kern.fn, grid, dim3(kPersistThreads), args, kern.lds, st) != hipSuccess)
             {
                 (void)hipGetLastError();
                 return PE_GAVE_UP;
