@@ -920,12 +920,15 @@ namespace k
 
     // Grids up to this many rows go one row per lane: more wavefronts and a
     // shorter chain for a product that lasts a few microseconds.  Above, the
-    // 16-byte loads win.  Measured on MI355X, jacobi, one row per lane against
-    // the vector form, us: FP32 129^2 4.3 (6.5 with guarded loads in the vector
-    // form), 513^2 4.3 / 7.3, 1025^2 11.3 / 14.3, 2049^2 39.8 / 41.0, 2897^2
-    // 84.6 / 77.6, 4097^2 150 / 142; FP64 1025^2 19.6 / 21.9, 2049^2 69.5 /
-    // 73.3, 2897^2 145 / 151, 4097^2 322 / 270.
-    constexpr int64_t kQ1RowRows = 1 << 23;
+    // 16-byte loads win.  Measured on MI355X, one row per lane against the
+    // vector form, us: FP32 sweep 129^2 4.3 (6.5 with guarded loads in the
+    // vector form), 513^2 4.3 / 7.3, 1025^2 11.3 / 14.3, 2049^2 39.8 / 41.0,
+    // 2897^2 84.6 / 77.6, 4097^2 150 / 142; FP64 sweep 1025^2 19.6 / 21.9,
+    // 2049^2 69.1 / 73.3, 2561^2 108 / 118, 4097^2 322 / 270; FP64 defect 2049^2
+    // 67.2 / 69.2; FP64 product 1449^2 34.4 / 35.7, 2049^2 65.4 / 62.0, 2305^2
+    // 81.4 / 84.7, 2561^2 100.8 / 99.4, 4097^2 254 / 219.
+    template <typename DT, int MODE>
+    constexpr int64_t kQ1RowRows = sizeof(DT) == 8 && MODE == 0 ? 1 << 22 : 1 << 23;
 
     // Launches the vectorised Q1 kernel on a large grid whose streamed arrays
     // are all 16-byte aligned, else the one-row-per-lane form.  MODE as
@@ -937,7 +940,7 @@ namespace k
         bool vec = aligned16(y) && (MODE == 0 || aligned16(rhs)) && (MODE != 2 || aligned16(dinv));
         for (int k = 0; k < 9; ++k)
             vec = vec && aligned16(B.b[k]);
-        if (vec && n > kQ1RowRows)
+        if (vec && n > kQ1RowRows<DT, MODE>)
         {
             constexpr int V = Vec16<DT>::V;
             const uint64_t lanes = ((uint64_t)n + V - 1) / V;

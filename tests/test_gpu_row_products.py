@@ -143,3 +143,16 @@ def test_first_grid_of_the_wide_kernels(hip, form):
         for op in ("product", "defect", "jacobi"):
             call(hip, A, op, v, y)
             assert np.array_equal(y.get(), run(op, s, x, rhs, dinv)), (side, op)
+
+
+def test_first_grid_of_the_wide_fp64_product(hip):
+    """4,194,304 and 4,198,401 rows, the two sides of the FP64 product's line."""
+    for side in (2048, 2049):
+        bands, _, x, rhs, dinv = inputs(side, np.float64, 0, False)
+        s = row_sums(bands, [np.ones(side * side, bool)] * 9, x, side, Q1_ORDER)
+        A = hip.Q1Matrix(bands)
+        v = [hip.DeviceVector.from_numpy(q) for q in (x, rhs, dinv)]
+        y = hip.DeviceVector(side * side, np.float64)
+        for op in ("product", "defect", "jacobi"):
+            call(hip, A, op, v, y)
+            assert np.array_equal(y.get(), run(op, s, x, rhs, dinv)), (side, op)
