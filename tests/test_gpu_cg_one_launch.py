@@ -1,4 +1,4 @@
-"""Krylov solves in one cooperative launch against the same solves by
+"""Krylov solves in one launch against the same solves by
 launches, bit for bit.  An ELL matrix with two lanes per row takes the
 launches; with the same entries in the same order its row sums, and so its
 solves, are those of the one-lane form."""
