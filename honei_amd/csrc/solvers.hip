@@ -643,11 +643,13 @@ namespace
             if (converged_out)
                 *converged_out = h.converged;
         };
+        persist_path() = PP_LAUNCHES;
         start();
         if (width != 0)
         {
             const PersistEnd e = run_persist<DT, VAR ? PK_VAR : PK_NONE>(persist_matrix(A), is_q1(A), width, w, x, P,
                                                                          n, &h, st);
+            persist_path() = e == PE_DONE ? PP_ONE : (e == PE_GAVE_UP ? PP_GAVE_UP : PP_LAUNCHES);
             if (e == PE_DONE)
                 return finish();
             if (e == PE_GAVE_UP)
@@ -771,10 +773,12 @@ namespace
             if (converged_out)
                 *converged_out = h.converged;
         };
+        persist_path() = PP_LAUNCHES;
         start();
         if (width != 0)
         {
             const PersistEnd e = run_persist<DT, PK_JAC>(persist_matrix(A), is_q1(A), width, w, x, dd, n, &h, st);
+            persist_path() = e == PE_DONE ? PP_ONE : (e == PE_GAVE_UP ? PP_GAVE_UP : PP_LAUNCHES);
             if (e == PE_DONE)
                 return finish();
             if (e == PE_GAVE_UP)
@@ -926,6 +930,7 @@ namespace
     void run_pcg_pmat(const Op & A, hsolve_ell Pm, uint64_t n, const DT * b, DT * x, uint64_t max_iters, double eps,
                       uint64_t * used_iters, double * defect_out, hipStream_t st, int * converged_out)
     {
+        persist_path() = PP_LAUNCHES;
         CgWork<DT> w(n);
         DeviceArray<DT> zbuf(n);
         DT * z = zbuf.p;
@@ -1028,6 +1033,22 @@ namespace
 using namespace hsolve;
 
 extern "C" {
+
+int hsolve_krylov_path(int * path)
+{
+    HSOLVE_API_BEGIN
+    require(path != nullptr, HSOLVE_ERR_INVALID, "krylov_path: null pointer");
+    *path = persist_path();
+    HSOLVE_API_END
+}
+
+int hsolve_krylov_limits(uint64_t iterations, uint64_t give_up)
+{
+    HSOLVE_API_BEGIN
+    persist_limits().iters = iterations ? iterations : kPersistIters;
+    persist_limits().fail = give_up;
+    HSOLVE_API_END
+}
 
 int hsolve_cg_q1(int dtype, const void * const * bands, uint64_t size, const void * b, void * x, uint64_t max_iters,
                  double eps, uint64_t * used_iters, double * defect_out, void * stream)

@@ -40,6 +40,30 @@
     constexpr int kSpins = 1 << 21;
     constexpr uint64_t kPersistIters = 1 << 14;               // iterations per launch at most
 
+    // The calling thread's limits (hsolve_krylov_limits) and how its last
+    // solve ran (hsolve_krylov_path).
+    struct PersistLimits
+    {
+        uint64_t iters = kPersistIters;     // per launch
+        uint64_t fail = ~(uint64_t)0;       // the launch of a solve that is made to give up
+    };
+    inline PersistLimits & persist_limits()
+    {
+        static thread_local PersistLimits l;
+        return l;
+    }
+    enum PersistPath : int
+    {
+        PP_LAUNCHES = 0,
+        PP_ONE = 1,
+        PP_GAVE_UP = 2
+    };
+    inline int & persist_path()
+    {
+        static thread_local int path = PP_LAUNCHES;
+        return path;
+    }
+
     enum PersistKind : int
     {
         PK_NONE = 0,
@@ -70,6 +94,8 @@
         uint64_t * sums;       // kPersistSums, then the give-up flag
         CgScalars<DT> * s;
         int resume;            // the launch continues a solve (z and talpha are the last update's)
+        uint64_t iters;        // iterations of this launch at most
+        unsigned absent;       // a workgroup that stays away, so that the others give up (~0: none)
     };
 
     __global__ __launch_bounds__(256) void persist_clear_kernel(uint64_t * sums)
@@ -173,6 +199,8 @@
         const int tid = threadIdx.x, wave = tid >> 6, half = tid >> 8;
         const unsigned nb = ar.nb, blk0 = blockIdx.x * 2 * RPT;
         const int64_t n = ar.n;
+        if (blockIdx.x == ar.absent)
+            return;
         if (tid == 0)
             gave_up = 0;
 
@@ -205,7 +233,7 @@
                 pn[q][k] = load_at(ar.p, c[q][k]);
         }
         CgScalars<DT> s = *ar.s;
-        uint64_t left = kPersistIters;
+        uint64_t left = ar.iters;
         unsigned turn = 0;
         __syncthreads();
 
@@ -518,9 +546,11 @@
             return PE_NOT;
         std::lock_guard<std::mutex> lock(persist_lock());
         hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);
-        PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0};
-        while (true)
+        const PersistLimits lim = persist_limits();
+        PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0, lim.iters, ~0u};
+        for (uint64_t launch = 0;; ++launch)
         {
+            ar.absent = launch == lim.fail && grid.x > 1 ? grid.x - 1 : ~0u;
             void * args[] = {&ar};
             if (hipLaunchKernel(kern.fn, grid, dim3(kPersistThreads), args, kern.lds, st) != hipSuccess)
             {

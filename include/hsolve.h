@@ -398,6 +398,17 @@ int hsolve_cg_iters_ell(hsolve_ell m, const void *rhs, void *x, uint64_t max_ite
 int hsolve_pcg_jac_ell(hsolve_ell m, const void *dd_inverted, const void *b, void *x, uint64_t max_iters,
                        double eps, uint64_t *used_iters, double *defect_out, void *stream);
 
+/* How the calling thread's last Krylov solve on one right-hand side ran: 0 by
+ * launches, 1 in one launch (systems of up to 524,288 rows with short rows),
+ * 2 in one launch that gave up waiting and again by launches.  The same bits
+ * each way. */
+int hsolve_krylov_path(int *path);
+/* For tests: one-launch solves of the calling thread run at most `iterations`
+ * iterations per launch (0: the default), and in a solve's launch number
+ * give_up (from 0; UINT64_MAX: none) one workgroup of several stays away, so
+ * that the others give up waiting. */
+int hsolve_krylov_limits(uint64_t iterations, uint64_t give_up);
+
 /* ---------------- many right-hand sides on one ELL matrix -------------------
  * A column-blocked multivector of nrhs <= 64 columns stores row i's entries
  * at [i*nrhs, i*nrhs + nrhs) (device memory, the handle's value type).  The

@@ -1,0 +1,102 @@
+"""Which way a Krylov solve runs (one launch or launches), and one-launch
+solves that give up waiting, in their first launch and in a later one: the
+launches that follow give the bits of the one launch."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from honei_amd import problems as P
+from honei_amd._lib import lib, u64
+from test_gpu_cg_one_launch import _banded, _solve
+
+pytestmark = pytest.mark.gpu
+
+NEVER = (1 << 64) - 1
+LAUNCHES, ONE, GAVE_UP = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from honei_amd import device
+    return device
+
+
+@pytest.fixture(autouse=True)
+def _default_limits():
+    yield
+    assert lib().hsolve_krylov_limits(u64(0), u64(NEVER)) == 0
+
+
+def limits(iterations=0, give_up=NEVER):
+    assert lib().hsolve_krylov_limits(u64(iterations), u64(give_up)) == 0
+
+
+def path():
+    p = C.c_int(-1)
+    assert lib().hsolve_krylov_path(C.byref(p)) == 0
+    return p.value
+
+
+def same(a, b):
+    return a[0] == b[0] and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("kind", ["none", "var", "jac", "plain"])
+def test_path_taken(hip, kind):
+    """One launch for one lane per row and up to 524,288 rows of nine entries, 262,144 of ten to sixteen."""
+    wide = (1, 2, 3, 64, 65, 66, 900)                     # 15 entries
+    for n, offsets, want in ((1, (1,), ONE), (513, (1, 17), ONE), (70001, (1, 17), ONE), (524288, (1, 17), ONE),
+                             (524289, (1, 17), LAUNCHES), (262144, wide, ONE), (262145, wide, LAUNCHES),
+                             (70001, wide + (950,), LAUNCHES)):
+        (one, two), dinv = _banded(n, offsets, np.float64, 1)
+        b = np.ones(n)
+        _solve(hip, kind, hip.EllMatrix.from_dict(one), dinv, b, 3, 1e-12)
+        assert path() == want, (n, offsets)
+        _solve(hip, kind, hip.EllMatrix.from_dict(two), dinv, b, 3, 1e-12)
+        assert path() == LAUNCHES, (n, offsets)
+
+
+@pytest.mark.parametrize("kind", ["none", "var", "jac", "plain"])
+def test_first_launch_gives_up(hip, kind):
+    n = 70001
+    (one, two), dinv = _banded(n, (1, 17, 300), np.float64, 2)
+    b = np.random.default_rng(2).uniform(-1, 1, n)
+    M = hip.EllMatrix.from_dict(one)
+    ref = _solve(hip, kind, hip.EllMatrix.from_dict(two), dinv, b, 25, 1e-12)
+    limits(give_up=0)
+    assert same(_solve(hip, kind, M, dinv, b, 25, 1e-12), ref) and path() == GAVE_UP
+    limits()
+    assert same(_solve(hip, kind, M, dinv, b, 25, 1e-12), ref) and path() == ONE
+
+
+@pytest.mark.parametrize("kind", ["none", "jac"])
+def test_later_launch_gives_up(hip, kind):
+    """25 iterations in launches of ten: the second or third finds the workspace of the one before advanced."""
+    n = 3000
+    (one, two), dinv = _banded(n, (1, 54), np.float64, 3)
+    b = np.random.default_rng(3).uniform(-1, 1, n)
+    M = hip.EllMatrix.from_dict(one)
+    ref = _solve(hip, kind, hip.EllMatrix.from_dict(two), dinv, b, 25, 1e-12)
+    for give_up, want in ((1, GAVE_UP), (2, GAVE_UP), (3, ONE)):
+        limits(10, give_up)
+        assert same(_solve(hip, kind, M, dinv, b, 25, 1e-12), ref), give_up
+        assert path() == want
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("side", [23, 129, 363, 600, 724])
+def test_banded_one_launch_equals_launches(hip, side, dtype):
+    """One to four rows per thread on Q1 bands."""
+    n = side * side
+    A = hip.Q1Matrix([x.astype(dtype) for x in P.poisson_q1_bands(n)])
+    b = hip.DeviceVector.from_numpy(P.rhs_uniform(n).astype(dtype))
+
+    def solve():
+        x = hip.DeviceVector.zeros(n, dtype)
+        return hip.cg_q1(A, b, x, 30, 1e-30, raise_on_cap=False), x.get()
+
+    one = solve()
+    assert path() == ONE
+    limits(give_up=0)
+    assert same(solve(), one) and path() == GAVE_UP
