@@ -15,6 +15,7 @@
 #include "ell_handle.hh"
 #include "kernels_la.hh"
 
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -1047,6 +1048,8 @@ int hsolve_krylov_limits(uint64_t iterations, uint64_t give_up)
     HSOLVE_API_BEGIN
     persist_limits().iters = iterations ? iterations : kPersistIters;
     persist_limits().fail = give_up;
+    if (PersistDevice * dev = persist_device())
+        dev->pause = 0;
     HSOLVE_API_END
 }
 

@@ -25,7 +25,12 @@
 //
 // Waits are bounded: a workgroup that has polled kSpins times gives up, and
 // the host then solves by launches; results go to buffers of the solve's own
-// until every workgroup has finished.
+// until every workgroup has finished.  A poll takes about 0.12 us, so a wait ends
+// after 8 ms: several times what other streams' kernels hold a CU for and of the
+// order of one solve (a bound in polls, not by the clock: time in which the
+// process is switched off the device does not count, and no register is spent).
+// After a solve that gave up, the device's next kPersistPause go by launches at
+// once: where the CUs stay taken, giving up costs each a quarter of a millisecond.
 //
 // The launch is an ordinary one, of at most one workgroup per CU (checked to
 // fit), so that all of them are resident as soon as other streams' kernels
@@ -37,7 +42,8 @@
 
     constexpr int kPersistThreads = 512;                      // two blocks of 256 rows side by side
     constexpr uint64_t kNoSum = 0x7ff8dead0000beefull;
-    constexpr int kSpins = 1 << 21;
+    constexpr int kSpins = 1 << 16;                           // polls after which a wait is given up
+    constexpr int kPersistPause = 32;                         // solves by launches after one that gave up
     constexpr uint64_t kPersistIters = 1 << 14;               // iterations per launch at most
 
     // The calling thread's limits (hsolve_krylov_limits) and how its last
@@ -490,34 +496,39 @@
         return PersistKernel();
     }
 
-    // Compute units of the current device (cached per device; 0: none known),
-    // and the lock under which its one-launch solves run.
-    inline std::mutex & persist_lock()
+    // What one-launch solves keep per device.
+    struct PersistDevice
     {
-        static std::mutex mu[kMaxDevices];
-        int dev = 0;
-        HIP_CHECK(hipGetDevice(&dev));
-        return mu[dev >= 0 && dev < kMaxDevices ? dev : 0];
-    }
-
-    inline unsigned persist_cus()
+        unsigned cus = 0;              // compute units
+        std::mutex solve;              // held by a one-launch solve
+        std::atomic<int> pause{0};     // solves still to go by launches after one that gave up
+        bool paused()
+        {
+            int p = pause.load();
+            while (p > 0)
+                if (pause.compare_exchange_weak(p, p - 1))
+                    return true;
+            return false;
+        }
+    };
+    // of the current device (null: beyond kMaxDevices)
+    inline PersistDevice * persist_device()
     {
         static std::mutex mu;
-        static int cus[kMaxDevices];
-        static bool known[kMaxDevices];
+        static PersistDevice devices[kMaxDevices];
         int dev = 0;
         HIP_CHECK(hipGetDevice(&dev));
         if (dev < 0 || dev >= kMaxDevices)
-            return 0;
+            return nullptr;
+        PersistDevice & d = devices[dev];
         std::lock_guard<std::mutex> lock(mu);
-        if (! known[dev])
+        if (d.cus == 0)
         {
             int cu = 0;
             HIP_CHECK(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev));
-            cus[dev] = cu;
-            known[dev] = true;
+            d.cus = (unsigned)cu;
         }
-        return (unsigned)cus[dev];
+        return &d;
     }
 
     enum PersistEnd : int
@@ -534,17 +545,20 @@
     {
         if (n > kPersistRows || w.sums == nullptr)
             return PE_NOT;
-        const unsigned nb = grid_for(n, 256), cus = persist_cus();
-        const int rpt = persist_rows_per_thread(nb, cus);
+        PersistDevice * const dev = persist_device();
+        if (! dev)
+            return PE_NOT;
+        const unsigned nb = grid_for(n, 256);
+        const int rpt = persist_rows_per_thread(nb, dev->cus);
         const PersistKernel kern = rpt ? persist_kernel<DT, KIND>(q1, width, rpt) : PersistKernel();
         if (! kern.fn)
             return PE_NOT;
         const dim3 grid(grid_for(nb, 2 * rpt));
         int fit = 0;
         HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kern.fn, kPersistThreads, kern.lds));
-        if (fit < 1 || grid.x > cus)
+        if (fit < 1 || grid.x > dev->cus || dev->paused())
             return PE_NOT;
-        std::lock_guard<std::mutex> lock(persist_lock());
+        std::lock_guard<std::mutex> lock(dev->solve);
         hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);
         const PersistLimits lim = persist_limits();
         PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0, lim.iters, ~0u};
@@ -562,7 +576,10 @@
             HIP_CHECK(hipMemcpyAsync(&gave_up, w.sums + kPersistSums, sizeof(gave_up), hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
             if (gave_up)
+            {
+                dev->pause = kPersistPause;
                 return PE_GAVE_UP;
+            }
             if (h->run == 0)
                 break;
             hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);

@@ -406,7 +406,8 @@ int hsolve_krylov_path(int *path);
 /* For tests: one-launch solves of the calling thread run at most `iterations`
  * iterations per launch (0: the default), and in a solve's launch number
  * give_up (from 0; UINT64_MAX: none) one workgroup of several stays away, so
- * that the others give up waiting. */
+ * that the others give up waiting.  Also ends the pause that a solve which
+ * gave up puts in (the current device's next 32 solves go by launches). */
 int hsolve_krylov_limits(uint64_t iterations, uint64_t give_up);
 
 /* ---------------- many right-hand sides on one ELL matrix -------------------

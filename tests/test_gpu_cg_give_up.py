@@ -2,6 +2,7 @@
 solves that give up waiting, in their first launch and in a later one: the
 launches that follow give the bits of the one launch."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -100,3 +101,23 @@ def test_banded_one_launch_equals_launches(hip, side, dtype):
     assert path() == ONE
     limits(give_up=0)
     assert same(solve(), one) and path() == GAVE_UP
+
+
+@pytest.mark.parametrize("n", [513, 70001, 524288])
+def test_giving_up_takes_milliseconds_and_pauses(hip, n):
+    """A wait ends after about 8 ms, and the device's next 32 solves do not try."""
+    (one, two), dinv = _banded(n, (1, 17), np.float64, 4)
+    b = np.random.default_rng(4).uniform(-1, 1, n)
+    M = hip.EllMatrix.from_dict(one)
+    ref = _solve(hip, "none", hip.EllMatrix.from_dict(two), dinv, b, 25, 1e-12)
+    limits(give_up=0)
+    t = time.perf_counter()
+    assert same(_solve(hip, "none", M, dinv, b, 25, 1e-12), ref) and path() == GAVE_UP
+    assert time.perf_counter() - t < 0.1
+    for _ in range(32):
+        assert same(_solve(hip, "none", M, dinv, b, 25, 1e-12), ref) and path() == LAUNCHES
+    _solve(hip, "none", M, dinv, b, 25, 1e-12)
+    assert path() == GAVE_UP
+    limits()
+    _solve(hip, "none", M, dinv, b, 25, 1e-12)
+    assert path() == ONE
