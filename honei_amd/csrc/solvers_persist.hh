@@ -33,11 +33,12 @@
 // once: where the CUs stay taken, giving up costs each a quarter of a millisecond.
 //
 // The launch is an ordinary one, of at most one workgroup per CU (checked to
-// fit), so that all of them are resident as soon as other streams' kernels
-// leave room; a lock keeps two such solves of a process from sharing a device.
-// A cooperative launch promises the same, but the queue that the runtime
-// opens for it stays: streams of the process that run side by side afterwards
-// (the request server's) took 10.7 ms instead of 8.5 ms for 48 mixed requests.
+// fit), on streams without a CU mask, so that all of them are resident as soon
+// as other streams' kernels leave room; a lock keeps two such solves of a
+// process from sharing a device.  A cooperative launch promises the same, but
+// the queue that the runtime opens for it stays: streams of the process that
+// run side by side afterwards (the request server's) took 10.7 ms instead of
+// 8.5 ms for 48 mixed requests.
 #pragma once
 
     constexpr int kPersistThreads = 512;                      // two blocks of 256 rows side by side
@@ -531,6 +532,23 @@
         return &d;
     }
 
+    // Whether stream st may use every compute unit of the current device (of
+    // cus): a stream or a process with a CU mask cannot hold the grid at once.
+    inline bool persist_whole_device(hipStream_t st, unsigned cus)
+    {
+        constexpr unsigned W = 64;
+        uint32_t mask[W] = {};
+        if (cus > 32 * W || hipExtStreamGetCUMask(st, W, mask) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            return false;
+        }
+        unsigned on = 0;
+        for (unsigned w = 0; w < W; ++w)
+            on += (unsigned)__builtin_popcount(mask[w]);
+        return on >= cus;
+    }
+
     enum PersistEnd : int
     {
         PE_NOT = 0,      // the system does not qualify: nothing was touched
@@ -556,7 +574,7 @@
         const dim3 grid(grid_for(nb, 2 * rpt));
         int fit = 0;
         HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kern.fn, kPersistThreads, kern.lds));
-        if (fit < 1 || grid.x > dev->cus || dev->paused())
+        if (fit < 1 || grid.x > dev->cus || ! persist_whole_device(st, dev->cus) || dev->paused())
             return PE_NOT;
         std::lock_guard<std::mutex> lock(dev->solve);
         hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);
