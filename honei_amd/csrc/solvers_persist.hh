@@ -34,11 +34,12 @@
 //
 // The launch is an ordinary one, of at most one workgroup per CU (checked to
 // fit), on streams without a CU mask, so that all of them are resident as soon
-// as other streams' kernels leave room; a lock keeps two such solves of a
-// process from sharing a device.  A cooperative launch promises the same, but
-// the queue that the runtime opens for it stays: streams of the process that
-// run side by side afterwards (the request server's) took 10.7 ms instead of
-// 8.5 ms for 48 mixed requests.
+// as other streams' kernels leave room.  Solves of several threads run side by
+// side while there is a CU for each of their workgroups (PersistHold); one that
+// finds too few goes by launches.  A cooperative launch promises the same, but the
+// queue that the runtime opens for it stays: streams of the process that run
+// side by side afterwards (the request server's) took 10.7 ms instead of 8.5 ms
+// for 48 mixed requests.
 #pragma once
 
     constexpr int kPersistThreads = 512;                      // two blocks of 256 rows side by side
@@ -501,7 +502,7 @@
     struct PersistDevice
     {
         unsigned cus = 0;              // compute units
-        std::mutex solve;              // held by a one-launch solve
+        std::atomic<unsigned> held{0}; // workgroups per shader engine of the solves that run
         std::atomic<int> pause{0};     // solves still to go by launches after one that gave up
         bool paused()
         {
@@ -531,6 +532,28 @@
         }
         return &d;
     }
+
+    // A solve's workgroups among the device's CUs.  Consecutive workgroups go to
+    // its 32 shader engines in turn (8 XCDs of 4), so the CUs are counted in each.
+    constexpr unsigned kEngines = 32;
+    struct PersistHold
+    {
+        PersistDevice & d;
+        const unsigned share;
+        bool ok = false;
+        PersistHold(PersistDevice & dev, unsigned workgroups) : d(dev), share((workgroups + kEngines - 1) / kEngines)
+        {
+            unsigned h = d.held.load();
+            while (! ok && h + share <= d.cus / kEngines)
+                ok = d.held.compare_exchange_weak(h, h + share);
+        }
+        ~PersistHold()
+        {
+            if (ok)
+                d.held -= share;
+        }
+        PersistHold(const PersistHold &) = delete;
+    };
 
     // Whether stream st may use every compute unit of the current device (of
     // cus): a stream or a process with a CU mask cannot hold the grid at once.
@@ -574,9 +597,11 @@
         const dim3 grid(grid_for(nb, 2 * rpt));
         int fit = 0;
         HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kern.fn, kPersistThreads, kern.lds));
-        if (fit < 1 || grid.x > dev->cus || ! persist_whole_device(st, dev->cus) || dev->paused())
+        if (fit < 1 || ! persist_whole_device(st, dev->cus) || dev->paused())
             return PE_NOT;
-        std::lock_guard<std::mutex> lock(dev->solve);
+        const PersistHold hold(*dev, grid.x);
+        if (! hold.ok)
+            return PE_NOT;
         hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);
         const PersistLimits lim = persist_limits();
         PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0, lim.iters, ~0u};
