@@ -69,11 +69,19 @@ namespace
     // (ell_stencil_row), larger ones two (ell_spmv_r2).  One row per lane has
     // twice the wavefronts and a shorter chain, which is what a product of a
     // few microseconds needs; two need half the instructions per byte, which
-    // is what the memory rate needs.  Measured on MI355X, product, one row
-    // against two, us: FP32 257^2 4.3 / 5.9, 513^2 4.4 / 6.4, 1025^2 8.2 /
-    // 11.8, 2049^2 31.8 / 41.5, 2897^2 72.5 / 75.4; FP64 513^2 5.7 / 8.2,
-    // 1025^2 17.8 / 23.0, 2049^2 67.1 / 69.6, 2897^2 131.8 / 129.2.
-    constexpr uint64_t kStencilRowRows = 1 << 23;
+    // is what the memory rate needs.  Measured on MI355X, one row against two,
+    // us: FP32 product 257^2 4.3 / 5.9, 513^2 4.4 / 6.4, 1025^2 8.2 / 11.8,
+    // 2049^2 31.8 / 41.4, 2305^2 44.2 / 45.4, 2432^2 56.1 / 50.0, 2561^2 47.6 /
+    // 57.2, 2700^2 63.4 / 60.0, 2896^2 74.1 / 67.9, 3071^2 68.5 / 74.0, 4097^2
+    // 122 / 124; FP64 product 513^2 5.7 / 8.2, 1025^2 17.8 / 23.0, 2049^2 67.5 /
+    // 68.1, 2100^2 70.6 / 67.9, 2176^2 77.4 / 74.6, 2305^2 83.3 / 82.4, 2432^2
+    // 95.9 / 92.1, 2700^2 115.8 / 109.4, 2896^2 136.9 / 132.3, 4097^2 277 / 258;
+    // FP64 defect 2100^2 73.2 / 72.0, 2305^2 85.9 / 87.9, 2561^2 106.3 / 108.3,
+    // 2896^2 142.8 / 138.9, 3600^2 228 / 219.  (Sides next to a multiple of 128
+    // favour one row, even ones two, by up to 15%: between 2^22 and 2^23 rows
+    // neither wins throughout but for the FP64 product.)
+    template <typename DT, int MODE>
+    constexpr uint64_t kStencilRowRows = sizeof(DT) == 8 && MODE == 0 ? 4300000 : 1 << 23;
 
     // rows [r0, r1) (r0 even: the rows pair up as in the whole product)
     template <typename DT, typename IT, typename LT, int MODE, int K>
@@ -221,7 +229,7 @@ namespace
             // rows)
             if constexpr (sizeof(IT) == 2 && sizeof(LT) == 1)
                 if (m->q1_side != 0 && (v & HSOLVE_ELL_FULL) && (m->variant & HSOLVE_ELL_SET) == 0 && m->ncpr != 0 &&
-                    r1 - r0 <= kStencilRowRows)
+                    r1 - r0 <= kStencilRowRows<DT, MODE>)
                 {
                     hipLaunchKernelGGL((k::ell_stencil_row<DT, IT, LT, MODE>), dim3(grid_for(r1 - r0, 64)), dim3(64), 0,
                                        st, x, y, Aj, Ax, Arl, rhs, dinv, r0, r1, m->stride, (uint32_t)m->ncpr,

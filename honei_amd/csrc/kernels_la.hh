@@ -922,11 +922,17 @@ namespace k
     // shorter chain for a product that lasts a few microseconds.  Above, the
     // 16-byte loads win.  Measured on MI355X, one row per lane against the
     // vector form, us: FP32 sweep 129^2 4.3 (6.5 with guarded loads in the
-    // vector form), 513^2 4.3 / 7.3, 1025^2 11.3 / 14.3, 2049^2 39.8 / 41.0,
-    // 2897^2 84.6 / 77.6, 4097^2 150 / 142; FP64 sweep 1025^2 19.6 / 21.9,
-    // 2049^2 69.1 / 73.3, 2561^2 108 / 118, 4097^2 322 / 270; FP64 defect 2049^2
-    // 67.2 / 69.2; FP64 product 1449^2 34.4 / 35.7, 2049^2 65.4 / 62.0, 2305^2
-    // 81.4 / 84.7, 2561^2 100.8 / 99.4, 4097^2 254 / 219.
+    // vector form), 513^2 4.3 / 7.3, 1025^2 11.3 / 14.3, 2049^2 37.7 / 42.1,
+    // 2305^2 48.7 / 48.9, 2432^2 60.2 / 54.6, 2561^2 54.7 / 60.0, 2896^2 80.7 /
+    // 74.4, 4097^2 145 / 140; FP64 sweep 1025^2 19.6 / 21.9, 2049^2 68.0 / 73.9,
+    // 2561^2 106 / 119, 2896^2 144.5 / 151.5, 3300^2 202 / 189, 4097^2 316 / 275;
+    // FP64 defect 2049^2 66.3 / 67.5, 2561^2 102.4 / 111.7, 2896^2 138.5 / 140.9,
+    // 3600^2 217 / 204.  The FP64 product, which has the fewest vectors beside
+    // its bands, turns earlier: 1449^2 35.7 / 36.7, 1773^2 50.8 / 50.1, 2049^2
+    // 65.6 / 62.5, 2100^2 68.9 / 63.4, 2176^2 74.5 / 69.7, 2305^2 80.8 / 80.4,
+    // 2432^2 93.0 / 90.9, 2561^2 100.2 / 103.0, 2700^2 113.0 / 109.5, 2896^2 132.7 /
+    // 130.5, 3300^2 167 / 162, 4097^2 256 / 226.  (Sides next to a multiple of 128
+    // favour one row per lane, even ones the vector form.)
     template <typename DT, int MODE>
     constexpr int64_t kQ1RowRows = sizeof(DT) == 8 && MODE == 0 ? 1 << 22 : 1 << 23;
 
