@@ -113,8 +113,12 @@ class Q1Matrix:
         self.bands = [DeviceVector.from_numpy(b) for b in bands]
         self.ptrs = (vp * 9)(*[b.ptr for b in self.bands])
         self._bands = C.addressof(self.ptrs)
+        calls().set_vector_type(DeviceVector)
         self._product, self._defect, self._jacobi = (
             getattr(calls(), f"{stem}_{_sfx(self.dtype)}") for stem in ("product_bmdv_q1", "defect_q1", "jacobi_q1"))
+
+    def band_ptrs(self):
+        return [vp(b.ptr) for b in self.bands]
 
 
 def fill_poisson_q1(A: Q1Matrix, stream=None):
@@ -274,13 +278,13 @@ def copy_kernel(src: DeviceBuffer, dst: DeviceBuffer, nbytes: int, stream=None):
 
 # ----------------------------------------------------------------- ops
 def q1_product(A: Q1Matrix, x: DeviceVector, y: DeviceVector, stream=None):
-    rc = A._product(A._bands, x.ptr, y.ptr, A.size, A.root, stream)
+    rc = A._product(A.bands, x.ptr, y.ptr, A.size, A.root, stream)
     if rc:
         check(rc, "product_q1")
 
 
 def q1_defect(A: Q1Matrix, rhs: DeviceVector, x: DeviceVector, y: DeviceVector, stream=None):
-    rc = A._defect(rhs.ptr, A._bands, x.ptr, y.ptr, A.size, A.root, stream)
+    rc = A._defect(rhs.ptr, A.bands, x.ptr, y.ptr, A.size, A.root, stream)
     if rc:
         check(rc, "defect_q1")
 
