@@ -682,11 +682,13 @@ namespace
             initial = first ? sqrtf((float)r) : s->inner_initial;
             nrm = sqrtf((float)d);
             const float limit = initial * tol;
-            tie = nrm != 0.0f && count < n_max_iter && fabsf(nrm - limit) <= kTie * limit;
+            tie = nrm != 0.0f && fabsf(nrm - limit) <= kTie * limit;
             s->inner_initial = initial;
         }
-        __syncthreads();
-        if (tie)
+        // (the last cycle ends the solve whatever the test says)
+        if (count < n_max_iter)
+            __syncthreads();
+        if (count < n_max_iter && tie)
         {
             const gptr<const float> fd = as_global<const float>(sl.v[L][F_D]);
             const gptr<const float> fr = as_global<const float>(sl.v[L][F_RHS]);
