@@ -18,6 +18,7 @@ dbl = C.c_double
 flt = C.c_float
 
 _lib = None
+_calls_module = None
 
 
 class HsolveError(RuntimeError):
@@ -224,10 +225,17 @@ def lib():
 
 
 def calls():
-    """The entry points of the shortest calls without ctypes (csrc/pycalls.c)."""
-    lib()
-    from . import _calls
-    return _calls
+    """The entry points of the shortest calls: the CPython module (csrc/pycalls.c), or the same through ctypes where
+    this interpreter has none."""
+    global _calls_module
+    if _calls_module is None:
+        lib()
+        try:
+            from . import _calls as m
+        except ImportError:
+            from . import _calls_ctypes as m
+        _calls_module = m
+    return _calls_module
 
 
 def check(code, what=""):
