@@ -721,14 +721,16 @@ namespace k
     // at its absent entries: a zero entry adds +-0 to a sum that is never
     // -0, so with finite x the result is the ELL product's, bit for bit.
     // x: a pointer, or any value whose x[j] yields the j-th entry
-    template <typename DT, int ORD = 0, typename XV>
+    //
+    // A neighbour outside [0, n) is replaced by the node itself and its
+    // product is not added, so that no branch separates the 18 loads: under
+    // guards each one is a round trip of its own, and the first and last m
+    // rows are the last to finish on a small grid.  GUARD: under guards all
+    // the same, in fewer registers (the FP64 CG of large systems).
+    template <typename DT, int ORD = 0, bool GUARD = false, typename XV>
     __device__ __forceinline__ DT q1_row(const Bands & B, const XV & x, int64_t i, int64_t n, int64_t m)
     {
         const DT * const * b = reinterpret_cast<const DT * const *>(B.b);
-        // A neighbour outside [0, n) is replaced by the node itself and its
-        // product is not added, so that no branch separates the 18 loads:
-        // under guards each one is a round trip of its own, and the first
-        // and last m rows are the last to finish on a small grid.
         DT s = ORD == 1 ? DT(0) : ld_stream(b[4] + i) * x[i];
 #pragma unroll
         for (int k = 0; k < 9; ++k)
@@ -741,6 +743,12 @@ namespace k
                 continue;
             }
             const bool in = k < 4 ? j >= 0 : j < n;
+            if (GUARD)
+            {
+                if (in)
+                    s += ld_stream(b[k] + i) * x[j];
+                continue;
+            }
             const DT t = ld_stream(b[k] + i) * x[in ? j : i];
             s = in ? s + t : s;
         }

@@ -38,15 +38,22 @@ namespace
 
     // --------------------------------------------------------------- operators
     // A row of y = A x for the fused kernels.
-    template <typename DT> struct Q1Op
+    template <typename DT, bool GUARD = false> struct Q1Op
     {
         k::Bands B;
         int64_t n, m;
         template <typename XV> __device__ __forceinline__ DT row(const XV & x, int64_t i) const
         {
-            return k::q1_row<DT>(B, x, i, n, m);
+            return k::q1_row<DT, 0, GUARD>(B, x, i, n, m);
         }
     };
+    // FP64 systems above this many rows take the guarded rows: their kernels
+    // are bound by memory, and waves in flight count for more than a short
+    // chain.  Measured on MI355X, us an iteration of CG, without guards and
+    // with: 733^2 33.0 / 36.3, 1025^2 43.5 / 44.6, 1449^2 74.9 / 72.8, 2049^2 137.2
+    // / 129.5, 4097^2 542 / 525 (FP32 29.8 / 34.2, 72.4 / 82.6 and 243 / 279 at
+    // 1025^2, 2049^2 and 4097^2).
+    constexpr uint64_t kGuardRows = 3 << 19;
 
     template <typename DT, typename IT, typename LT> using EllOp = EllRowOp<DT, IT, LT>;
 
@@ -588,7 +595,7 @@ namespace
 
 #include "solvers_persist.hh"
 
-    template <typename DT> PersistMatrix persist_matrix(const Q1Op<DT> & A)
+    template <typename DT, bool GUARD> PersistMatrix persist_matrix(const Q1Op<DT, GUARD> & A)
     {
         PersistMatrix m{};
         m.B = A.B;
@@ -606,7 +613,7 @@ namespace
         m.stride = A.stride;
         return m;
     }
-    template <typename DT> constexpr bool is_q1(const Q1Op<DT> &) { return true; }
+    template <typename DT, bool GUARD> constexpr bool is_q1(const Q1Op<DT, GUARD> &) { return true; }
     template <typename DT, typename IT, typename LT> constexpr bool is_q1(const EllOp<DT, IT, LT> &) { return false; }
 
     // width: the longest row of an ELL matrix with one lane per row (0: the
@@ -1064,9 +1071,15 @@ int hsolve_cg_q1(int dtype, const void * const * bands, uint64_t size, const voi
     int conv = 0;
     if (dtype)
     {
-        Q1Op<double> A{bands9(bands), (int64_t)size, m};
-        run_cg<double, Q1Op<double>, false>(A, size, (const double *)b, (double *)x, nullptr, max_iters, eps,
-                                            used_iters, defect_out, st, &conv, 9);
+        auto run = [&](auto guard) {
+            using Op = Q1Op<double, decltype(guard)::value>;
+            run_cg<double, Op, false>(Op{bands9(bands), (int64_t)size, m}, size, (const double *)b, (double *)x,
+                                      nullptr, max_iters, eps, used_iters, defect_out, st, &conv, 9);
+        };
+        if (size > kGuardRows)
+            run(std::true_type{});
+        else
+            run(std::false_type{});
     }
     else
     {
