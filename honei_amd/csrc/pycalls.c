@@ -4,7 +4,7 @@
  * and sizes of its hsolve.h counterpart as integers (None is a null pointer)
  * and returns the status.  Measured, host time of one banded sweep without
  * the launch: 2.25 us through ctypes with an object for each argument, 0.53 us
- * here (a product or defect, which reads nine bands' pointers, 0.3 us more);
+ * here (a product or defect, which reads nine bands' pointers, 0.2 us more);
  * the launch itself takes 2.75 us. */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -28,16 +28,26 @@ static int integer(PyObject * o, uint64_t * a)
     return 1;
 }
 
-/* b.ptr; of a vector_type, whose ptr is a property, without the frame for it */
+/* o.name from o's own dictionary (borrowed), or NULL where it is not there */
+static PyObject * own(PyObject * o, PyObject * name)
+{
+    PyObject * d = PyObject_GenericGetDict(o, NULL);
+    PyObject * v = d != NULL ? PyDict_GetItemWithError(d, name) : NULL;
+    Py_XDECREF(d);
+    if (v == NULL)
+        PyErr_Clear();
+    return v;
+}
+
+/* b.ptr (a new reference); of a vector_type, whose ptr is a property that
+ * gives buf.ptr, without the frame for it */
 static PyObject * pointer_of(PyObject * b)
 {
-    if (Py_TYPE(b) != vector_type)
+    PyObject * buf = Py_TYPE(b) == vector_type ? own(b, buf_name) : NULL;
+    PyObject * p = buf != NULL ? own(buf, ptr_name) : NULL;
+    if (p == NULL)
         return PyObject_GetAttr(b, ptr_name);
-    PyObject * buf = PyObject_GetAttr(b, buf_name);
-    if (buf == NULL)
-        return NULL;
-    PyObject * p = PyObject_GetAttr(buf, ptr_name);
-    Py_DECREF(buf);
+    Py_INCREF(p);
     return p;
 }
 
