@@ -69,17 +69,16 @@ namespace
     // (ell_stencil_row), larger ones two (ell_spmv_r2).  One row per lane has
     // twice the wavefronts and a shorter chain, which is what a product of a
     // few microseconds needs; two need half the instructions per byte, which
-    // is what the memory rate needs.  Measured on MI355X, one row against two,
-    // us: FP32 product 257^2 4.3 / 5.9, 513^2 4.4 / 6.4, 1025^2 8.2 / 11.8,
-    // 2049^2 31.8 / 41.4, 2305^2 44.2 / 45.4, 2432^2 56.1 / 50.0, 2561^2 47.6 /
-    // 57.2, 2700^2 63.4 / 60.0, 2896^2 74.1 / 67.9, 3071^2 68.5 / 74.0, 4097^2
-    // 122 / 124; FP64 product 513^2 5.7 / 8.2, 1025^2 17.8 / 23.0, 2049^2 67.5 /
-    // 68.1, 2100^2 70.6 / 67.9, 2176^2 77.4 / 74.6, 2305^2 83.3 / 82.4, 2432^2
-    // 95.9 / 92.1, 2700^2 115.8 / 109.4, 2896^2 136.9 / 132.3, 4097^2 277 / 258;
-    // FP64 defect 2100^2 73.2 / 72.0, 2305^2 85.9 / 87.9, 2561^2 106.3 / 108.3,
-    // 2896^2 142.8 / 138.9, 3600^2 228 / 219.  (Sides next to a multiple of 128
-    // favour one row, even ones two, by up to 15%: between 2^22 and 2^23 rows
-    // neither wins throughout but for the FP64 product.)
+    // is what the memory rate needs.  Measured on MI355X in turn on three sets
+    // of arrays, one row against two, us: FP32 product 257^2 4.3 / 5.9, 513^2 4.4 /
+    // 6.4, 1025^2 8.2 / 11.8, 2049^2 32.3 / 41.3, 2176^2 45.7 / 41.0, 2305^2 44.7 /
+    // 46.4, 2432^2 56.3 / 50.1, 2561^2 48.1 / 58.0, 2700^2 63.4 / 60.2, 2896^2 74.1 /
+    // 68.4, 3071^2 67.9 / 77.0, 3300^2 87.5 / 92.9; FP64 product 513^2 5.7 / 8.2,
+    // 1025^2 17.8 / 23.0, 1773^2 51.5 / 53.0, 2049^2 67.5 / 69.6, 2100^2 73.1 / 67.7,
+    // 2305^2 87.0 / 84.6, 2561^2 112.4 / 108.9, 2896^2 143.4 / 138.6; FP64 defect 1773^2
+    // 53.4 / 55.7, 2049^2 77.1 / 75.4, 2561^2 122.3 / 118.6, 2896^2 154.1 / 149.0.
+    // (FP32 sides that are a multiple of 128, whose slots lie a multiple of 64 KB
+    // apart, favour two rows between 2^22 and 2^23 rows, the others one.)
     template <typename DT, int MODE>
     constexpr uint64_t kStencilRowRows = sizeof(DT) == 8 && MODE == 0 ? 4300000 : 1 << 23;
 

@@ -760,16 +760,18 @@ namespace k
 
     // mode 0: y = A x; mode 1: y = rhs - A x;
     // mode 2: y = x + (rhs - A x) * dinv (one Jacobi sweep into y)
-    template <typename DT, int MODE>
-    __global__ __launch_bounds__(kQ1Block) void q1_kernel(Bands B, const DT * __restrict__ x,
+    // BLOCK 256: for large grids whose arrays are not 16-byte aligned, where
+    // FP64 rows go under guards.
+    template <typename DT, int MODE, int BLOCK>
+    __global__ __launch_bounds__(BLOCK) void q1_kernel(Bands B, const DT * __restrict__ x,
             DT * __restrict__ y, const DT * __restrict__ rhs, const DT * __restrict__ dinv,
             int64_t n, int64_t m)
     {
         // a lane past the end repeats the last row: no branch stands between
         // the launch and the loads
-        const int64_t r = (int64_t)blockIdx.x * kQ1Block + threadIdx.x;
+        const int64_t r = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
         const int64_t i = r < n ? r : n - 1;
-        DT o = q1_row<DT>(B, x, i, n, m);
+        DT o = q1_row<DT, 0, BLOCK == 256 && sizeof(DT) == 8>(B, x, i, n, m);
         if (MODE == 1)
             o = rhs[i] - o;
         else if (MODE == 2)
@@ -928,21 +930,21 @@ namespace k
 
     // Grids up to this many rows go one row per lane: more wavefronts and a
     // shorter chain for a product that lasts a few microseconds.  Above, the
-    // 16-byte loads win.  Measured on MI355X, one row per lane against the
-    // vector form, us: FP32 sweep 129^2 4.3 (6.5 with guarded loads in the
-    // vector form), 513^2 4.3 / 7.3, 1025^2 11.3 / 14.3, 2049^2 37.7 / 42.1,
-    // 2305^2 48.7 / 48.9, 2432^2 60.2 / 54.6, 2561^2 54.7 / 60.0, 2896^2 80.7 /
-    // 74.4, 4097^2 145 / 140; FP64 sweep 1025^2 19.6 / 21.9, 2049^2 68.0 / 73.9,
-    // 2561^2 106 / 119, 2896^2 144.5 / 151.5, 3300^2 202 / 189, 4097^2 316 / 275;
-    // FP64 defect 2049^2 66.3 / 67.5, 2561^2 102.4 / 111.7, 2896^2 138.5 / 140.9,
-    // 3600^2 217 / 204.  The FP64 product, which has the fewest vectors beside
-    // its bands, turns earlier: 1449^2 35.7 / 36.7, 1773^2 50.8 / 50.1, 2049^2
-    // 65.6 / 62.5, 2100^2 68.9 / 63.4, 2176^2 74.5 / 69.7, 2305^2 80.8 / 80.4,
-    // 2432^2 93.0 / 90.9, 2561^2 100.2 / 103.0, 2700^2 113.0 / 109.5, 2896^2 132.7 /
-    // 130.5, 3300^2 167 / 162, 4097^2 256 / 226.  (Sides next to a multiple of 128
-    // favour one row per lane, even ones the vector form.)
-    template <typename DT, int MODE>
-    constexpr int64_t kQ1RowRows = sizeof(DT) == 8 && MODE == 0 ? 1 << 22 : 1 << 23;
+    // 16-byte loads win.  The line lies where a call's arrays outgrow the 256 MB
+    // cache in front of HBM, or half of it (FP32).  Measured on MI355X in turn on
+    // three sets of arrays, one row per lane against the vector form, us: FP64
+    // product 1773^2 51.2 / 51.1, 1900^2 58.8 / 54.7, 2100^2 70.3 / 63.9, 2305^2 85.4
+    // / 81.4, 2896^2 140.5 / 136.0; FP64 defect 1773^2 52.1 / 54.2, 1900^2 61.7 /
+    // 58.6, 2100^2 76.8 / 69.4, 2561^2 118.3 / 112.6; FP64 sweep 1600^2 44.4 / 47.5,
+    // 1773^2 57.6 / 58.4, 1900^2 68.7 / 62.9, 2049^2 83.5 / 75.3, 2100^2 87.0 / 74.7,
+    // 2896^2 161.8 / 156.0.  FP32 sweep 129^2 4.3 (6.5 with guarded loads in the
+    // vector form), 513^2 4.3 / 7.3, 1025^2 11.3 / 14.3, 2049^2 35.4 / 41.5, 2100^2 38.4
+    // / 42.0, 2176^2 49.0 / 44.6, 2305^2 48.4 / 49.4, 2432^2 60.9 / 55.2, 2561^2 62.5 /
+    // 60.5, 2896^2 86.3 / 74.4; FP32 product 2100^2 36.3 / 37.0, 2176^2 44.6 / 39.2,
+    // 2400^2 54.7 / 47.0, 2500^2 50.0 / 51.9, 2700^2 62.9 / 57.7, 2896^2 73.8 / 65.6.
+    // (On one set of arrays over and over, part of which the cache keeps, FP64
+    // sweeps of 1951^2 to 2800^2 are up to 9% faster one row per lane.)
+    template <typename DT> constexpr int64_t kQ1RowRows = sizeof(DT) == 8 ? 3400000 : 4500000;
 
     // Launches the vectorised Q1 kernel on a large grid whose streamed arrays
     // are all 16-byte aligned, else the one-row-per-lane form.  MODE as
@@ -954,16 +956,22 @@ namespace k
         bool vec = aligned16(y) && (MODE == 0 || aligned16(rhs)) && (MODE != 2 || aligned16(dinv));
         for (int k = 0; k < 9; ++k)
             vec = vec && aligned16(B.b[k]);
-        if (vec && n > kQ1RowRows<DT, MODE>)
+        auto rows = [&](auto block) {
+            constexpr int BLOCK = decltype(block)::value;
+            hipLaunchKernelGGL((q1_kernel<DT, MODE, BLOCK>), dim3(grid_for((uint64_t)n, BLOCK)), dim3(BLOCK), 0, st, B,
+                               x, y, rhs, dinv, n, m);
+        };
+        if (n <= kQ1RowRows<DT>)
+            rows(std::integral_constant<int, kQ1Block>{});
+        else if (! vec)
+            rows(std::integral_constant<int, 256>{});
+        else
         {
             constexpr int V = Vec16<DT>::V;
             const uint64_t lanes = ((uint64_t)n + V - 1) / V;
             hipLaunchKernelGGL((q1_kernel_v<DT, MODE>), dim3(grid_for(lanes, 256)), dim3(256), 0, st, B, x, y, rhs,
                                dinv, n, m);
         }
-        else
-            hipLaunchKernelGGL((q1_kernel<DT, MODE>), dim3(grid_for((uint64_t)n, kQ1Block)), dim3(kQ1Block), 0, st, B, x,
-                               y, rhs, dinv, n, m);
     }
 
     // ------------------------------------------------------------ reductions
