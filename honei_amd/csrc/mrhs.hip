@@ -991,7 +991,15 @@ namespace
         // window; other matrices would gather both for every entry)
         const size_t rest = pb + sizeof(MState<DT>) + 256;
         void * block = nullptr;
-        bool fused = K < 0;
+        // FP32 with a preconditioner: on small multivectors the fused step's
+        // longer chain costs more than the vectors it saves.  Measured on MI355X,
+        // us an iteration, fused and separate: 65^2 64 columns 70.8 / 67.0, 161^2
+        // 80.9 / 73.1, 193^2 82.6 / 83.6, 257^2 90.1 / 97.8; 16 columns 65^2 72.5 / 70.5,
+        // 321^2 87.7 / 82.7, 513^2 123.0 / 123.4; 2 columns 513^2 116.6 / 111.4.  (Without
+        // one 65.5 / 66.3, 75.5 / 72.4, 77.3 / 82.3; FP64 71.5 / 79.1, 86.5 / 95.2, 90.4 /
+        // 99.8.)
+        const bool small = sizeof(DT) == 4 && VAR && n * R < (uint64_t)1 << 21;
+        bool fused = K < 0 && ! small;
         if (fused && hipMalloc(&block, 4 * vb + rest) != hipSuccess)
         {
             (void)hipGetLastError();
