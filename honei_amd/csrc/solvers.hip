@@ -18,6 +18,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -34,7 +35,8 @@ namespace
     // three sets, used in turn, of two partials per block, and a flag.
     constexpr uint64_t kPersistRows = 256 * (uint64_t)kSolverBlocks;
     constexpr size_t kPersistSums = 3 * 2 * kSolverBlocks;
-    constexpr size_t kPersistBytes = sizeof(uint64_t) * (kPersistSums + 8);
+    constexpr size_t kPersistFlags = 8;
+    constexpr size_t kPersistBytes = sizeof(uint64_t) * (kPersistSums + kPersistFlags);
 
     // --------------------------------------------------------------- operators
     // A row of y = A x for the fused kernels.

@@ -111,8 +111,20 @@
         const unsigned i = blockIdx.x * 256 + threadIdx.x;
         if (i < kPersistSums)
             sums[i] = kNoSum;
-        else if (i < kPersistSums + 8)
+        else if (i < kPersistSums + kPersistFlags)
             sums[i] = 0;
+    }
+
+    // The iterate of a solve that has ended, and in which no workgroup gave up,
+    // to the caller's array.
+    template <typename DT>
+    __global__ __launch_bounds__(256) void persist_copy_kernel(const DT * __restrict__ from, DT * __restrict__ to,
+            int64_t n, const uint64_t * sums, const CgScalars<DT> * s)
+    {
+        if (s->run != 0 || sums[kPersistSums] != 0)
+            return;
+        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+            to[i] = from[i];
     }
 
     template <typename T> __device__ __forceinline__ T load_device(const T * p)
@@ -467,14 +479,7 @@
         PersistKernel p;
         p.fn = (const void *)persist_cg_kernel<DT, KIND, Q1, K, RPT>;
         if (kEntriesInLds<DT, K, RPT>)
-        {
             p.lds = sizeof(DT) * K * RPT * kPersistThreads;
-            if (hipFuncSetAttribute(p.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) != hipSuccess)
-            {
-                (void)hipGetLastError();
-                p.fn = nullptr;
-            }
-        }
         return p;
     }
 
@@ -504,6 +509,25 @@
         unsigned cus = 0;              // compute units
         std::atomic<unsigned> held{0}; // workgroups per shader engine of the solves that run
         std::atomic<int> pause{0};     // solves still to go by launches after one that gave up
+        std::mutex mu;
+        std::map<const void *, bool> fits;
+        // whether a workgroup of kernel k fits a CU (looked up once)
+        bool fit(const PersistKernel & k)
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            auto it = fits.find(k.fn);
+            if (it != fits.end())
+                return it->second;
+            int n = 0;
+            const bool ok =
+                (k.lds == 0 || hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds) ==
+                                   hipSuccess) &&
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k.fn, kPersistThreads, k.lds) == hipSuccess && n > 0;
+            if (! ok)
+                (void)hipGetLastError();
+            fits.emplace(k.fn, ok);
+            return ok;
+        }
         bool paused()
         {
             int p = pause.load();
@@ -584,7 +608,9 @@
     PersistEnd run_persist(const PersistMatrix & A, bool q1, uint64_t width, const Work & w, DT * x, const DT * P, uint64_t n,
                      CgScalars<DT> * h, hipStream_t st)
     {
-        if (n > kPersistRows || w.sums == nullptr)
+        // (one iteration by launches is over before the one launch has read its
+        // rows: 129^2 Jacobi-PCG 44 us against 51, three iterations 82 against 64)
+        if (n > kPersistRows || w.sums == nullptr || h->max_iters < 2)
             return PE_NOT;
         PersistDevice * const dev = persist_device();
         if (! dev)
@@ -595,14 +621,12 @@
         if (! kern.fn)
             return PE_NOT;
         const dim3 grid(grid_for(nb, 2 * rpt));
-        int fit = 0;
-        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kern.fn, kPersistThreads, kern.lds));
-        if (fit < 1 || ! persist_whole_device(st, dev->cus) || dev->paused())
+        if (! dev->fit(kern) || ! persist_whole_device(st, dev->cus) || dev->paused())
             return PE_NOT;
         const PersistHold hold(*dev, grid.x);
         if (! hold.ok)
             return PE_NOT;
-        hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);
+        hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + kPersistFlags, 256)), dim3(256), 0, st, w.sums);
         const PersistLimits lim = persist_limits();
         PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0, lim.iters, ~0u};
         for (uint64_t launch = 0;; ++launch)
@@ -614,22 +638,28 @@
                 (void)hipGetLastError();
                 return PE_GAVE_UP;
             }
-            uint64_t gave_up = 0;
-            HIP_CHECK(hipMemcpyAsync(h, w.s, sizeof(*h), hipMemcpyDeviceToHost, st));
-            HIP_CHECK(hipMemcpyAsync(&gave_up, w.sums + kPersistSums, sizeof(gave_up), hipMemcpyDeviceToHost, st));
+            hipLaunchKernelGGL((persist_copy_kernel<DT>), dim3(std::min<unsigned>(grid_for(n, 1024), 256)), dim3(256), 0,
+                               st, (const DT *)w.p2, x, (int64_t)n, (const uint64_t *)w.sums, (const CgScalars<DT> *)w.s);
+            // the give-up flag and the scalars behind it
+            struct
+            {
+                uint64_t gave_up[kPersistFlags];
+                CgScalars<DT> s;
+            } end;
+            static_assert(sizeof(end) == sizeof(end.gave_up) + sizeof(end.s), "laid out as CgWork lays them out");
+            HIP_CHECK(hipMemcpyAsync(&end, w.sums + kPersistSums, sizeof(end), hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
-            if (gave_up)
+            if (end.gave_up[0])
             {
                 dev->pause = kPersistPause;
                 return PE_GAVE_UP;
             }
+            *h = end.s;
             if (h->run == 0)
-                break;
-            hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + 8, 256)), dim3(256), 0, st, w.sums);
+                return PE_DONE;
+            hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + kPersistFlags, 256)), dim3(256), 0, st,
+                               w.sums);
             ar.x = w.p2;
             ar.resume = 1;
         }
-        HIP_CHECK(hipMemcpyAsync(x, w.p2, sizeof(DT) * n, hipMemcpyDeviceToDevice, st));
-        HIP_CHECK(hipStreamSynchronize(st));
-        return PE_DONE;
     }
