@@ -1052,11 +1052,10 @@ int hsolve_krylov_path(int * path)
     HSOLVE_API_END
 }
 
-int hsolve_krylov_limits(uint64_t iterations, uint64_t give_up)
+int hsolve_krylov_give_up(uint64_t launch)
 {
     HSOLVE_API_BEGIN
-    persist_limits().iters = iterations ? iterations : kPersistIters;
-    persist_limits().fail = give_up;
+    persist_fail() = launch;
     if (PersistDevice * dev = persist_device())
         dev->pause = 0;
     HSOLVE_API_END

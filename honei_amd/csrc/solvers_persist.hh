@@ -26,11 +26,13 @@
 // Waits are bounded: a workgroup that has polled kSpins times gives up, and
 // the host then solves by launches; results go to buffers of the solve's own
 // until every workgroup has finished.  A poll takes about 0.12 us, so a wait ends
-// after 8 ms: several times what other streams' kernels hold a CU for and of the
+// after 10 ms: several times what other streams' kernels hold a CU for and of the
 // order of one solve (a bound in polls, not by the clock: time in which the
-// process is switched off the device does not count, and no register is spent).
+// process is switched off the device does not count, and no register is spent; a
+// bound of 16 bits shortens the loop's code by four bytes, which moved it within
+// the fetch lines and made 513^2 Jacobi-PCG 5% slower).
 // After a solve that gave up, the device's next kPersistPause go by launches at
-// once: where the CUs stay taken, giving up costs each a quarter of a millisecond.
+// once: where the CUs stay taken, giving up costs each a third of a millisecond.
 //
 // The launch is an ordinary one, of at most one workgroup per CU (checked to
 // fit), on streams without a CU mask, so that all of them are resident as soon
@@ -44,21 +46,16 @@
 
     constexpr int kPersistThreads = 512;                      // two blocks of 256 rows side by side
     constexpr uint64_t kNoSum = 0x7ff8dead0000beefull;
-    constexpr int kSpins = 1 << 16;                           // polls after which a wait is given up
+    constexpr int kSpins = 80000;                             // polls after which a wait is given up
     constexpr int kPersistPause = 32;                         // solves by launches after one that gave up
     constexpr uint64_t kPersistIters = 1 << 14;               // iterations per launch at most
 
-    // The calling thread's limits (hsolve_krylov_limits) and how its last
-    // solve ran (hsolve_krylov_path).
-    struct PersistLimits
+    // The launch of the calling thread's solves that is made to give up
+    // (hsolve_krylov_give_up) and how its last solve ran (hsolve_krylov_path).
+    inline uint64_t & persist_fail()
     {
-        uint64_t iters = kPersistIters;     // per launch
-        uint64_t fail = ~(uint64_t)0;       // the launch of a solve that is made to give up
-    };
-    inline PersistLimits & persist_limits()
-    {
-        static thread_local PersistLimits l;
-        return l;
+        static thread_local uint64_t launch = ~(uint64_t)0;
+        return launch;
     }
     enum PersistPath : int
     {
@@ -102,8 +99,6 @@
         uint64_t * sums;       // kPersistSums, then the give-up flag
         CgScalars<DT> * s;
         int resume;            // the launch continues a solve (z and talpha are the last update's)
-        uint64_t iters;        // iterations of this launch at most
-        unsigned absent;       // a workgroup that stays away, so that the others give up (~0: none)
     };
 
     __global__ __launch_bounds__(256) void persist_clear_kernel(uint64_t * sums)
@@ -219,8 +214,6 @@
         const int tid = threadIdx.x, wave = tid >> 6, half = tid >> 8;
         const unsigned nb = ar.nb, blk0 = blockIdx.x * 2 * RPT;
         const int64_t n = ar.n;
-        if (blockIdx.x == ar.absent)
-            return;
         if (tid == 0)
             gave_up = 0;
 
@@ -253,7 +246,7 @@
                 pn[q][k] = load_at(ar.p, c[q][k]);
         }
         CgScalars<DT> s = *ar.s;
-        uint64_t left = ar.iters;
+        uint64_t left = kPersistIters;
         unsigned turn = 0;
         __syncthreads();
 
@@ -627,13 +620,13 @@
         if (! hold.ok)
             return PE_NOT;
         hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + kPersistFlags, 256)), dim3(256), 0, st, w.sums);
-        const PersistLimits lim = persist_limits();
-        PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0, lim.iters, ~0u};
+        PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0};
         for (uint64_t launch = 0;; ++launch)
         {
-            ar.absent = launch == lim.fail && grid.x > 1 ? grid.x - 1 : ~0u;
+            // (the launch that is made to give up lacks a workgroup)
+            const unsigned present = launch == persist_fail() && grid.x > 1 ? grid.x - 1 : grid.x;
             void * args[] = {&ar};
-            if (hipLaunchKernel(kern.fn, grid, dim3(kPersistThreads), args, kern.lds, st) != hipSuccess)
+            if (hipLaunchKernel(kern.fn, dim3(present), dim3(kPersistThreads), args, kern.lds, st) != hipSuccess)
             {
                 (void)hipGetLastError();
                 return PE_GAVE_UP;

@@ -403,12 +403,12 @@ int hsolve_pcg_jac_ell(hsolve_ell m, const void *dd_inverted, const void *b, voi
  * 2 in one launch that gave up waiting and again by launches.  The same bits
  * each way. */
 int hsolve_krylov_path(int *path);
-/* For tests: one-launch solves of the calling thread run at most `iterations`
- * iterations per launch (0: the default), and in a solve's launch number
- * give_up (from 0; UINT64_MAX: none) one workgroup of several stays away, so
- * that the others give up waiting.  Also ends the pause that a solve which
- * gave up puts in (the current device's next 32 solves go by launches). */
-int hsolve_krylov_limits(uint64_t iterations, uint64_t give_up);
+/* For tests: in launch number `launch` (from 0, of 16,384 iterations each;
+ * UINT64_MAX: none) of every one-launch solve of the calling thread one
+ * workgroup of several stays away, so that the others give up waiting.  Also
+ * ends the pause that a solve which gave up puts in (the current device's next
+ * 32 solves go by launches). */
+int hsolve_krylov_give_up(uint64_t launch);
 
 /* ---------------- many right-hand sides on one ELL matrix -------------------
  * A column-blocked multivector of nrhs <= 64 columns stores row i's entries

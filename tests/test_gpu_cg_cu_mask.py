@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from honei_amd._lib import lib
-from test_gpu_cg_give_up import LAUNCHES, ONE, limits, path, same
+from test_gpu_cg_give_up import LAUNCHES, NEVER, ONE, give_up_in, path, same
 from test_gpu_cg_one_launch import _banded, _solve
 
 pytestmark = pytest.mark.gpu
@@ -26,7 +26,7 @@ def test_masked_streams(hip, kind):
     (one, _), dinv = _banded(n, (1, 17), np.float64, 7)
     b = np.random.default_rng(7).uniform(-1, 1, n)
     M = hip.EllMatrix.from_dict(one)
-    limits()
+    give_up_in(NEVER)
     ref = _solve(hip, kind, M, dinv, b, 50, 1e-12)
     assert path() == ONE
     for words, want in (((0xffffffff,) * 8, ONE), ((0xffffffff,) + (0,) * 7, LAUNCHES),

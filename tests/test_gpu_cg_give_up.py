@@ -24,13 +24,13 @@ def hip():
 
 
 @pytest.fixture(autouse=True)
-def _default_limits():
+def _default():
     yield
-    assert lib().hsolve_krylov_limits(u64(0), u64(NEVER)) == 0
+    give_up_in(NEVER)
 
 
-def limits(iterations=0, give_up=NEVER):
-    assert lib().hsolve_krylov_limits(u64(iterations), u64(give_up)) == 0
+def give_up_in(launch):
+    assert lib().hsolve_krylov_give_up(u64(launch)) == 0
 
 
 def path():
@@ -65,24 +65,26 @@ def test_first_launch_gives_up(hip, kind):
     b = np.random.default_rng(2).uniform(-1, 1, n)
     M = hip.EllMatrix.from_dict(one)
     ref = _solve(hip, kind, hip.EllMatrix.from_dict(two), dinv, b, 25, 1e-12)
-    limits(give_up=0)
+    give_up_in(0)
     assert same(_solve(hip, kind, M, dinv, b, 25, 1e-12), ref) and path() == GAVE_UP
-    limits()
+    give_up_in(NEVER)
     assert same(_solve(hip, kind, M, dinv, b, 25, 1e-12), ref) and path() == ONE
 
 
 @pytest.mark.parametrize("kind", ["none", "jac"])
 def test_later_launch_gives_up(hip, kind):
-    """25 iterations in launches of ten: the second or third finds the workspace of the one before advanced."""
-    n = 3000
-    (one, two), dinv = _banded(n, (1, 54), np.float64, 3)
+    """40,000 iterations (with eps 0 a solve runs to its cap), three launches of at most 16,384: the second and the
+    third find the workspace of the one before advanced."""
+    n = 700
+    (one, two), dinv = _banded(n, (1, 26), np.float64, 3)
     b = np.random.default_rng(3).uniform(-1, 1, n)
     M = hip.EllMatrix.from_dict(one)
-    ref = _solve(hip, kind, hip.EllMatrix.from_dict(two), dinv, b, 25, 1e-12)
-    for give_up, want in ((1, GAVE_UP), (2, GAVE_UP), (3, ONE)):
-        limits(10, give_up)
-        assert same(_solve(hip, kind, M, dinv, b, 25, 1e-12), ref), give_up
+    ref = _solve(hip, kind, hip.EllMatrix.from_dict(two), dinv, b, 40000, 0.0)
+    for launch, want in ((1, GAVE_UP), (2, GAVE_UP), (3, ONE)):
+        give_up_in(launch)
+        got = _solve(hip, kind, M, dinv, b, 40000, 0.0)
         assert path() == want
+        assert got[0][0] == ref[0][0] == 40000 and np.array_equal(got[1], ref[1], equal_nan=True), launch
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
@@ -99,18 +101,18 @@ def test_banded_one_launch_equals_launches(hip, side, dtype):
 
     one = solve()
     assert path() == ONE
-    limits(give_up=0)
+    give_up_in(0)
     assert same(solve(), one) and path() == GAVE_UP
 
 
 @pytest.mark.parametrize("n", [513, 70001, 524288])
 def test_giving_up_takes_milliseconds_and_pauses(hip, n):
-    """A wait ends after about 8 ms, and the device's next 32 solves do not try."""
+    """A wait ends after about 10 ms, and the device's next 32 solves do not try."""
     (one, two), dinv = _banded(n, (1, 17), np.float64, 4)
     b = np.random.default_rng(4).uniform(-1, 1, n)
     M = hip.EllMatrix.from_dict(one)
     ref = _solve(hip, "none", hip.EllMatrix.from_dict(two), dinv, b, 25, 1e-12)
-    limits(give_up=0)
+    give_up_in(0)
     t = time.perf_counter()
     assert same(_solve(hip, "none", M, dinv, b, 25, 1e-12), ref) and path() == GAVE_UP
     assert time.perf_counter() - t < 0.1
@@ -118,6 +120,6 @@ def test_giving_up_takes_milliseconds_and_pauses(hip, n):
         assert same(_solve(hip, "none", M, dinv, b, 25, 1e-12), ref) and path() == LAUNCHES
     _solve(hip, "none", M, dinv, b, 25, 1e-12)
     assert path() == GAVE_UP
-    limits()
+    give_up_in(NEVER)
     _solve(hip, "none", M, dinv, b, 25, 1e-12)
     assert path() == ONE

@@ -8,7 +8,7 @@ import pytest
 
 from honei_amd import problems as P
 from honei_amd._lib import lib, u64, vp
-from test_gpu_cg_give_up import LAUNCHES, ONE, limits, path, same
+from test_gpu_cg_give_up import LAUNCHES, NEVER, ONE, give_up_in, path, same
 from test_gpu_cg_one_launch import _banded
 
 pytestmark = pytest.mark.gpu
@@ -39,7 +39,7 @@ def test_a_solve_does_not_wait_for_another_thread(hip, n, want):
     (one, _), dinv = _banded(n, (1, 150), np.float64, 8)
     b = np.random.default_rng(8).uniform(-1, 1, n)
     M = hip.EllMatrix.from_dict(one)
-    limits()
+    give_up_in(NEVER)
     v = [_vectors(hip, b) for _ in range(3)]
     ref = (_solve("hsolve_cg_ell", M, v[2], None), v[2][1].get())
     side = 129
