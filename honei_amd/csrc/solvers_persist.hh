@@ -30,18 +30,19 @@
 // order of one solve (a bound in polls, not by the clock: time in which the
 // process is switched off the device does not count, and no register is spent; a
 // bound of 16 bits shortens the loop's code by four bytes, which moved it within
-// the fetch lines and made 513^2 Jacobi-PCG 5% slower).
-// After a solve that gave up, the device's next kPersistPause go by launches at
-// once: where the CUs stay taken, giving up costs each a third of a millisecond.
+// the fetch lines and made 513^2 Jacobi-PCG 5% slower).  After a solve that gave
+// up, the device's next kPersistPause go by launches at once: where the CUs stay
+// taken, giving up costs each a third of a millisecond.
 //
 // The launch is an ordinary one, of at most one workgroup per CU (checked to
 // fit), on streams without a CU mask, so that all of them are resident as soon
 // as other streams' kernels leave room.  Solves of several threads run side by
-// side while there is a CU for each of their workgroups (PersistHold); one that
-// finds too few goes by launches.  A cooperative launch promises the same, but the
-// queue that the runtime opens for it stays: streams of the process that run
-// side by side afterwards (the request server's) took 10.7 ms instead of 8.5 ms
-// for 48 mixed requests.
+// side while there is a CU for each of their workgroups (PersistHold), with more
+// rows a thread if need be; one that finds too few CUs goes by launches (measured,
+// four threads solving 257^2 by CG: 2.05 ms a solve, one after another 3.5).  A
+// cooperative launch promises the same, but the queue that the runtime opens for
+// it stays: streams of the process that run side by side afterwards (the request
+// server's) took 10.7 ms instead of 8.5 ms for 48 mixed requests.
 #pragma once
 
     constexpr int kPersistThreads = 512;                      // two blocks of 256 rows side by side
@@ -556,19 +557,21 @@
     struct PersistHold
     {
         PersistDevice & d;
-        const unsigned share;
-        bool ok = false;
-        PersistHold(PersistDevice & dev, unsigned workgroups) : d(dev), share((workgroups + kEngines - 1) / kEngines)
+        unsigned share = 0;
+        explicit PersistHold(PersistDevice & dev) : d(dev) {}
+        bool take(unsigned workgroups)
         {
+            const unsigned want = (workgroups + kEngines - 1) / kEngines;
             unsigned h = d.held.load();
-            while (! ok && h + share <= d.cus / kEngines)
-                ok = d.held.compare_exchange_weak(h, h + share);
+            while (h + want <= d.cus / kEngines)
+                if (d.held.compare_exchange_weak(h, h + want))
+                {
+                    share = want;
+                    return true;
+                }
+            return false;
         }
-        ~PersistHold()
-        {
-            if (ok)
-                d.held -= share;
-        }
+        ~PersistHold() { d.held -= share; }
         PersistHold(const PersistHold &) = delete;
     };
 
@@ -609,15 +612,21 @@
         if (! dev)
             return PE_NOT;
         const unsigned nb = grid_for(n, 256);
-        const int rpt = persist_rows_per_thread(nb, dev->cus);
-        const PersistKernel kern = rpt ? persist_kernel<DT, KIND>(q1, width, rpt) : PersistKernel();
+        if (! persist_whole_device(st, dev->cus) || dev->paused())
+            return PE_NOT;
+        // the fewest rows a thread, or more of them where other solves have
+        // left fewer CUs
+        PersistHold hold(*dev);
+        PersistKernel kern;
+        dim3 grid(0);
+        for (int rpt = persist_rows_per_thread(nb, dev->cus); rpt != 0 && rpt <= 4 && hold.share == 0; ++rpt)
+        {
+            kern = persist_kernel<DT, KIND>(q1, width, rpt);
+            grid.x = grid_for(nb, 2 * rpt);
+            if (! kern.fn || ! dev->fit(kern) || ! hold.take(grid.x))
+                kern.fn = nullptr;
+        }
         if (! kern.fn)
-            return PE_NOT;
-        const dim3 grid(grid_for(nb, 2 * rpt));
-        if (! dev->fit(kern) || ! persist_whole_device(st, dev->cus) || dev->paused())
-            return PE_NOT;
-        const PersistHold hold(*dev, grid.x);
-        if (! hold.ok)
             return PE_NOT;
         hipLaunchKernelGGL(persist_clear_kernel, dim3(grid_for(kPersistSums + kPersistFlags, 256)), dim3(256), 0, st, w.sums);
         PersistArgs<DT> ar{A, x, w.p2, w.r, w.p, w.v, P, (int64_t)n, nb, w.sums, w.s, 0};

@@ -31,11 +31,11 @@ def _solve(entry, M, v, stream):
     return used.value, defect.value
 
 
-@pytest.mark.parametrize("n,want", [(30000, ONE), (262144, LAUNCHES)])
+@pytest.mark.parametrize("n,want", [(30000, ONE), (66049, ONE), (262144, LAUNCHES)])
 def test_a_solve_does_not_wait_for_another_thread(hip, n, want):
     """The first thread's solve stands behind most of a second of other work on its stream; the second thread's, on a
-    stream of its own, ends meanwhile.  Two of 30,000 rows run side by side in one launch each; 262,144 rows take
-    every CU, so the second goes by launches."""
+    stream of its own, ends meanwhile.  Two of 30,000 rows run side by side in one launch each, of 66,049 rows the
+    second with two rows a thread; 262,144 rows take every CU, so the second goes by launches."""
     (one, _), dinv = _banded(n, (1, 150), np.float64, 8)
     b = np.random.default_rng(8).uniform(-1, 1, n)
     M = hip.EllMatrix.from_dict(one)
