@@ -642,13 +642,16 @@
             }
             hipLaunchKernelGGL((persist_copy_kernel<DT>), dim3(std::min<unsigned>(grid_for(n, 1024), 256)), dim3(256), 0,
                                st, (const DT *)w.p2, x, (int64_t)n, (const uint64_t *)w.sums, (const CgScalars<DT> *)w.s);
-            // the give-up flag and the scalars behind it
+            // the give-up flag and the scalars behind it (after a wait of its own:
+            // a copy to host memory right behind the kernels took up to 4 ms for a
+            // solve on arrays that were new)
             struct
             {
                 uint64_t gave_up[kPersistFlags];
                 CgScalars<DT> s;
             } end;
             static_assert(sizeof(end) == sizeof(end.gave_up) + sizeof(end.s), "laid out as CgWork lays them out");
+            HIP_CHECK(hipStreamSynchronize(st));
             HIP_CHECK(hipMemcpyAsync(&end, w.sums + kPersistSums, sizeof(end), hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
             if (end.gave_up[0])
