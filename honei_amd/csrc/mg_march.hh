@@ -9,13 +9,14 @@
 // multiplications take as an operand.  Waves share nothing, so there is no
 // barrier and no LDS traffic between the stages.
 //
-// What bounds them: on large levels the vector units and HBM about equally
-// (finest 4097^2 pre-smoothing 64 us for 302 MB, 4.7 TB/s; post-smoothing 72
-// us, 4.2 TB/s), on levels below 1025^2 the chain of th + 6 steps (8 to 13 us
-// a launch).  The form before, 256 columns per workgroup with the rings in LDS
-// and two or three barriers a step, took 118 and 159 us there, 44 us a
-// kernel at 2049^2 (now 20), 13 to 23 us from 65^2 to 513^2, and with plain
-// bands and 64 slots at 513^2 204 and 235 us (now 105 and 114).
+// What bounds them: on large levels HBM, and the post-smoothing the vector
+// units as well (finest 4097^2, 302 MB each and the tiles' halos: pre-smoothing
+// 66 us for 364 MB, 5.4 TB/s, vector units busy 64% of the time; post-smoothing
+// 74 us for 352 MB, 4.6 TB/s, 88%), on levels below 1025^2 the chain of th + 6
+// steps (8 to 13 us a launch).  The form before, 256 columns per workgroup with
+// the rings in LDS and two or three barriers a step, took 118 and 159 us there,
+// 44 us a kernel at 2049^2 (now 20), 13 to 23 us from 65^2 to 513^2, and with
+// plain bands and 64 slots at 513^2 204 and 235 us (now 105 and 114).
 //
 // A tile's lanes hold linear node indices i = r m + c for columns c0 - kHalo
 // .. c0 + W + kHalo - 1, so columns past a grid row's ends are the
